@@ -596,11 +596,14 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
     precision = eff_precision(c, precision);
     if ((rc = ring_chunks(c)) != GDT_OK) return rc;
     if ((rc = build_cells(c, d_xy, s, true)) != GDT_OK) return rc;
-    if (tiled_sets(c) && precision != GDT_PREC_EXACT) {
+    if (tiled_sets(c)) {
         // A grid of at most one tile per CU runs one wave of blocks: each lane
         // (or lane group) then takes a single point (1024 threads for about
         // 1024 points of a 32x32 tile), so the block ends after its longest
         // ring instead of after two.
+        // (Every precision: the exact mode's tile and star kernels were 6 to 10
+        // times the per-point kernel's speed on random points and near-degenerate
+        // lattices alike.)
         const int ts = c->sets[0].tshift, lanes = lanes_for(c);
         c->stats.tile_shift = ts;
         if (lanes == GDT_STAR_LANES) {
@@ -611,18 +614,18 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
             const long long avg = (c->total_n + c->ntch - 1) / c->ntch;
             int nsplit = (int)std::max(1LL, (avg + nw - 1) / nw);
             nsplit = std::min(nsplit, std::max(1, 4 * c->num_cu / c->ntch));
-            GDT_CHECK(gdt_tiles::one_ring_star(ts, c->d_sets.p, (int)c->sets.size(), c->tch.p,
-                                               c->ntch, nsplit, block, c->total_n,
+            GDT_CHECK(gdt_tiles::one_ring_star(ts, precision, c->d_sets.p, (int)c->sets.size(), c->tch.p,
+                                               c->ntch, nsplit, block,
                                                ring_io(c, d_nbrs, stride), d_counts, c->status.p,
                                                c->counters.p, c->defer.p,
                                                c->cfg.profile ? c->ev[2] : nullptr, s));
         } else {
-            c->stats.lanes = lanes == 4 && precision == GDT_PREC_FP32F ? 2 : lanes;
+            c->stats.lanes = lanes == 4 && precision != GDT_PREC_FP64 ? 2 : lanes;
             const int one_each = std::min(1024, (1 << (2 * ts)) * lanes);
             const int block =
                 c->ntch <= c->num_cu ? std::max(tile_block(c), one_each) : tile_block(c);
             GDT_CHECK(gdt_tiles::one_ring(ts, precision, c->d_sets.p, (int)c->sets.size(),
-                                          c->tch.p, c->ntch, block, lanes, c->total_n, nullptr,
+                                          c->tch.p, c->ntch, block, lanes, nullptr,
                                           nullptr, nullptr, nullptr, ring_io(c, d_nbrs, stride),
                                           d_counts, c->status.p, c->counters.p, c->defer.p,
                                           c->cfg.profile ? c->ev[2] : nullptr, s));
@@ -634,12 +637,12 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
         // (the exact mode hands no point on: one beyond the search radius is an error)
         const bool exact = precision == GDT_PREC_EXACT;
         GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), c->rch.p, c->nrch,
-                                      c->cfg.block, nullptr, nullptr, 0, 0, io, d_counts,
+                                      c->cfg.block, nullptr, nullptr, 0, io, d_counts,
                                       c->status.p, c->counters.p, exact ? nullptr : c->defer.p, s));
         if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[2], s));
         if (!exact)
-            GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), c->total_n,
-                                          io, d_counts, c->status.p, c->counters.p, c->defer.p, s));
+            GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
+                                          c->status.p, c->counters.p, c->defer.p, s));
     }
     if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
     rc = finish_rings(c, stride, required, s);
@@ -811,7 +814,7 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
     if (tiled_sets(c) && !exact) {
         GDT_CHECK(gdt_tiles::one_ring(c->sets[0].tshift, precision, c->d_sets.p,
                                       (int)c->sets.size(), c->tch.p, c->ntch, tile_block(c),
-                                      c->cfg.repair_lanes ? c->cfg.repair_lanes : 2, c->total_n,
+                                      c->cfg.repair_lanes ? c->cfg.repair_lanes : 2,
                                       nullptr, nullptr, d_repair, c->halt,
                                       ring_io(c, d_nbrs, stride), d_counts, c->status.p,
                                       c->counters.p, c->defer.p, nullptr, s));
@@ -826,12 +829,12 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
                                  c->worklist.p, worklen, c->scan_tmp.p, c->halt, s));
     const GdtRingIO io = ring_io(c, d_nbrs, stride);
     GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), nullptr, 0,
-                                  c->cfg.block, c->worklist.p, worklen, 0, c->total_n, io,
+                                  c->cfg.block, c->worklist.p, worklen, c->total_n, io,
                                   d_counts, c->status.p, c->counters.p,
                                   exact ? nullptr : c->defer.p, s));
     if (!exact)
-        GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), c->total_n, io,
-                                      d_counts, c->status.p, c->counters.p, c->defer.p, s));
+        GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
+                                      c->status.p, c->counters.p, c->defer.p, s));
     return GDT_OK;
 }
 

@@ -24,6 +24,11 @@
 
 #define GDT_XN 32
 
+// The expansion routines are calls, not inlined: they are reached by exact
+// ties only, and their code (tens of kilobytes per inlined predicate) would
+// lie between the instructions of every other decision.
+#define GDT_XCALL __attribute__((noinline))
+
 struct GdtX {
     double t[GDT_XN];
     int n;
@@ -141,7 +146,7 @@ GDT_HD inline int gdt_x_sign(const GdtX& e)
 // Exact displacement of caller point c seen from caller point v (rectangle
 // lx x ly), the image the FP64 displacement (fx, fy) chose:
 // (x_c - x_v) + m lx with m = round((fx - (x_c - x_v)) / lx), likewise y.
-GDT_HD inline void gdt_x_disp(const gdt_d2& pv, const gdt_d2& pc, double lx, double ly, double fx,
+GDT_HD GDT_XCALL inline void gdt_x_disp(const gdt_d2& pv, const gdt_d2& pc, double lx, double ly, double fx,
                               double fy, GdtX& X, GdtX& Y, GdtXCtx& cx)
 {
     double s, e;
@@ -185,7 +190,7 @@ GDT_HD inline void gdt_x_det2(GdtX& h, const GdtX& p, const GdtX& q, const GdtX&
 }
 
 // sign(a x c), the orientation of gdt_orient64.
-GDT_HD inline int gdt_x_orient(const GdtXVec& a, const GdtXVec& c, GdtXCtx& cx)
+GDT_HD GDT_XCALL inline int gdt_x_orient(const GdtXVec& a, const GdtXVec& c, GdtXCtx& cx)
 {
     GdtX h, tmp;
     gdt_x_det2(h, a.x, c.y, a.y, c.x, tmp, cx);
@@ -200,7 +205,7 @@ GDT_HD inline void gdt_x_norm2(GdtX& h, const GdtXVec& a, GdtX& tmp, GdtXCtx& cx
 }
 
 // sign(|c|^2 - |b|^2).
-GDT_HD inline int gdt_x_dist_cmp(const GdtXVec& c, const GdtXVec& b, GdtXCtx& cx)
+GDT_HD GDT_XCALL inline int gdt_x_dist_cmp(const GdtXVec& c, const GdtXVec& b, GdtXCtx& cx)
 {
     GdtX p, q, tmp;
     gdt_x_norm2(p, c, tmp, cx);
@@ -212,7 +217,7 @@ GDT_HD inline int gdt_x_dist_cmp(const GdtXVec& c, const GdtXVec& b, GdtXCtx& cx
 // sign of P(c) = K0 |c|^2 + Kx cx + Ky cy for the circle through the origin,
 // a and b (the polynomial of gdt_circ64 / gdt_incircle64: < 0 iff c strictly
 // inside when a, b are counter-clockwise).
-GDT_HD inline int gdt_x_incircle(const GdtXVec& a, const GdtXVec& b, const GdtXVec& c,
+GDT_HD GDT_XCALL inline int gdt_x_incircle(const GdtXVec& a, const GdtXVec& b, const GdtXVec& c,
                                  GdtXCtx& cx)
 {
     GdtX aa, bb, k, t, tmp, acc;
@@ -263,6 +268,123 @@ GDT_HD inline double gdt_x_tol4(double e, double M)
     return 2. * (48. * e * Me * Me * Me + GDT_XTOL_SCALE * 32. * GDT_XU * M * M * M * M);
 }
 
+// ---------------------------------------------------------------------------
+// Double-double stage.  Between the FP64 value and the expansions: the same
+// polynomials on the displacements rounded to pairs of doubles (about 106
+// bits), in registers, with the same error bounds one precision up.  It
+// decides every sign but those of exact (or nearly exact) zeros, which alone
+// go on to the expansions.  Addition and multiplication are the standard
+// error-free ones (Dekker 1971, Knuth), each within a few u^2 of the exact
+// result relative to its operands; GDT_XU2 takes 16 u^2 for each.
+// ---------------------------------------------------------------------------
+struct GdtDD {
+    double h, l;
+};
+struct GdtDDVec {
+    GdtDD x, y;
+};
+
+GDT_HD inline GdtDD gdt_dd_add(const GdtDD& a, const GdtDD& b)
+{
+    double s, e, t, f;
+    gdt_two_sum(a.h, b.h, s, e);
+    gdt_two_sum(a.l, b.l, t, f);
+    e += t;
+    gdt_fast_two_sum(s, e, s, e);
+    e += f;
+    GdtDD r;
+    gdt_fast_two_sum(s, e, r.h, r.l);
+    return r;
+}
+GDT_HD inline GdtDD gdt_dd_sub(const GdtDD& a, const GdtDD& b)
+{
+    const GdtDD n = {-b.h, -b.l};
+    return gdt_dd_add(a, n);
+}
+GDT_HD inline GdtDD gdt_dd_mul(const GdtDD& a, const GdtDD& b)
+{
+    double p, e;
+    gdt_two_prod(a.h, b.h, p, e);
+    e = fma(a.h, b.l, fma(a.l, b.h, e));
+    GdtDD r;
+    gdt_fast_two_sum(p, e, r.h, r.l);
+    return r;
+}
+// p q - r s
+GDT_HD inline GdtDD gdt_dd_det2(const GdtDD& p, const GdtDD& q, const GdtDD& r, const GdtDD& s)
+{
+    return gdt_dd_sub(gdt_dd_mul(p, q), gdt_dd_mul(r, s));
+}
+GDT_HD inline GdtDD gdt_dd_norm2(const GdtDDVec& a)
+{
+    return gdt_dd_add(gdt_dd_mul(a.x, a.x), gdt_dd_mul(a.y, a.y));
+}
+
+// gdt_x_disp rounded to double-doubles (one axis): (c - v) + m L.
+GDT_HD inline GdtDD gdt_dd_disp1(double v, double c, double L, double f)
+{
+    double s, e;
+    gdt_two_sum(c, -v, s, e);
+    GdtDD r = {s, e};
+    const double m = rint((f - s) / L);
+    if (m != 0.) {
+        double p, q, h, l;
+        gdt_two_prod(m, L, p, q);
+        gdt_two_sum(s, p, h, l);
+        l += e + q;
+        gdt_fast_two_sum(h, l, r.h, r.l);
+    }
+    return r;
+}
+GDT_HD inline GdtDDVec gdt_dd_disp(const gdt_d2& pv, const gdt_d2& pc, double lx, double ly,
+                                   double fx, double fy)
+{
+    GdtDDVec d;
+    d.x = gdt_dd_disp1(pv.x, pc.x, lx, fx);
+    d.y = gdt_dd_disp1(pv.y, pc.y, ly, fy);
+    return d;
+}
+
+// Values of the three predicates (signs as gdt_x_orient, gdt_x_dist_cmp,
+// gdt_x_incircle).
+GDT_HD inline double gdt_dd_orient(const GdtDDVec& a, const GdtDDVec& c)
+{
+    return gdt_dd_det2(a.x, c.y, a.y, c.x).h;
+}
+GDT_HD inline double gdt_dd_dist_cmp(const GdtDDVec& c, const GdtDDVec& b)
+{
+    return gdt_dd_sub(gdt_dd_norm2(c), gdt_dd_norm2(b)).h;
+}
+GDT_HD inline double gdt_dd_incircle(const GdtDDVec& a, const GdtDDVec& b, const GdtDDVec& c)
+{
+    const GdtDD aa = gdt_dd_norm2(a), bb = gdt_dd_norm2(b);
+    GdtDD P = gdt_dd_mul(gdt_dd_det2(a.x, b.y, a.y, b.x), gdt_dd_norm2(c));
+    P = gdt_dd_add(P, gdt_dd_mul(gdt_dd_det2(bb, a.y, aa, b.y), c.x));
+    P = gdt_dd_add(P, gdt_dd_mul(gdt_dd_det2(aa, b.x, bb, a.x), c.y));
+    return P.h;
+}
+
+// Their error bounds: those of gdt_x_tol2 and gdt_x_tol4 with a displacement
+// error of 64 u^2 (L + |d|) (the pair holds (c - v) exactly; the rounding of
+// its sum with m L, |m L| at most five box lengths, is below 16 u^2 L) and
+// 16 u^2 for u.
+#define GDT_XU2 (16. * GDT_XU * GDT_XU)
+GDT_HD inline double gdt_dd_err(double L, double d)
+{
+    return GDT_XTOL_SCALE * 64. * GDT_XU * GDT_XU * (L + fabs(d));
+}
+GDT_HD inline double gdt_dd_tol2(double e, double M)
+{
+    return 2. * (4. * (e * M + e * e) + GDT_XTOL_SCALE * 4. * GDT_XU2 * M * M);
+}
+GDT_HD inline double gdt_dd_tol4(double e, double M)
+{
+    const double Me = M + e;
+    return 2. * (48. * e * Me * Me * Me + GDT_XTOL_SCALE * 32. * GDT_XU2 * M * M * M * M);
+}
+// +1, -1, or 0 where the bound does not certify a sign.
+GDT_HD inline int gdt_dd_sign(double v, double tol) { return v > tol ? 1 : (v < -tol ? -1 : 0); }
+
 // a - b, componentwise.
 GDT_HD inline void gdt_x_sub(GdtXVec& h, const GdtXVec& a, const GdtXVec& b, GdtXCtx& cx)
 {
@@ -282,7 +404,7 @@ GDT_HD inline void gdt_x_neg(GdtXVec& h, const GdtXVec& a)
 // The symbolic perturbation of gdt_incircle_tie (caller indices pv, pa, pb,
 // pc; v at the origin), with the orientations it reads taken exactly: whether
 // c, on the circle through v, a, b, counts as inside.
-GDT_HD inline bool gdt_x_incircle_tie(int pv, int pa, int pb, int pc, const GdtXVec& a,
+GDT_HD GDT_XCALL inline bool gdt_x_incircle_tie(int pv, int pa, int pb, int pc, const GdtXVec& a,
                                       const GdtXVec& b, const GdtXVec& c, GdtXCtx& cx)
 {
     const int m = gdt_imin(gdt_imin(pv, pa), gdt_imin(pb, pc));

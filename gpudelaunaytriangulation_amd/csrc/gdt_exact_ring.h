@@ -5,7 +5,8 @@
 // Chebyshev rings of cells with certified stops), with every decision taken
 // on the exact displacements of the caller's coordinates: a comparison whose
 // FP64 value lies outside its error bound (gdt_exact.h) keeps the FP64
-// answer, which is then the exact one; inside it the sign is computed with
+// answer, which is then the exact one; inside it the sign is taken from the
+// double-double value where that clears its own bound, else computed with
 // expansions, and an exact zero falls to the symbolic perturbation of
 // gdt_nn_tie / gdt_incircle_tie (with exact orientations), so the rings are
 // the Delaunay triangulation of the caller's points perturbed as the FP64
@@ -86,6 +87,35 @@ GDT_HD inline GdtRingResult gdt_one_ring_exact(const GdtSet& S, int j, const Gdt
         return X;
     };
     auto mag = [](const GdtXCand& c) { return fmax(fabs(c.x), fabs(c.y)); };
+    auto dd = [&](const GdtXCand& c) {
+        return gdt_dd_disp(pv, io.xy[io.perm[c.k]], S.lx, S.ly, c.x, c.y);
+    };
+    // Signs of the three predicates where FP64 does not certify them: the
+    // double-double value, or the expansions inside its bound (M: the largest
+    // displacement coordinate).
+    auto dist_sign = [&](GdtXCand& c, GdtXCand& b) {
+        const double M = fmax(mag(c), mag(b));
+        const int s = gdt_dd_sign(gdt_dd_dist_cmp(dd(c), dd(b)),
+                                  2. * gdt_dd_tol2(gdt_dd_err(L, M), M));
+        if (s == 0) return gdt_x_dist_cmp(exact(c), exact(b), xc);
+        GDT_XAUDIT(2, s, gdt_x_dist_cmp(exact(c), exact(b), xc));
+        return s;
+    };
+    auto orient_sign = [&](GdtXCand& a, GdtXCand& c) {
+        const double M = fmax(mag(a), mag(c));
+        const int s = gdt_dd_sign(gdt_dd_orient(dd(a), dd(c)), gdt_dd_tol2(gdt_dd_err(L, M), M));
+        if (s == 0) return gdt_x_orient(exact(a), exact(c), xc);
+        GDT_XAUDIT(0, s, gdt_x_orient(exact(a), exact(c), xc));
+        return s;
+    };
+    auto incircle_sign = [&](GdtXCand& a, GdtXCand& b, GdtXCand& c) {
+        const double M = fmax(fmax(mag(a), mag(b)), mag(c));
+        const int s = gdt_dd_sign(gdt_dd_incircle(dd(a), dd(b), dd(c)),
+                                  gdt_dd_tol4(gdt_dd_err(L, M), M));
+        if (s == 0) return gdt_x_incircle(exact(a), exact(b), exact(c), xc);
+        GDT_XAUDIT(1, s, gdt_x_incircle(exact(a), exact(b), exact(c), xc));
+        return s;
+    };
 
     // 1. nearest neighbour: c beats b when |c|^2 < |b|^2, exact ties by caller index
     GdtXCand nn, cand, a, best;
@@ -115,7 +145,7 @@ GDT_HD inline GdtRingResult gdt_one_ring_exact(const GdtSet& S, int j, const Gdt
                 } else if (d2 > nd2 + tol) {
                     GDT_XAUDIT(2, 1, gdt_x_dist_cmp(exact(cand), exact(nn), xc));
                 } else {
-                    const int s = gdt_x_dist_cmp(exact(cand), exact(nn), xc);
+                    const int s = dist_sign(cand, nn);
                     take = s < 0 || (s == 0 && gdt_nn_tie(io.perm[k], io.perm[nn.k]));
                 }
             }
@@ -164,7 +194,7 @@ GDT_HD inline GdtRingResult gdt_one_ring_exact(const GdtSet& S, int j, const Gdt
                     bool left = O > tol;
                     if (left) GDT_XAUDIT(0, 1, gdt_x_orient(exact(a), exact(cand), xc));
                     else if (O < -tol) GDT_XAUDIT(0, -1, gdt_x_orient(exact(a), exact(cand), xc));
-                    else left = gdt_x_orient(exact(a), exact(cand), xc) > 0;
+                    else left = orient_sign(a, cand) > 0;
                     if (!left) continue;
                 }
                 if (best.k >= 0) {
@@ -178,7 +208,7 @@ GDT_HD inline GdtRingResult gdt_one_ring_exact(const GdtSet& S, int j, const Gdt
                     else if (P > tol)
                         GDT_XAUDIT(1, 1, gdt_x_incircle(exact(a), exact(best), exact(cand), xc));
                     else {
-                        const int s = gdt_x_incircle(exact(a), exact(best), exact(cand), xc);
+                        const int s = incircle_sign(a, best, cand);
                         inside = s < 0 ||
                                  (s == 0 && gdt_x_incircle_tie(io.perm[j], io.perm[a.k],
                                                                io.perm[best.k], io.perm[k],

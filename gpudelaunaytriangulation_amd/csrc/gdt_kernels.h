@@ -68,26 +68,29 @@ hipError_t gdt_export_cells(const GdtSet* d_sets, const GdtSet& h_set, const Gdt
                             unsigned int* cell_sizes, int* idxs, int nmax, hipStream_t s);
 hipError_t gdt_max_occupancy(const uint32_t* ccount, int total_keys, int* d_out, hipStream_t s);
 
-// One-ring of every point (chunks of `block` points) or of the worklist slots
-// [skip, *worklen) (max_work bounds *worklen).  With `defer`, points whose
+// One-ring of every point (chunks of `block` points) or of the *worklen slots
+// of the worklist (max_work bounds *worklen).  With `defer`, points whose
 // search the grid's search radius cannot certify are appended there (count
 // in status[ST_NDEFER], zero on entry) for gdt_launch_deferred.
 hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                const GdtChunk* chunks, int nch, int block, const int* worklist,
-                               const uint32_t* worklen, int skip, int max_work,
+                               const uint32_t* worklen, int max_work,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s);
 
 // Deferred points: the first GDT_WAVE_CAP one wavefront each (GDT_WAVE_BLOCKS
-// blocks of 256 threads), the rest one lane each.
+// blocks of 256 threads), the rest one lane each, in one launch.
 #define GDT_WAVE_CAP 8192
 #define GDT_WAVE_BLOCKS 512
+// Threads per block (at most) of the exact mode's tile and star kernels: two
+// waves per SIMD, so that the double-double decisions keep 256 registers.
+#define GDT_XTILE_BLOCK 512
 // Deferred points a tile block finishes itself (the rest go to the list).
 #define GDT_TILE_DEFER 64
 
 // Deferred points of the tile kernel (defer[0..status[ST_NDEFER]), count read
-// on the device): the wavefront kernel, then one lane each beyond GDT_WAVE_CAP.
-hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets, int total_n,
+// on the device): a wavefront each, then one lane each beyond GDT_WAVE_CAP.
+hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s);
 
@@ -100,13 +103,14 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets, i
     namespace ns {                                                                                \
     hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles, int ntiles, int block, int lanes, \
-                                        int total_n, const int* list, const uint32_t* lscan,     \
+                                        const int* list, const uint32_t* lscan,                  \
                                         const int* flags, const int* halt,                       \
                                         const GdtRingIO& io, int* counts, int* status,           \
                                         unsigned long long* counters, int* defer,                \
                                         hipEvent_t after_tile, hipStream_t s);                   \
-    hipError_t gdt_launch_one_ring_star(const GdtSet* d_sets, int nsets, const GdtChunk* tiles,  \
-                                        int ntiles, int nsplit, int block, int total_n,          \
+    hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,          \
+                                        const GdtChunk* tiles,                                   \
+                                        int ntiles, int nsplit, int block,                       \
                                         const GdtRingIO& io, int* counts, int* status,           \
                                         unsigned long long* counters, int* defer,                \
                                         hipEvent_t after_tile, hipStream_t s);                   \
@@ -141,7 +145,7 @@ hipError_t gdt_launch_test(const GdtSet* d_sets, int nsets, const int* tris, con
 // flagged slots, status[ST_NFLAGGED] += their count, which must start at zero;
 // nothing with *halt set), one block per tile of the tiled cell order,
 // `lanes` (1, 2 or 4) lanes per point.  Points the tile kernel cannot finish
-// from LDS are deferred (gdt_launch_deferred over `defer`, size total_n, count
+// from LDS are deferred (gdt_launch_deferred over `defer`, a slot per point, count
 // in status[ST_NDEFER]).
 //
 // The same rings of every point with one wavefront per point (the star
@@ -160,24 +164,24 @@ static_assert(GDT_TSHIFT_MIN == 4 && GDT_TSHIFT_MAX == 5, "a launcher per suppor
 
 namespace gdt_tiles {
 inline hipError_t one_ring(int tshift, int precision, const GdtSet* d_sets, int nsets,
-                           const GdtChunk* tiles, int ntiles, int block, int lanes, int total_n,
+                           const GdtChunk* tiles, int ntiles, int block, int lanes,
                            const int* list, const uint32_t* lscan, const int* flags,
                            const int* halt, const GdtRingIO& io, int* counts, int* status,
                            unsigned long long* counters, int* defer, hipEvent_t after_tile,
                            hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_tile : ts5::gdt_launch_one_ring_tile)(
-        precision, d_sets, nsets, tiles, ntiles, block, lanes, total_n, list, lscan, flags, halt,
+        precision, d_sets, nsets, tiles, ntiles, block, lanes, list, lscan, flags, halt,
         io, counts, status, counters, defer, after_tile, s);
 }
-inline hipError_t one_ring_star(int tshift, const GdtSet* d_sets, int nsets,
+inline hipError_t one_ring_star(int tshift, int precision, const GdtSet* d_sets, int nsets,
                                 const GdtChunk* tiles, int ntiles, int nsplit, int block,
-                                int total_n, const GdtRingIO& io, int* counts, int* status,
+                                const GdtRingIO& io, int* counts, int* status,
                                 unsigned long long* counters, int* defer, hipEvent_t after_tile,
                                 hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_star : ts5::gdt_launch_one_ring_star)(
-        d_sets, nsets, tiles, ntiles, nsplit, block, total_n, io, counts, status, counters, defer,
+        precision, d_sets, nsets, tiles, ntiles, nsplit, block, io, counts, status, counters, defer,
         after_tile, s);
 }
 inline hipError_t ring_test(int tshift, const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,

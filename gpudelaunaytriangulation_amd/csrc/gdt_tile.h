@@ -21,6 +21,7 @@
 // written for general (eps1, eps0), doubled for slack.
 #pragma once
 
+#include "gdt_exact.h"
 #include "gdt_point.h"
 
 #ifndef GDT_SCAN0
@@ -520,17 +521,42 @@ GDT_HD inline int gdt_tile_advance(const GdtTileLds& L, const GdtRingIO& io, Gdt
 // W lanes may share the point (W = 2 or 4, device only): each scans its part
 // of every row segment, and the group then agrees on the best of their bests,
 // so all end every step in the same state.
-template <int W = 1>
+// CERT (the exact mode): a decision is taken from its FP64 value only outside
+// the error bound of gdt_exact.h -- the window's displacement meets the bound
+// of the per-point routine's: its frame coordinates add roundings of at most
+// 20 cells, below three box lengths since the window's scan block must fit
+// the grid -- and from the double-double value of the caller's coordinates
+// (*xio) outside that one's; a sign neither certifies hands the point on
+// (GDT_TIE), as an exact tie does.
+template <int W = 1, bool CERT = false>
 GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
                                       const GdtTileLane<double>& st, unsigned& npred, int sub,
                                       bool ext, int& bk, double& bx, double& by,
                                       const uint32_t* pre = nullptr, unsigned npre = 0,
-                                      int ph = GDT_SCAN0)
+                                      int ph = GDT_SCAN0, const GdtRingIO* xio = nullptr)
 {
     static_assert(W == 1 || W == 2 || W == 4, "1, 2 or 4 lanes per point");
     const bool wrap = st.ak >= 0;
     bk = -1;
     const double ax = st.ax, ay = st.ay, vx = st.vx, vy = st.vy;
+    // CERT: bounds over the region being scanned (displacements up to h + 1
+    // cells and |a|); the nearest-neighbour search compares two distances and
+    // no orientation (O = 0)
+    double tO = 0., tP = 0.;
+    const double Lbox = CERT ? GDT_FMAX(S.lx, S.ly) : 0.;
+    const double ma = CERT ? GDT_FMAX(fabs(ax), fabs(ay)) : 0.;
+    auto set_region = [&](int h) {
+        if constexpr (CERT) {
+            const double M = GDT_FMAX(ma, (double)(h + 1) * GDT_FMAX(S.bsx, S.bsy));
+            const double e = gdt_x_err(Lbox, M);
+            tO = wrap ? gdt_x_tol2(e, M) : 0.;
+            tP = wrap ? gdt_x_tol4(e, M) : 2. * gdt_x_tol2(e, M);
+        }
+    };
+    if constexpr (CERT) {
+        // the clip to the left half-plane needs a's direction to 1e-6
+        if (wrap && ma < 1e6 * gdt_x_err(Lbox, ma)) return STEP_DEFER;
+    }
     const int wx = st.c0 % GDT_WIN, wy = st.c0 / GDT_WIN;
     // Both searches as one test, c taken when O(c) > Othr, P(c) < Pthr and
     // c is not the excluded entry:
@@ -558,11 +584,54 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     // hands the point to the wavefront routine, which decides ties by the
     // symbolic perturbation of gdt_incircle_tie / gdt_nn_tie.  No other state:
     // the test is the branch's own comparison.
+    // CERT: the double-double decision (1: k is the new best, 0: it is not,
+    // -1: not certified) where the FP64 values are inside their bounds
+    auto decide_dd = [&](int k, double px, double py, double O, double P) -> int {
+        const gdt_d2 pv = xio->xy[L.orig[st.iv]];
+        auto dd = [&](int q, double x, double y) {
+            return gdt_dd_disp(pv, xio->xy[L.orig[q]], S.lx, S.ly, x, y);
+        };
+        const GdtDDVec c = dd(k, px, py);
+        const double mc = GDT_FMAX(ma, GDT_FMAX(fabs(px), fabs(py)));
+        GdtDDVec a = {{0., 0.}, {0., 0.}};
+        if (wrap) a = dd(st.ak, ax, ay);
+        if (!(O > Othr + tO)) {         // (successor only: tO = 0 else)
+            const int s = gdt_dd_sign(gdt_dd_orient(a, c),
+                                      gdt_dd_tol2(gdt_dd_err(Lbox, mc), mc));
+            if (s <= 0) return s < 0 ? 0 : -1;
+        }
+        if (bk < 0 || P < Pthr - tP) return 1;
+        const gdt_d2 X = L.X64[bk];
+        const double qx = X.x - vx, qy = X.y - vy;
+        const double M = GDT_FMAX(mc, GDT_FMAX(fabs(qx), fabs(qy)));
+        const double e = gdt_dd_err(Lbox, M);
+        const GdtDDVec b = dd(bk, qx, qy);
+        const int s = wrap ? gdt_dd_sign(gdt_dd_incircle(a, b, c), gdt_dd_tol4(e, M))
+                           : gdt_dd_sign(gdt_dd_dist_cmp(c, b), 2. * gdt_dd_tol2(e, M));
+        return s == 0 ? -1 : (s < 0 ? 1 : 0);
+    };
     auto visit = [&](int k, const gdt_d2 X) {
         const double px = X.x - vx, py = X.y - vy;
         const double cc = gdt_dist2_64(px, py);
         const double O = gdt_orient64(ax, ay, px, py);
         const double P = gdt_incircle_cc64(K, px, py, cc);
+        if constexpr (CERT) {
+            if ((O >= Othr - tO) & (P <= Pthr + tP) & (k != ex) & (k != st.iv)) {
+                const bool sure = (O > Othr + tO) & ((P < Pthr - tP) | (bk < 0));
+                const int d = sure ? 1 : decide_dd(k, px, py, O, P);
+                if (d == 1) {
+                    bk = k;
+                    K.k0 = O + nnf;
+                    K.kx = fma(cc, ay, -(aa * py));
+                    K.ky = fma(aa, px, -(cc * ax));
+                    Pthr = nnf * cc;
+                } else if (d < 0) {
+                    bk = GDT_TIE;
+                    Pthr = -1e300;
+                }
+            }
+            return;
+        }
         // one branch, taken only for a new best (or an exact tie)
         if ((O > Othr) & (P <= Pthr) & (k != ex)) {
             const bool t = P == Pthr;
@@ -597,7 +666,15 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
                         const gdt_d2 X = L.X64[pk];
                         const double px = X.x - vx, py = X.y - vy;
                         const double P = gdt_incircle_cc64(K, px, py, gdt_dist2_64(px, py));
-                        if (P < Pthr) win = pk;
+                        if constexpr (CERT) {
+                            if (P < Pthr - tP) {
+                                win = pk;
+                            } else if (P <= Pthr + tP) {
+                                // (both lanes' bests are certainly left of v->a)
+                                const int d = decide_dd(pk, px, py, 1e300, P);
+                                win = d == 1 ? pk : (d < 0 ? GDT_TIE : bk);
+                            }
+                        } else if (P < Pthr) win = pk;
                         else if (P == Pthr) win = GDT_TIE;
                     }
                 }
@@ -633,6 +710,7 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     // nearest neighbour: the 3x3 block; successor: the 5x5 block, clipped to
     // the columns that may hold points left of v->a
     int hs = pre ? ph : (wrap ? GDT_SCAN0 : GDT_SCAN_NN);
+    set_region(hs);
     const double ox = gdt_cell_offset(vx, wx, S.bsx), oy = gdt_cell_offset(vy, wy, S.bsy);
     const GdtClip cl = gdt_left_clip(wrap, (float)ax, (float)ay, (float)ox, (float)oy,
                                      (float)S.bsx, (float)S.bsy, 1e-3f);
@@ -648,6 +726,7 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     pair_reduce();
     if (bk < 0 && hs < GDT_SCAN) {
         if (!ext) return STEP_DEFER;
+        set_region(GDT_SCAN);
         npred += gdt_lds_block(L, wx, wy, -GDT_SCAN, GDT_SCAN, -GDT_SCAN, GDT_SCAN, hs, visit_k);
         hs = GDT_SCAN;
     }
@@ -663,24 +742,40 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     auto certify = [&]() {
         best();
         const double cov = (double)hs * GDT_FMIN(S.bsx, S.bsy) + st.covb;
+        bool sure = true;       // (CERT: the circle is known to within its margins)
         ok = boxed = false;
         if (bk >= 0 && K.k0 > 1e-6 * (fabs(ax * by) + fabs(ay * bx))) {
             const double i2k = gdt_rcp64(2. * K.k0);
             const double qx = -K.kx * i2k, qy = -K.ky * i2k;
             const double R2 = wrap ? qx * qx + qy * qy : bd2;
             const double rad = gdt_sqrt64(R2) * (1.0 + 1e-9);
-            const double m = 1e-6 * (fabs(qx) + fabs(qy) + rad) + 1e-9 * S.bsx;
+            double m = 1e-6 * (fabs(qx) + fabs(qy) + rad) + 1e-9 * S.bsx;
+            if constexpr (CERT) {
+                // the exact circle's centre and radius differ from these by at
+                // most (the error of Kx, Ky + 2 |q| that of K0) / (2 K0) each
+                const double M = GDT_FMAX(ma, GDT_FMAX(fabs(bx), fabs(by)));
+                const double e = gdt_x_err(Lbox, M), eK0 = wrap ? gdt_x_tol2(e, M) : 0.;
+                const double eq = wrap ? 2. * (24. * e * M * M + 2. * rad * eK0) * i2k : 2. * e;
+                m += 2. * eq;
+                // (and, as in the per-point routine, the search radius covers it)
+                const double cmax = (double)S.rmax * GDT_FMIN(S.bsx, S.bsy) + st.covb -
+                                    (wrap ? 0. : 4. * gdt_x_err(Lbox, (S.rmax + 1) * S.bsx));
+                sure = K.k0 > 4. * eK0 && eq <= 1e-7 * cov &&
+                       (wrap ? 4. : 1.) * R2 <= cmax * cmax * (1.0 - 2e-6);
+            }
             gdt_circle_cells<double>(qx - m, qx + m, qy - m, qy + m, rad, ox, oy, S.ibsx, S.ibsy,
                                      1e-3, dx0, dx1, dy0, dy1);
             ok = (dx0 >= -hs && dx1 <= hs && dy0 >= -hs && dy1 <= hs) ||
                  (cov > 0. && (wrap ? 4. : 1.) * R2 <= cov * cov * (1.0 - 1e-6));
-            boxed = true;
+            ok = ok && sure;
+            boxed = sure;
         }
     };
     certify();
     if (!ok && !ext) return STEP_DEFER;
     // a box leaving the window: the full block first (it lies in the window)
     if (!ok && hs < GDT_SCAN && !(boxed && gdt_in_window(S, st.c0, dx0, dx1, dy0, dy1))) {
+        set_region(GDT_SCAN);
         npred += gdt_lds_block(L, wx, wy, -GDT_SCAN, GDT_SCAN, -GDT_SCAN, GDT_SCAN, hs, visit_k);
         hs = GDT_SCAN;
         certify();
@@ -688,6 +783,10 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     if (!ok && boxed && gdt_in_window(S, st.c0, dx0, dx1, dy0, dy1)) {
         // the rest of the circle's cell box, left of v->a, outside the scanned
         // square (every later best's circle lies inside)
+        if constexpr (CERT) {
+            const int h0 = dx0 < dy0 ? dx0 : dy0, h1 = dx1 > dy1 ? dx1 : dy1;
+            set_region(-h0 > h1 ? -h0 : h1);
+        }
         for (int dy = dy0; dy <= dy1;) {
             const unsigned ne = gdt_box_rows(L, st.c0, dy, dy1, dx0, dx1, hs, cl, st.tbl, sub, W);
             gdt_scan_tbl(st.tbl, ne, load, visit);
@@ -701,13 +800,26 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     return STEP_RUN;
 }
 
-template <int W = 1>
+// Whether the exact mode's bounds hold for caller point i (its coordinates
+// within four box lengths of the box); others go on to the per-point routine,
+// which reports them.
+GDT_HD inline bool gdt_tile_x_range(const GdtSet& S, const GdtRingIO& io, int i)
+{
+    const gdt_d2 p = io.xy[i];
+    return fabs(p.x) <= 4. * S.lx && fabs(p.y) <= 4. * S.ly;
+}
+
+template <int W = 1, bool CERT = false>
 GDT_HD inline int gdt_tile_step_f64(const GdtSet& S, const GdtTileLds& L, const GdtRingIO& io,
                                     GdtTileLane<double>& st, unsigned& npred, int sub = 0)
 {
     int bk;
     double bx, by;
-    const int rc = gdt_tile_search_f64<W>(S, L, st, npred, sub, true, bk, bx, by);
+    if constexpr (CERT) {
+        if (st.ak < 0 && !gdt_tile_x_range(S, io, L.orig[st.iv])) return STEP_DEFER;
+    }
+    const int rc = gdt_tile_search_f64<W, CERT>(S, L, st, npred, sub, true, bk, bx, by, nullptr, 0,
+                                                GDT_SCAN0, &io);
     if (rc != STEP_RUN) return rc;
     return gdt_tile_advance<double>(L, io, st, st.ak >= 0, bk, bx, by);
 }
@@ -1010,7 +1122,8 @@ GDT_HD inline GdtRingResult gdt_tile_ring(const GdtSet& S, const GdtTileWin& w, 
         GdtTileLane<double> st;
         gdt_tile_lane_init<double>(w, L, j, io, S, st);
         st.tbl = tbl;
-        while (rc == STEP_RUN) rc = gdt_tile_step_f64<1>(S, L, io, st, res.npred);
+        while (rc == STEP_RUN)
+            rc = gdt_tile_step_f64<1, PREC == GDT_EXACT>(S, L, io, st, res.npred);
         res.count = st.count;
     }
     if (rc == STEP_DEFER) res.err = ERR_DEFER;

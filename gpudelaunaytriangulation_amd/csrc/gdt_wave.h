@@ -102,6 +102,20 @@ struct GdtWaveHost {
                 if (gdt_wave_better<TIES>(wrap, ax, ay, t, lb[i], lb[i + off])) lb[i] = lb[i + off];
         return lb[0];
     }
+    // ring() with the comparison better(best, candidate) given.
+    template <class Fn, class Better>
+    GdtWaveBest ring_by(const GdtWaveBest& start, Fn& lane_fn, Better& better)
+    {
+        GdtWaveBest lb[GDT_WAVE];
+        for (int l = 0; l < GDT_WAVE; ++l) {
+            lb[l] = start;
+            lane_fn(l, lb[l]);
+        }
+        for (int off = GDT_WAVE / 2; off > 0; off >>= 1)
+            for (int i = 0; i < off; ++i)
+                if (better(lb[i], lb[i + off])) lb[i] = lb[i + off];
+        return lb[0];
+    }
 };
 
 // One point's ring.  `lead` is true on the one lane that writes the row.

@@ -31,6 +31,16 @@ struct GdtWaveDev {
     __device__ GdtWaveBest ring(const GdtWaveBest& start, bool wrap, double ax, double ay,
                                 GdtTieIds& t, Fn& fn)
     {
+        auto better = [&](const GdtWaveBest& b, const GdtWaveBest& c) {
+            return gdt_wave_better<TIES>(wrap, ax, ay, t, b, c);
+        };
+        const GdtWaveBest g = ring_by(start, fn, better);
+        if constexpr (!TIES) t.tie = __ballot(t.tie) != 0;
+        return g;
+    }
+    template <class Fn, class Better>
+    __device__ GdtWaveBest ring_by(const GdtWaveBest& start, Fn& fn, Better& better)
+    {
         GdtWaveBest m = start;
         fn(lane, m);
 #pragma unroll
@@ -40,15 +50,13 @@ struct GdtWaveDev {
             p.x = __shfl_down(m.x, off, 64);
             p.y = __shfl_down(m.y, off, 64);
             p.d2 = __shfl_down(m.d2, off, 64);
-            if (lane < off && gdt_wave_better<TIES>(wrap, ax, ay, t, m, p)) m = p;
+            if (lane < off && better(m, p)) m = p;
         }
         GdtWaveBest g;
         g.k = __shfl(m.k, 0, 64);
         g.x = __shfl(m.x, 0, 64);
         g.y = __shfl(m.y, 0, 64);
         g.d2 = __shfl(m.d2, 0, 64);
-        if constexpr (!TIES) t.tie = __ballot(t.tie) != 0;
         return g;
     }
 };
-

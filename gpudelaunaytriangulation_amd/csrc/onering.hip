@@ -8,7 +8,7 @@
 // (DelaunayGPU.cu:649-675, 981-1006) and their masked repair variants
 // (DelaunayGPU.cu:611-640, 945-975), which instead launch every point and
 // mask most of them out.
-#include "gdt_exact_ring.h"
+#include "gdt_exact_wave.h"
 #include "gdt_kernels.h"
 #include "gdt_wavedev.h"
 
@@ -69,24 +69,19 @@ __global__ __launch_bounds__(1024) void k_one_ring(const GdtSet* __restrict__ se
     one_ring_lane<PREC>(active, S, S.p0 + li, io, counts, status, counters, defer);
 }
 
-// Worklist of slots (count in device memory): grid-stride, set found per lane.
-// Entries [skip, *worklen) of the list are processed.
+// Entries [first, len) of a slot list, one lane each over the grid, set found
+// per lane.
 template <int PREC>
-__global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict__ sets, int nsets,
-                                                        const int* __restrict__ worklist,
-                                                        const uint32_t* __restrict__ worklen,
-                                                        int skip, GdtRingIO io,
-                                                        int* __restrict__ counts,
-                                                        int* __restrict__ status,
-                                                        unsigned long long* __restrict__ counters,
-                                                        int* __restrict__ defer)
+__device__ inline void one_ring_lanes(const GdtSet* __restrict__ sets, int nsets,
+                                      const int* __restrict__ worklist, int first, int len,
+                                      const GdtRingIO& io, int* __restrict__ counts,
+                                      int* __restrict__ status,
+                                      unsigned long long* __restrict__ counters,
+                                      int* __restrict__ defer)
 {
-    const int len = max((int)*worklen - skip, 0);
-    worklist += skip;
     const int stride = gridDim.x * blockDim.x;
-    const int first = blockIdx.x * blockDim.x + threadIdx.x;
     // uniform trip count per wave so the reductions see every lane
-    const int wave_first = first - (int)(threadIdx.x & 63);
+    const int wave_first = first + (int)(blockIdx.x * blockDim.x + (threadIdx.x & ~63u));
     for (int base = wave_first; base < len; base += stride) {
         const int t = base + (int)(threadIdx.x & 63);
         const bool active = t < len;
@@ -100,20 +95,39 @@ __global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict
     }
 }
 
-// Deferred points, one wavefront per point (FP64 in both precision paths):
-// list entries [0, min(*worklen, cap)), grid-stride over the waves.
-__global__ __launch_bounds__(256) void k_one_ring_wave(const GdtSet* __restrict__ sets, int nsets,
-                                                       const int* __restrict__ worklist,
-                                                       const uint32_t* __restrict__ worklen,
-                                                       int cap, GdtRingIO io,
-                                                       int* __restrict__ counts,
-                                                       int* __restrict__ status,
-                                                       unsigned long long* __restrict__ counters)
+// Worklist of slots (count in device memory), one lane each.
+template <int PREC>
+__global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict__ sets, int nsets,
+                                                        const int* __restrict__ worklist,
+                                                        const uint32_t* __restrict__ worklen,
+                                                        GdtRingIO io, int* __restrict__ counts,
+                                                        int* __restrict__ status,
+                                                        unsigned long long* __restrict__ counters,
+                                                        int* __restrict__ defer)
+{
+    one_ring_lanes<PREC>(sets, nsets, worklist, 0, (int)*worklen, io, counts, status, counters,
+                         defer);
+}
+
+// Deferred points (count in device memory): the first `cap` one wavefront
+// each, grid-stride over the waves (FP64 in both precision paths; exact
+// decisions in the exact mode), any beyond (dense clusters, exact lattices)
+// one lane each.  One launch for both: the second part is nearly always
+// empty, and as a kernel of its own cost its launch, 4.7 us of every call.
+template <int PREC>
+__global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restrict__ sets,
+                                                           int nsets,
+                                                           const int* __restrict__ worklist,
+                                                           const uint32_t* __restrict__ worklen,
+                                                           int cap, GdtRingIO io,
+                                                           int* __restrict__ counts,
+                                                           int* __restrict__ status,
+                                                           unsigned long long* __restrict__ counters)
 {
     const int lane = (int)(threadIdx.x & 63);
     const int wid = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const int nw = (int)((gridDim.x * blockDim.x) >> 6);
-    const int len = min((int)*worklen, cap);
+    const int all = (int)*worklen, len = min(all, cap);
     GdtWaveDev w;
     w.lane = lane;
     unsigned npred = 0, nsum = 0;
@@ -121,45 +135,57 @@ __global__ __launch_bounds__(256) void k_one_ring_wave(const GdtSet* __restrict_
     for (int t = wid; t < len; t += nw) {
         const int j = worklist[t];
         const GdtSet S = sets[gdt_set_of(sets, nsets, j)];
-        const GdtRingResult r = gdt_wave_ring(S, j, io, w, lane == 0);
+        GdtRingResult r;
+        if constexpr (PREC == GDT_EXACT)
+            r = gdt_wave_ring_exact(S, j, io, w, lane == 0);
+        else
+            r = gdt_wave_ring(S, j, io, w, lane == 0);
         npred += r.npred;
+        er |= r.err;
         if (lane == 0) {
             counts[io.perm[j]] = r.count;
             mx = max(mx, r.count);
-            er |= r.err;
             nsum += (unsigned)r.count;
         }
     }
-    mx = wave_max_i32(mx);
-    er = wave_or_i32(er);
-    npred = wave_sum_u32(npred);
-    nsum = wave_sum_u32(nsum);
-    if (lane == 0) {
-        if (mx > 0) atomicMax(&status[ST_REQUIRED], mx);
-        if (er) atomicOr(&status[ST_ERRFLAGS], er);
-        if (npred) atomicAdd(&counters[CT_PRED], (unsigned long long)npred);
-        if (nsum) atomicAdd(&counters[CT_NBRSUM], (unsigned long long)nsum);
+    if (wid < len) {        // (wave-uniform)
+        mx = wave_max_i32(mx);
+        er = wave_or_i32(er);
+        npred = wave_sum_u32(npred);
+        nsum = wave_sum_u32(nsum);
+        if (lane == 0) {
+            if (mx > 0) atomicMax(&status[ST_REQUIRED], mx);
+            if (er) atomicOr(&status[ST_ERRFLAGS], er);
+            if (npred) atomicAdd(&counters[CT_PRED], (unsigned long long)npred);
+            if (nsum) atomicAdd(&counters[CT_NBRSUM], (unsigned long long)nsum);
+        }
     }
+    if (all > cap)
+        one_ring_lanes<PREC>(sets, nsets, worklist, cap, all, io, counts, status, counters,
+                             nullptr);
 }
 
-hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets, int total_n,
+hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s)
 {
-    // the count is read on the device: the first GDT_WAVE_CAP one wavefront
-    // each, any beyond (dense clusters) one lane each
+    // (the count is read on the device)
     const uint32_t* ndefer = reinterpret_cast<const uint32_t*>(status + ST_NDEFER);
-    hipLaunchKernelGGL(k_one_ring_wave, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets, nsets, defer,
-                       ndefer, GDT_WAVE_CAP, io, counts, status, counters);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return e;
-    return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer, ndefer,
-                               GDT_WAVE_CAP, total_n, io, counts, status, counters, nullptr, s);
+    if (precision == 32)
+        hipLaunchKernelGGL(k_one_ring_deferred<32>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
+                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
+    else if (precision == GDT_EXACT)
+        hipLaunchKernelGGL(k_one_ring_deferred<GDT_EXACT>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s,
+                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
+    else
+        hipLaunchKernelGGL(k_one_ring_deferred<64>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
+                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
+    return hipGetLastError();
 }
 
 hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                const GdtChunk* chunks, int nch, int block, const int* worklist,
-                               const uint32_t* worklen, int skip, int max_work,
+                               const uint32_t* worklen, int max_work,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s)
 {
@@ -176,18 +202,17 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                counts, status, counters, defer);
         return hipGetLastError();
     }
-    max_work -= skip;
     if (max_work <= 0) return hipSuccess;
     int grid = (max_work + block - 1) / block;
     if (grid > 4096) grid = 4096;
     if (precision == 32)
         hipLaunchKernelGGL(k_one_ring_list<32>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, skip, io, counts, status, counters, defer);
+                           worklist, worklen, io, counts, status, counters, defer);
     else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_list<GDT_EXACT>, dim3(grid), dim3(block), 0, s, d_sets,
-                           nsets, worklist, worklen, skip, io, counts, status, counters, defer);
+                           nsets, worklist, worklen, io, counts, status, counters, defer);
     else
         hipLaunchKernelGGL(k_one_ring_list<64>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, skip, io, counts, status, counters, defer);
+                           worklist, worklen, io, counts, status, counters, defer);
     return hipGetLastError();
 }

@@ -24,11 +24,17 @@ namespace GDT_TS_NS {
 // the block gathers first into a bit mask in LDS (status[ST_NFLAGGED] += their
 // count).  A tile with none exits before staging.  The points of a window that does not fit the LDS budget, or of a
 // grid too small for the scan block, and points with a step whose circle
-// leaves the window, are appended to `defer` and handled by k_one_ring_wave
+// leaves the window, are appended to `defer` and handled by k_one_ring_deferred
 // in the next launch.  With W = 2 or 4 (FP64) neighbouring lanes share each
 // point, each scanning its part of every row (a list leaves most lanes of a
 // block without a point otherwise, and a small grid leaves most of the chip
 // idle; the launcher takes W from the caller).
+// PREC = GDT_EXACT: the FP64 steps with every decision certified
+// (gdt_tile_search_f64, CERT), bound as they are by the lanes' chains of steps;
+// all its deferred points go to the next launch, where a wavefront per point
+// takes the expansions.  Kernel times against the per-point exact kernel: 2^18
+// random points 290 us (2,427 us), 65,536 points of a square lattice off by
+// 1e-13 207 us + 147 us deferred (4,171 us).
 
 // The tile's flagged slots (flags mode): slot T0 + 64 w + b is flagged when bit
 // b of mask[w] is set; pre[w] = flagged slots before word w.
@@ -91,7 +97,7 @@ __device__ inline void ring_block_totals(int mx, int er, unsigned npred, unsigne
 }
 
 template <int PREC, int W>
-__global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict__ sets, const GdtChunk* __restrict__ tiles,
+__global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_tile(const GdtSet* __restrict__ sets, const GdtChunk* __restrict__ tiles,
                      const int* __restrict__ list, const uint32_t* __restrict__ lscan,
                      const int* __restrict__ flags, const int* __restrict__ halt,
                      GdtRingIO io, int* __restrict__ counts, int* __restrict__ status,
@@ -178,6 +184,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
     // iteration; a lane whose point is finished takes the next one, so a
     // wave's iterations track the total number of steps, not the longest ring.
     static_assert(W == 1 || W == 2 || (W == 4 && PREC == 64), "1, 2 or (FP64) 4 lanes per point");
+    static_assert(PREC == 32 || PREC == 64 || PREC == GDT_EXACT, "a precision code");
     if (tid == 0) {
         s_next = Q0 + nt / W;
         s_dn = 0u;
@@ -199,12 +206,13 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
             if constexpr (PREC == 32)
                 rc = gdt_tile_step_f32<W>(S, L, io, st, npred, nfb, sub);
             else
-                rc = gdt_tile_step_f64<W>(S, L, io, st, npred, sub);
+                rc = gdt_tile_step_f64<W, PREC == GDT_EXACT>(S, L, io, st, npred, sub);
             // (both lanes of a pair end each step in the same state; the first reports)
             if (rc != STEP_RUN && sub == 0) {
                 if (rc == STEP_DEFER) {
                     // the block's own waves finish it after the tile (below)
-                    const uint32_t dpos = atomicAdd(&s_dn, 1u);
+                    // (the exact mode's go to the per-point routine)
+                    const uint32_t dpos = PREC == GDT_EXACT ? GDT_TILE_DEFER : atomicAdd(&s_dn, 1u);
                     if (dpos < GDT_TILE_DEFER) {
                         s_dlist[dpos] = j;
                     } else {
@@ -234,6 +242,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
             }
         }
     }
+    if constexpr (PREC != GDT_EXACT) {
     // Points whose circle left the window: one wavefront each, read from
     // global memory (gdt_wave_ring), by this block's waves while other blocks
     // still run their tiles.
@@ -247,7 +256,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
             const int jd = s_dlist[t];
             // (built without the tie rule and for rectangles only, which would
             // cost this kernel's main loop registers: a point with an exact tie
-            // goes to k_one_ring_wave)
+            // goes to k_one_ring_deferred)
             const GdtRingResult r = gdt_wave_ring<false, false>(S, jd, io, wv, wv.lane == 0);
             npred += r.npred;
             if (r.err & ERR_TIE) {
@@ -262,6 +271,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
                 nsum += (unsigned)r.count;
             }
         }
+    }
     }
     ring_block_totals(mx, er, npred, nfb, nsum, status, counters);
 }
@@ -285,8 +295,9 @@ __global__ __launch_bounds__(1024) void k_one_ring_tile(const GdtSet* __restrict
 // block of more than 64 entries runs the sequential steps in lane 0.  Blocks
 // (tile, y) share a tile's points: wave w of block y takes the points
 // T0 + y nw + w + m gridDim.y nw.  Deferred points go to `defer` (handled by
-// k_one_ring_wave in the next launch).
-__global__ __launch_bounds__(1024) void k_one_ring_star(const GdtSet* __restrict__ sets,
+// k_one_ring_deferred in the next launch).
+template <bool CERT>
+__global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star(const GdtSet* __restrict__ sets,
                                                         const GdtChunk* __restrict__ tiles,
                                                         GdtRingIO io, int* __restrict__ counts,
                                                         int* __restrict__ status,
@@ -354,14 +365,16 @@ __global__ __launch_bounds__(1024) void k_one_ring_star(const GdtSet* __restrict
                 sl.ay = X.y - st.vy;
             }
             double bx, by;
-            rc = gdt_tile_search_f64<1>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
-                                        (unsigned)tot, ph);
+            rc = gdt_tile_search_f64<1, CERT>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
+                                              (unsigned)tot, ph, &io);
         }
         int res = STEP_RUN, count = 0;
-        if (tot > 64) {
+        if (CERT && !gdt_tile_x_range(S, io, L.orig[st.iv])) {
+            res = STEP_DEFER;
+        } else if (tot > 64) {
             if (lane == 0) {
                 int r = STEP_RUN;
-                while (r == STEP_RUN) r = gdt_tile_step_f64<1>(S, L, io, st, npred);
+                while (r == STEP_RUN) r = gdt_tile_step_f64<1, CERT>(S, L, io, st, npred);
                 res = r;
                 count = st.count;
             }
@@ -373,7 +386,8 @@ __global__ __launch_bounds__(1024) void k_one_ring_star(const GdtSet* __restrict
                 // not certified over the block: lane 0 runs the full search
                 if (lane == 0) {
                     double bx, by;
-                    nrc = gdt_tile_search_f64<1>(S, L, st, npred, 0, true, nn, bx, by);
+                    nrc = gdt_tile_search_f64<1, CERT>(S, L, st, npred, 0, true, nn, bx, by,
+                                                       nullptr, 0, GDT_SCAN0, &io);
                 }
                 nrc = __shfl(nrc, 0, 64);
                 nn = __shfl(nn, 0, 64);
@@ -399,7 +413,8 @@ __global__ __launch_bounds__(1024) void k_one_ring_star(const GdtSet* __restrict
                             sl.ax = X.x - st.vx;
                             sl.ay = X.y - st.vy;
                             double bx, by;
-                            r = gdt_tile_search_f64<1>(S, L, sl, npred, 0, true, b, bx, by);
+                            r = gdt_tile_search_f64<1, CERT>(S, L, sl, npred, 0, true, b, bx, by,
+                                                             nullptr, 0, GDT_SCAN0, &io);
                         }
                         if (__shfl(r, 0, 64) != STEP_RUN) {
                             res = STEP_DEFER;
@@ -437,7 +452,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_star(const GdtSet* __restrict
 
 hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,
                                     const GdtChunk* tiles, int ntiles, int block, int lanes,
-                                    int total_n, const int* list, const uint32_t* lscan,
+                                    const int* list, const uint32_t* lscan,
                                     const int* flags, const int* halt,
                                     const GdtRingIO& io, int* counts, int* status,
                                     unsigned long long* counters, int* defer,
@@ -448,7 +463,16 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     const size_t tbl = (5 * (size_t)block + 1) * sizeof(uint32_t);
     // (the FP32-filtered step shares a point between at most two lanes)
     const bool two = lanes == 2 || (lanes == 4 && precision == 32);
-    if (precision == 64 && lanes == 4)
+    if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) block = GDT_XTILE_BLOCK;
+    if (precision == GDT_EXACT && (lanes == 2 || lanes == 4))
+        hipLaunchKernelGGL((k_one_ring_tile<GDT_EXACT, 2>), dim3(ntiles), dim3(block), tbl, s,
+                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
+                           defer);
+    else if (precision == GDT_EXACT)
+        hipLaunchKernelGGL((k_one_ring_tile<GDT_EXACT, 1>), dim3(ntiles), dim3(block), tbl, s,
+                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
+                           defer);
+    else if (precision == 64 && lanes == 4)
         hipLaunchKernelGGL((k_one_ring_tile<64, 4>), dim3(ntiles), dim3(block), tbl, s, d_sets,
                            tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
     else if (precision == 32 && two)
@@ -466,12 +490,13 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
-    return gdt_launch_deferred(precision, d_sets, nsets, total_n, io, counts, status, counters,
+    return gdt_launch_deferred(precision, d_sets, nsets, io, counts, status, counters,
                                defer, s);
 }
 
-hipError_t gdt_launch_one_ring_star(const GdtSet* d_sets, int nsets, const GdtChunk* tiles,
-                                    int ntiles, int nsplit, int block, int total_n,
+hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,
+                                    const GdtChunk* tiles,
+                                    int ntiles, int nsplit, int block,
                                     const GdtRingIO& io, int* counts, int* status,
                                     unsigned long long* counters, int* defer,
                                     hipEvent_t after_tile, hipStream_t s)
@@ -480,12 +505,18 @@ hipError_t gdt_launch_one_ring_star(const GdtSet* d_sets, int nsets, const GdtCh
     if (block < 64 || block > 1024 || (block & 63) || nsplit < 1 || nsplit > 65535)
         return hipErrorInvalidValue;
     const size_t tbl = (STAR_TBL * (size_t)block + 1) * sizeof(uint32_t);
-    hipLaunchKernelGGL(k_one_ring_star, dim3(ntiles, nsplit), dim3(block), tbl, s, d_sets, tiles,
-                       io, counts, status, counters, defer);
+    if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) return hipErrorInvalidValue;
+    if (precision == GDT_EXACT)
+        hipLaunchKernelGGL(k_one_ring_star<true>, dim3(ntiles, nsplit), dim3(block), tbl, s, d_sets,
+                           tiles, io, counts, status, counters, defer);
+    else
+        hipLaunchKernelGGL(k_one_ring_star<false>, dim3(ntiles, nsplit), dim3(block), tbl, s,
+                           d_sets, tiles, io, counts, status, counters, defer);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
-    return gdt_launch_deferred(64, d_sets, nsets, total_n, io, counts, status, counters, defer, s);
+    return gdt_launch_deferred(precision == GDT_EXACT ? GDT_EXACT : 64, d_sets, nsets, io, counts,
+                               status, counters, defer, s);
 }
 
 }  // namespace GDT_TS_NS
