@@ -105,6 +105,11 @@ struct gdt_context {
     }
 };
 
+// Cell keys of a call (at most), and the search radius the windows of the LDS
+// tile kernels need (their widest scan block).
+#define GDT_MAX_KEYS 0x7ffffff0LL
+#define GDT_MIN_TILE_RMAX 3
+
 #define GDT_CHECK(expr)                                   \
     do {                                                  \
         hipError_t e_ = (expr);                           \
@@ -145,7 +150,7 @@ static int configure(gdt_context* c, std::vector<GdtSet> sets)
         s.p0 = p0;
         s.c0 = c0;
         p0 += s.n;
-        if ((long long)c0 + s.nkeys > 0x7ffffff0LL) return GDT_ERR_INVALID;
+        if ((long long)c0 + s.nkeys > GDT_MAX_KEYS) return GDT_ERR_INVALID;
         c0 += s.nkeys;
     }
     if (same_sets(sets, c->sets) && c->d_sets.p) return GDT_OK;
@@ -256,8 +261,8 @@ static bool box_ok(const double b[4], int words)
     return std::isfinite(det) && std::fabs(det) > 0.;
 }
 
-// General boxes run the row-major cell order and FP64 predicates (the LDS tile
-// kernels and the FP32 filter's bounds are for rectangular cells).
+// General boxes run FP64 predicates (the FP32 filter's bounds are for
+// rectangular cells).
 static bool any_general(const gdt_context* c)
 {
     for (const auto& s : c->sets)
@@ -277,23 +282,60 @@ static bool ring_precision_ok(int p)
 }
 static_assert((int)GDT_PREC_EXACT == (int)GDT_EXACT, "one code for the exact mode");
 
+// The sets of a call (set s = caller points [offsets[s], offsets[s+1]) in box s
+// of `boxes`, words per box 2 or 4 as box_of): in the configured cell order,
+// tiled orders with the tile edge of the configuration or the automatic one.
+// General boxes take the tile kernels too (2^20 points in a box sheared by 0.31:
+// 581 us per call, 2,841 with the row-major per-point kernel).
+// Sets of which one is a general box keep the row-major order where the tile
+// kernels could not take them: a grid smaller than the windows' scan block
+// (every point of such a tile is handed on), or tiles whose padding outgrows
+// the cell keys.
+static std::vector<GdtSet> sets_of(const gdt_context* c, int nsets, const int* offsets,
+                                   const double* boxes, double cell_size, int words)
+{
+    std::vector<GdtSet> sets((size_t)nsets);
+    bool general = false;
+    auto make = [&](int tiled, int ts) {
+        for (int k = 0; k < nsets; ++k) {
+            double b[4];
+            box_of(boxes, words, k, b);
+            sets[(size_t)k] = gdt_make_set_box(offsets[k], offsets[k + 1] - offsets[k], 0, b,
+                                               cell_size * c->cfg.cell_scale, tiled, ts);
+            general = general || sets[(size_t)k].general;
+        }
+    };
+    make(c->cfg.tiled, GDT_TSHIFT_MAX);
+    if (general && c->cfg.tiled) {
+        long long keys = 0;
+        bool ok = true;
+        for (const auto& s : sets) {
+            keys += s.nkeys;
+            ok = ok && s.rmax >= GDT_MIN_TILE_RMAX;
+        }
+        if (!ok || keys > GDT_MAX_KEYS) {
+            make(0, GDT_TSHIFT_MAX);
+            return sets;
+        }
+    }
+    const int ts = tile_shift_for(c, sets);
+    if (ts != GDT_TSHIFT_MAX) make(c->cfg.tiled, ts);
+    return sets;
+}
+
 static int single_set_box(gdt_context* c, int n, const double* box, int words, double cell_size)
 {
-    if (n < 4 || !box_ok(box, words) || !(cell_size > 0.) || !std::isfinite(cell_size))
+    double b[4];
+    box_of(box, words, 0, b);
+    if (n < 4 || !box_ok(b, words) || !(cell_size > 0.) || !std::isfinite(cell_size))
         return GDT_ERR_INVALID;
-    const double a = cell_size * c->cfg.cell_scale;
-    if (!gdt_box_is_rect(box))
-        return configure(c, std::vector<GdtSet>(1, gdt_make_set_box(0, n, 0, box, a, 0)));
-    const double lx = box[0], ly = box[3];
-    std::vector<GdtSet> sets(1, gdt_make_set(0, n, 0, lx, ly, a, c->cfg.tiled, GDT_TSHIFT_MAX));
-    const int ts = tile_shift_for(c, sets);
-    if (ts != GDT_TSHIFT_MAX) sets[0] = gdt_make_set(0, n, 0, lx, ly, a, c->cfg.tiled, ts);
-    return configure(c, sets);
+    const int off[2] = {0, n};
+    return configure(c, sets_of(c, 1, off, box, cell_size, words));
 }
 
 static int single_set(gdt_context* c, int n, double lx, double ly, double cell_size)
 {
-    const double b[4] = {lx, 0., 0., ly};
+    const double b[2] = {lx, ly};
     return single_set_box(c, n, b, 2, cell_size);
 }
 
@@ -305,31 +347,12 @@ static int batch_sets(gdt_context* c, int nsets, const int* offsets, const doubl
     if (nsets <= 0 || !offsets || !boxes || offsets[0] != 0 || !(cell_size > 0.) ||
         !std::isfinite(cell_size))
         return GDT_ERR_INVALID;
-    bool general = false;
     for (int k = 0; k < nsets; ++k) {
         double b[4];
         box_of(boxes, words, k, b);
         if (offsets[k + 1] - offsets[k] < 4 || !box_ok(b, words)) return GDT_ERR_INVALID;
-        general = general || !gdt_box_is_rect(b);
     }
-    const int tiled = general ? 0 : c->cfg.tiled;
-    std::vector<GdtSet> sets;
-    sets.reserve((size_t)nsets);
-    for (int k = 0; k < nsets; ++k) {
-        double b[4];
-        box_of(boxes, words, k, b);
-        sets.push_back(gdt_make_set_box(offsets[k], offsets[k + 1] - offsets[k], 0, b,
-                                        cell_size * c->cfg.cell_scale, tiled, GDT_TSHIFT_MAX));
-    }
-    const int ts = tile_shift_for(c, sets);
-    if (!general && ts != GDT_TSHIFT_MAX)
-        for (int k = 0; k < nsets; ++k) {
-            double b[4];
-            box_of(boxes, words, k, b);
-            sets[(size_t)k] = gdt_make_set_box(offsets[k], sets[(size_t)k].n, 0, b,
-                                               cell_size * c->cfg.cell_scale, tiled, ts);
-        }
-    return configure(c, sets);
+    return configure(c, sets_of(c, nsets, offsets, boxes, cell_size, words));
 }
 
 static int reset_status(gdt_context* c, hipStream_t s)
@@ -596,7 +619,9 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
     precision = eff_precision(c, precision);
     if ((rc = ring_chunks(c)) != GDT_OK) return rc;
     if ((rc = build_cells(c, d_xy, s, true)) != GDT_OK) return rc;
-    if (tiled_sets(c)) {
+    const bool general = any_general(c);
+    // (the exact mode refuses general boxes point by point, in the per-point kernel)
+    if (tiled_sets(c) && !(general && precision == GDT_PREC_EXACT)) {
         // A grid of at most one tile per CU runs one wave of blocks: each lane
         // (or lane group) then takes a single point (1024 threads for about
         // 1024 points of a 32x32 tile), so the block ends after its longest
@@ -615,17 +640,17 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
             int nsplit = (int)std::max(1LL, (avg + nw - 1) / nw);
             nsplit = std::min(nsplit, std::max(1, 4 * c->num_cu / c->ntch));
             GDT_CHECK(gdt_tiles::one_ring_star(ts, precision, c->d_sets.p, (int)c->sets.size(), c->tch.p,
-                                               c->ntch, nsplit, block,
+                                               c->ntch, nsplit, block, general,
                                                ring_io(c, d_nbrs, stride), d_counts, c->status.p,
                                                c->counters.p, c->defer.p,
                                                c->cfg.profile ? c->ev[2] : nullptr, s));
         } else {
-            c->stats.lanes = lanes == 4 && precision != GDT_PREC_FP64 ? 2 : lanes;
+            c->stats.lanes = lanes == 4 && (general || precision != GDT_PREC_FP64) ? 2 : lanes;
             const int one_each = std::min(1024, (1 << (2 * ts)) * lanes);
             const int block =
                 c->ntch <= c->num_cu ? std::max(tile_block(c), one_each) : tile_block(c);
             GDT_CHECK(gdt_tiles::one_ring(ts, precision, c->d_sets.p, (int)c->sets.size(),
-                                          c->tch.p, c->ntch, block, lanes, nullptr,
+                                          c->tch.p, c->ntch, block, lanes, general, nullptr,
                                           nullptr, nullptr, nullptr, ring_io(c, d_nbrs, stride),
                                           d_counts, c->status.p, c->counters.p, c->defer.p,
                                           c->cfg.profile ? c->ev[2] : nullptr, s));
@@ -730,14 +755,14 @@ static int test_triangles(gdt_context* c, const double* d_xy, int cap, hipStream
 }
 
 // Triangles of the current rings and their empty-circle test: with the tiled
-// cell order in one pass over the rings (no triangle array), else enumerate()
-// then test_triangles().  Leaves the triangle count in toff[n] and the sum of
-// counts in counters[CT_INSUM] either way.
+// cell order of rectangles in one pass over the rings (no triangle array),
+// else enumerate() then test_triangles().  Leaves the triangle count in
+// toff[n] and the sum of counts in counters[CT_INSUM] either way.
 static int triangles_and_test(gdt_context* c, const double* d_xy, const int* d_nbrs,
                               const int* d_counts, int stride, int cap, hipStream_t s)
 {
     const int n = c->total_n;
-    if (!tiled_sets(c)) {
+    if (!tiled_sets(c) || any_general(c)) {
         int rc;
         if ((rc = enumerate(c, d_nbrs, d_counts, stride, c->tris.p, cap, false, s)) != GDT_OK) return rc;
         return test_triangles(c, d_xy, cap, s);
@@ -815,7 +840,7 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
         GDT_CHECK(gdt_tiles::one_ring(c->sets[0].tshift, precision, c->d_sets.p,
                                       (int)c->sets.size(), c->tch.p, c->ntch, tile_block(c),
                                       c->cfg.repair_lanes ? c->cfg.repair_lanes : 2,
-                                      nullptr, nullptr, d_repair, c->halt,
+                                      any_general(c), nullptr, nullptr, d_repair, c->halt,
                                       ring_io(c, d_nbrs, stride), d_counts, c->status.p,
                                       c->counters.p, c->defer.p, nullptr, s));
         return GDT_OK;

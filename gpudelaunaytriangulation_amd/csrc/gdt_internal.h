@@ -351,7 +351,6 @@ inline void gdt_reduce_basis(double& ax, double& ay, double& bx, double& by)
 // cells binned in the unit-cell coordinates of the reduced basis: cell
 // counts from the thicknesses T of the unit cell across each pair of walls
 // (the rectangle's side lengths for a rectangle), by the rule of gdt_grid.
-// Row-major cell order (the LDS tile kernels handle rectangles only).
 // A rectangular box gives gdt_make_set's set.
 inline GdtSet gdt_make_set_box(int p0, int n, int c0, const double* box, double cell_size,
                                int tiled, int tshift = GDT_TILE_SHIFT)
@@ -361,7 +360,7 @@ inline GdtSet gdt_make_set_box(int p0, int n, int c0, const double* box, double 
     gdt_reduce_basis(ax, ay, bx, by);
     const double det = ax * by - ay * bx;
     const double tx = det / sqrt(bx * bx + by * by), ty = det / sqrt(ax * ax + ay * ay);
-    GdtSet s = gdt_make_set(p0, n, c0, tx, ty, cell_size, 0, tshift);
+    GdtSet s = gdt_make_set(p0, n, c0, tx, ty, cell_size, tiled, tshift);
     s.general = 1;
     s.lat[0] = ax; s.lat[1] = bx; s.lat[2] = ay; s.lat[3] = by;
     s.ilat[0] = by / det; s.ilat[1] = -bx / det; s.ilat[2] = -ay / det; s.ilat[3] = ax / det;

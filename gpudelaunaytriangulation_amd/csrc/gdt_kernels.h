@@ -103,6 +103,7 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
     namespace ns {                                                                                \
     hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles, int ntiles, int block, int lanes, \
+                                        bool general,                                            \
                                         const int* list, const uint32_t* lscan,                  \
                                         const int* flags, const int* halt,                       \
                                         const GdtRingIO& io, int* counts, int* status,           \
@@ -110,7 +111,7 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                         hipEvent_t after_tile, hipStream_t s);                   \
     hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles,                                   \
-                                        int ntiles, int nsplit, int block,                       \
+                                        int ntiles, int nsplit, int block, bool general,         \
                                         const GdtRingIO& io, int* counts, int* status,           \
                                         unsigned long long* counters, int* defer,                \
                                         hipEvent_t after_tile, hipStream_t s);                   \
@@ -146,7 +147,8 @@ hipError_t gdt_launch_test(const GdtSet* d_sets, int nsets, const int* tris, con
 // nothing with *halt set), one block per tile of the tiled cell order,
 // `lanes` (1, 2 or 4) lanes per point.  Points the tile kernel cannot finish
 // from LDS are deferred (gdt_launch_deferred over `defer`, a slot per point, count
-// in status[ST_NDEFER]).
+// in status[ST_NDEFER]).  general: the sets include general boxes (FP64, at
+// most two lanes; the star kernel too).
 //
 // The same rings of every point with one wavefront per point (the star
 // kernel, FP64 predicates): the lanes run the search steps from every
@@ -164,24 +166,24 @@ static_assert(GDT_TSHIFT_MIN == 4 && GDT_TSHIFT_MAX == 5, "a launcher per suppor
 
 namespace gdt_tiles {
 inline hipError_t one_ring(int tshift, int precision, const GdtSet* d_sets, int nsets,
-                           const GdtChunk* tiles, int ntiles, int block, int lanes,
+                           const GdtChunk* tiles, int ntiles, int block, int lanes, bool general,
                            const int* list, const uint32_t* lscan, const int* flags,
                            const int* halt, const GdtRingIO& io, int* counts, int* status,
                            unsigned long long* counters, int* defer, hipEvent_t after_tile,
                            hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_tile : ts5::gdt_launch_one_ring_tile)(
-        precision, d_sets, nsets, tiles, ntiles, block, lanes, list, lscan, flags, halt,
+        precision, d_sets, nsets, tiles, ntiles, block, lanes, general, list, lscan, flags, halt,
         io, counts, status, counters, defer, after_tile, s);
 }
 inline hipError_t one_ring_star(int tshift, int precision, const GdtSet* d_sets, int nsets,
                                 const GdtChunk* tiles, int ntiles, int nsplit, int block,
-                                const GdtRingIO& io, int* counts, int* status,
+                                bool general, const GdtRingIO& io, int* counts, int* status,
                                 unsigned long long* counters, int* defer, hipEvent_t after_tile,
                                 hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_star : ts5::gdt_launch_one_ring_star)(
-        precision, d_sets, nsets, tiles, ntiles, nsplit, block, io, counts, status, counters, defer,
+        precision, d_sets, nsets, tiles, ntiles, nsplit, block, general, io, counts, status, counters, defer,
         after_tile, s);
 }
 inline hipError_t ring_test(int tshift, const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,

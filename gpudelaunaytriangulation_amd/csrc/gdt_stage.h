@@ -51,7 +51,7 @@ __device__ inline void block_scan_lds(uint32_t* a, int n, uint32_t* wsum)
 // through L.orig, which its caller index then overwrites.  Without L.gstart
 // an entry's cell start is read again from the cell list (a cached read: the
 // block read it in phase 1), which keeps that array out of LDS.
-template <bool F32>
+template <bool F32, bool GEN = false>
 __device__ inline bool gdt_stage_window(const GdtSet& S, const GdtTileWin& w, const GdtRingIO& io,
                                         const GdtTileLds& L, uint32_t* wsum)
 {
@@ -115,8 +115,12 @@ __device__ inline bool gdt_stage_window(const GdtSet& S, const GdtTileWin& w, co
                 if (k < np) {
                     const int fx = cell[j] % GDT_WIN - GDT_FRAME, fy = cell[j] / GDT_WIN - GDT_FRAME;
                     gdt_d2 X;
-                    X.x = gdt_frame64(fx, S.bsx, o[j].x);
-                    X.y = gdt_frame64(fy, S.bsy, o[j].y);
+                    if constexpr (GEN) {
+                        X = gdt_frame64_gen(S, fx, fy, o[j]);
+                    } else {
+                        X.x = gdt_frame64(fx, S.bsx, o[j].x);
+                        X.y = gdt_frame64(fy, S.bsy, o[j].y);
+                    }
                     L.X64[k] = X;
                     L.orig[k] = p[j];
                     if (F32) {

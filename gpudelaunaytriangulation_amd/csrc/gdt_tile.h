@@ -91,6 +91,15 @@ GDT_HD inline void gdt_tile_count(const GdtSet& S, const GdtTileWin& w, int c,
     cnt = e - b;
 }
 
+// Frame coordinates of a point at offset off in the cell (fx, fy) of the
+// frame, every box shape (rectangles: gdt_frame64 per axis, bit for bit).
+GDT_HD inline gdt_d2 gdt_frame64_gen(const GdtSet& S, int fx, int fy, const gdt_d2& off)
+{
+    gdt_d2 X;
+    X.x = fma((double)fy, S.ey_x, (double)fx * S.ex_x) + off.x;
+    X.y = fma((double)fx, S.ex_y, (double)fy * S.ey_y) + off.y;
+    return X;
+}
 GDT_HD inline double gdt_frame64(int f, double bs, double off) { return (double)f * bs + off; }
 GDT_HD inline float gdt_frame32(int f, float bs, float off) { return (float)f * bs + off; }
 
@@ -447,6 +456,16 @@ GDT_HD inline void gdt_tile_lane_init<double>(const GdtTileWin& w, const GdtTile
     st.row = io.nbrs + (size_t)i * (size_t)io.stride;
 }
 
+// The FP64 lane of a point in a general box.
+GDT_HD inline void gdt_tile_lane_init_gen(const GdtTileWin& w, const GdtTileLds& L, int j,
+                                          const GdtRingIO& io, const GdtSet& S,
+                                          GdtTileLane<double>& st)
+{
+    gdt_tile_lane_init<double>(w, L, j, io, S, st);
+    const gdt_d2 ov = io.off64[j];
+    st.covb = gdt_cover0(S, ov.x, ov.y);
+}
+
 template <>
 GDT_HD inline void gdt_tile_lane_init<float>(const GdtTileWin& w, const GdtTileLds& L, int j,
                                              const GdtRingIO& io, const GdtSet& S,
@@ -528,7 +547,11 @@ GDT_HD inline int gdt_tile_advance(const GdtTileLds& L, const GdtRingIO& io, Gdt
 // the grid -- and from the double-double value of the caller's coordinates
 // (*xio) outside that one's; a sign neither certifies hands the point on
 // (GDT_TIE), as an exact tie does.
-template <int W = 1, bool CERT = false>
+// GEN (general boxes): the cells are parallelograms.  The left half-plane's
+// columns and the circle's cells are found in cell coordinates (an affine map
+// of positive determinant keeps "left of"; a disc of radius R spans R times
+// the norms of the map's rows), everything else is as for rectangles.
+template <int W = 1, bool CERT = false, bool GEN = false>
 GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
                                       const GdtTileLane<double>& st, unsigned& npred, int sub,
                                       bool ext, int& bk, double& bx, double& by,
@@ -711,9 +734,20 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     // the columns that may hold points left of v->a
     int hs = pre ? ph : (wrap ? GDT_SCAN0 : GDT_SCAN_NN);
     set_region(hs);
-    const double ox = gdt_cell_offset(vx, wx, S.bsx), oy = gdt_cell_offset(vy, wy, S.bsy);
-    const GdtClip cl = gdt_left_clip(wrap, (float)ax, (float)ay, (float)ox, (float)oy,
-                                     (float)S.bsx, (float)S.bsy, 1e-3f);
+    // v's offset in its cell (GEN: its cell coordinates there, in [0, 1])
+    double ox, oy;
+    GdtClip cl;
+    if constexpr (GEN) {
+        ox = fma(S.rxx, vx, S.rxy * vy) - (double)(wx - GDT_FRAME);
+        oy = fma(S.ryx, vx, S.ryy * vy) - (double)(wy - GDT_FRAME);
+        const double au = fma(S.rxx, ax, S.rxy * ay), av = fma(S.ryx, ax, S.ryy * ay);
+        cl = gdt_left_clip(wrap, (float)au, (float)av, (float)ox, (float)oy, 1.f, 1.f, 1e-3f);
+    } else {
+        ox = gdt_cell_offset(vx, wx, S.bsx);
+        oy = gdt_cell_offset(vy, wy, S.bsy);
+        cl = gdt_left_clip(wrap, (float)ax, (float)ay, (float)ox, (float)oy, (float)S.bsx,
+                           (float)S.bsy, 1e-3f);
+    }
     unsigned nb;
     if (pre) {
         nb = npre;
@@ -741,7 +775,7 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
     // is within cov of v: 2R <= cov (successor), R <= cov (nearest neighbour).
     auto certify = [&]() {
         best();
-        const double cov = (double)hs * GDT_FMIN(S.bsx, S.bsy) + st.covb;
+        const double cov = (double)hs * GDT_FMIN(S.bsx, S.bsy) + st.covb;   // (bsx, bsy: cell heights)
         bool sure = true;       // (CERT: the circle is known to within its margins)
         ok = boxed = false;
         if (bk >= 0 && K.k0 > 1e-6 * (fabs(ax * by) + fabs(ay * bx))) {
@@ -763,8 +797,17 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
                 sure = K.k0 > 4. * eK0 && eq <= 1e-7 * cov &&
                        (wrap ? 4. : 1.) * R2 <= cmax * cmax * (1.0 - 2e-6);
             }
-            gdt_circle_cells<double>(qx - m, qx + m, qy - m, qy + m, rad, ox, oy, S.ibsx, S.ibsy,
-                                     1e-3, dx0, dx1, dy0, dy1);
+            if constexpr (GEN) {
+                const double u = ox + fma(S.rxx, qx, S.rxy * qy), ru = (rad + 2. * m) * S.nrx + 1e-3;
+                const double v = oy + fma(S.ryx, qx, S.ryy * qy), rv = (rad + 2. * m) * S.nry + 1e-3;
+                dx0 = gdt_cell_floor(u - ru);
+                dx1 = gdt_cell_floor(u + ru);
+                dy0 = gdt_cell_floor(v - rv);
+                dy1 = gdt_cell_floor(v + rv);
+            } else {
+                gdt_circle_cells<double>(qx - m, qx + m, qy - m, qy + m, rad, ox, oy, S.ibsx,
+                                         S.ibsy, 1e-3, dx0, dx1, dy0, dy1);
+            }
             ok = (dx0 >= -hs && dx1 <= hs && dy0 >= -hs && dy1 <= hs) ||
                  (cov > 0. && (wrap ? 4. : 1.) * R2 <= cov * cov * (1.0 - 1e-6));
             ok = ok && sure;
@@ -809,7 +852,7 @@ GDT_HD inline bool gdt_tile_x_range(const GdtSet& S, const GdtRingIO& io, int i)
     return fabs(p.x) <= 4. * S.lx && fabs(p.y) <= 4. * S.ly;
 }
 
-template <int W = 1, bool CERT = false>
+template <int W = 1, bool CERT = false, bool GEN = false>
 GDT_HD inline int gdt_tile_step_f64(const GdtSet& S, const GdtTileLds& L, const GdtRingIO& io,
                                     GdtTileLane<double>& st, unsigned& npred, int sub = 0)
 {
@@ -818,8 +861,8 @@ GDT_HD inline int gdt_tile_step_f64(const GdtSet& S, const GdtTileLds& L, const 
     if constexpr (CERT) {
         if (st.ak < 0 && !gdt_tile_x_range(S, io, L.orig[st.iv])) return STEP_DEFER;
     }
-    const int rc = gdt_tile_search_f64<W, CERT>(S, L, st, npred, sub, true, bk, bx, by, nullptr, 0,
-                                                GDT_SCAN0, &io);
+    const int rc = gdt_tile_search_f64<W, CERT, GEN>(S, L, st, npred, sub, true, bk, bx, by,
+                                                     nullptr, 0, GDT_SCAN0, &io);
     if (rc != STEP_RUN) return rc;
     return gdt_tile_advance<double>(L, io, st, st.ak >= 0, bk, bx, by);
 }

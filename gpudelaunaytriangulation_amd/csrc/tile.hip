@@ -29,6 +29,8 @@ namespace GDT_TS_NS {
 // point, each scanning its part of every row (a list leaves most lanes of a
 // block without a point otherwise, and a small grid leaves most of the chip
 // idle; the launcher takes W from the caller).
+// GEN: sets in general boxes (gdt_tile_search_f64), 527 us at 2^20 points where
+// the rectangles' kernel takes 496.
 // PREC = GDT_EXACT: the FP64 steps with every decision certified
 // (gdt_tile_search_f64, CERT), bound as they are by the lanes' chains of steps;
 // all its deferred points go to the next launch, where a wavefront per point
@@ -96,7 +98,7 @@ __device__ inline void ring_block_totals(int mx, int er, unsigned npred, unsigne
     }
 }
 
-template <int PREC, int W>
+template <int PREC, int W, bool GEN = false>
 __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_tile(const GdtSet* __restrict__ sets, const GdtChunk* __restrict__ tiles,
                      const int* __restrict__ list, const uint32_t* __restrict__ lscan,
                      const int* __restrict__ flags, const int* __restrict__ halt,
@@ -171,7 +173,7 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     auto item = [&](int q) { return flags ? tile_flagged_slot(tf, T0, q) : (list ? list[q] : q); };
     if (Q0 >= Q1) return;    // block-uniform: nothing to do in this tile
 
-    const bool fits = gdt_stage_window<PREC == 32>(S, w, io, L, s_wsum);
+    const bool fits = gdt_stage_window<PREC == 32, GEN>(S, w, io, L, s_wsum);
 
     if (!fits) {
         for (int q = Q0 + tid; q < Q1; q += nt) {
@@ -184,6 +186,7 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     // iteration; a lane whose point is finished takes the next one, so a
     // wave's iterations track the total number of steps, not the longest ring.
     static_assert(W == 1 || W == 2 || (W == 4 && PREC == 64), "1, 2 or (FP64) 4 lanes per point");
+    static_assert(!GEN || (PREC == 64 && W <= 2), "general boxes: FP64, one or two lanes");
     static_assert(PREC == 32 || PREC == 64 || PREC == GDT_EXACT, "a precision code");
     if (tid == 0) {
         s_next = Q0 + nt / W;
@@ -197,7 +200,11 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     int q = Q0 + tid / W;
     bool have = q < Q1;
     int j = have ? item(q) : 0;
-    if (have) gdt_tile_lane_init<Real>(w, L, j, io, S, st);
+    auto lane_init = [&]() {
+        if constexpr (GEN) gdt_tile_lane_init_gen(w, L, j, io, S, st);
+        else gdt_tile_lane_init<Real>(w, L, j, io, S, st);
+    };
+    if (have) lane_init();
     unsigned npred = 0, nfb = 0, nsum = 0;
     int mx = 0, er = 0;
     while (__ballot(have) != 0) {
@@ -206,7 +213,7 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
             if constexpr (PREC == 32)
                 rc = gdt_tile_step_f32<W>(S, L, io, st, npred, nfb, sub);
             else
-                rc = gdt_tile_step_f64<W, PREC == GDT_EXACT>(S, L, io, st, npred, sub);
+                rc = gdt_tile_step_f64<W, PREC == GDT_EXACT, GEN>(S, L, io, st, npred, sub);
             // (both lanes of a pair end each step in the same state; the first reports)
             if (rc != STEP_RUN && sub == 0) {
                 if (rc == STEP_DEFER) {
@@ -237,7 +244,7 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
                 have = q < Q1;
                 if (have) {
                     j = item(q);
-                    gdt_tile_lane_init<Real>(w, L, j, io, S, st);
+                    lane_init();
                 }
             }
         }
@@ -254,10 +261,10 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
         wv.lane = tid & 63;
         for (int t = tid >> 6; t < ndl; t += nt >> 6) {
             const int jd = s_dlist[t];
-            // (built without the tie rule and for rectangles only, which would
+            // (built without the tie rule and the other box shape, which would
             // cost this kernel's main loop registers: a point with an exact tie
             // goes to k_one_ring_deferred)
-            const GdtRingResult r = gdt_wave_ring<false, false>(S, jd, io, wv, wv.lane == 0);
+            const GdtRingResult r = gdt_wave_ring<false, GEN>(S, jd, io, wv, wv.lane == 0);
             npred += r.npred;
             if (r.err & ERR_TIE) {
                 if (wv.lane == 0) {
@@ -296,7 +303,7 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
 // (tile, y) share a tile's points: wave w of block y takes the points
 // T0 + y nw + w + m gridDim.y nw.  Deferred points go to `defer` (handled by
 // k_one_ring_deferred in the next launch).
-template <bool CERT>
+template <bool CERT, bool GEN = false>
 __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star(const GdtSet* __restrict__ sets,
                                                         const GdtChunk* __restrict__ tiles,
                                                         GdtRingIO io, int* __restrict__ counts,
@@ -323,7 +330,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
     const int qb = T0 + (int)blockIdx.y * nw;
     if (qb >= T1) return;    // block-uniform: no point for this block
 
-    const bool fits = gdt_stage_window<false>(S, w, io, L, s_wsum);
+    const bool fits = gdt_stage_window<false, GEN>(S, w, io, L, s_wsum);
     if (!fits) {
         if (lane == 0)
             for (int q = qb + (tid >> 6); q < T1; q += qstep) {
@@ -337,7 +344,8 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
     for (int q = qb + (tid >> 6); q < T1; q += qstep) {     // wave-uniform
         GdtTileLane<double> st;
         st.tbl = s_tbl + STAR_TBL * tid;
-        gdt_tile_lane_init<double>(w, L, q, io, S, st);
+        if constexpr (GEN) gdt_tile_lane_init_gen(w, L, q, io, S, st);
+        else gdt_tile_lane_init<double>(w, L, q, io, S, st);
         // the lanes' block, as one row table (every lane the same): the
         // (2 GDT_SCAN + 1)^2 cells when they hold at most 64 entries, else
         // the (2 GDT_SCAN0 + 1)^2 cells; and this lane's entry of it
@@ -365,7 +373,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
                 sl.ay = X.y - st.vy;
             }
             double bx, by;
-            rc = gdt_tile_search_f64<1, CERT>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
+            rc = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
                                               (unsigned)tot, ph, &io);
         }
         int res = STEP_RUN, count = 0;
@@ -374,7 +382,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
         } else if (tot > 64) {
             if (lane == 0) {
                 int r = STEP_RUN;
-                while (r == STEP_RUN) r = gdt_tile_step_f64<1, CERT>(S, L, io, st, npred);
+                while (r == STEP_RUN) r = gdt_tile_step_f64<1, CERT, GEN>(S, L, io, st, npred);
                 res = r;
                 count = st.count;
             }
@@ -386,7 +394,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
                 // not certified over the block: lane 0 runs the full search
                 if (lane == 0) {
                     double bx, by;
-                    nrc = gdt_tile_search_f64<1, CERT>(S, L, st, npred, 0, true, nn, bx, by,
+                    nrc = gdt_tile_search_f64<1, CERT, GEN>(S, L, st, npred, 0, true, nn, bx, by,
                                                        nullptr, 0, GDT_SCAN0, &io);
                 }
                 nrc = __shfl(nrc, 0, 64);
@@ -413,7 +421,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
                             sl.ax = X.x - st.vx;
                             sl.ay = X.y - st.vy;
                             double bx, by;
-                            r = gdt_tile_search_f64<1, CERT>(S, L, sl, npred, 0, true, b, bx, by,
+                            r = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, true, b, bx, by,
                                                              nullptr, 0, GDT_SCAN0, &io);
                         }
                         if (__shfl(r, 0, 64) != STEP_RUN) {
@@ -452,6 +460,7 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
 
 hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,
                                     const GdtChunk* tiles, int ntiles, int block, int lanes,
+                                    bool general,
                                     const int* list, const uint32_t* lscan,
                                     const int* flags, const int* halt,
                                     const GdtRingIO& io, int* counts, int* status,
@@ -464,7 +473,16 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     // (the FP32-filtered step shares a point between at most two lanes)
     const bool two = lanes == 2 || (lanes == 4 && precision == 32);
     if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) block = GDT_XTILE_BLOCK;
-    if (precision == GDT_EXACT && (lanes == 2 || lanes == 4))
+    if (general && precision != 64) return hipErrorInvalidValue;
+    if (general && lanes > 1)
+        hipLaunchKernelGGL((k_one_ring_tile<64, 2, true>), dim3(ntiles), dim3(block), tbl, s,
+                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
+                           defer);
+    else if (general)
+        hipLaunchKernelGGL((k_one_ring_tile<64, 1, true>), dim3(ntiles), dim3(block), tbl, s,
+                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
+                           defer);
+    else if (precision == GDT_EXACT && (lanes == 2 || lanes == 4))
         hipLaunchKernelGGL((k_one_ring_tile<GDT_EXACT, 2>), dim3(ntiles), dim3(block), tbl, s,
                            d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
                            defer);
@@ -496,7 +514,7 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
 
 hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,
                                     const GdtChunk* tiles,
-                                    int ntiles, int nsplit, int block,
+                                    int ntiles, int nsplit, int block, bool general,
                                     const GdtRingIO& io, int* counts, int* status,
                                     unsigned long long* counters, int* defer,
                                     hipEvent_t after_tile, hipStream_t s)
@@ -506,7 +524,11 @@ hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nse
         return hipErrorInvalidValue;
     const size_t tbl = (STAR_TBL * (size_t)block + 1) * sizeof(uint32_t);
     if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) return hipErrorInvalidValue;
-    if (precision == GDT_EXACT)
+    if (general && precision != 64) return hipErrorInvalidValue;
+    if (general)
+        hipLaunchKernelGGL((k_one_ring_star<false, true>), dim3(ntiles, nsplit), dim3(block), tbl,
+                           s, d_sets, tiles, io, counts, status, counters, defer);
+    else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_star<true>, dim3(ntiles, nsplit), dim3(block), tbl, s, d_sets,
                            tiles, io, counts, status, counters, defer);
     else

@@ -325,10 +325,11 @@ int gdt_host_voronoi_vertices(const double* xy, int n, double lx, double ly, con
  * images round unit-cell coordinates (periodicBoundaries::minDist,
  * periodicBoundaries.h:165-178).  Points may lie anywhere (they are wrapped);
  * the Brownian loop wraps moved points into the caller's own box
- * (putInBoxReal, periodicBoundaries.h:131-152).  General boxes run the
- * row-major cell order and FP64 predicates whatever the configuration and
- * precision arguments (the rings are the same); gdt_celllist_info then
- * reports the cell heights as bsx, bsy.  A matrix with x12 = x21 = 0 and a
+ * (putInBoxReal, periodicBoundaries.h:131-152).  General boxes run FP64
+ * predicates whatever the precision argument (the rings are the same); in
+ * grids too small for the LDS tile kernels also the row-major cell order
+ * whatever the configuration.  gdt_celllist_info then reports the cell heights
+ * as bsx, bsy.  A matrix with x12 = x21 = 0 and a
  * positive diagonal runs the rectangular path.  Batched forms take four
  * doubles per set in `boxes`; otherwise as the rectangular calls. */
 int gdt_celllist_build_general(gdt_context* ctx, const double* d_xy, int n, const double* box,

@@ -1,7 +1,12 @@
-// The exact mode's tile routine (gdt_tile.h with GDT_EXACT: FP64 and
-// double-double decisions inside their error bounds, everything else handed to
-// the wavefront's exact routine, 64 emulated lanes) against the per-point exact
-// routine, for every point of a set; and that wavefront routine itself.  Usage: exact_tile <points.bin> <n> <lx> <ly> <cell size>
+// The tile routines (gdt_tile.h) against the per-point routines, for every
+// point of a set; points a tile routine hands on go to the wavefront routine (64
+// emulated lanes), as on the device.
+// Usage: tile_rows <points.bin> <n> <lx> <ly> <cell size>
+//   the exact mode (GDT_EXACT: FP64 and double-double decisions inside their
+//   error bounds) against gdt_one_ring_exact, and every seventh point's row
+//   again by the wavefront routine;
+// or     tile_rows <points.bin> <n> <x11> <x22> <cell size> <x12> <x21>
+//   FP64 in a general box (lattice vectors as columns) against gdt_one_ring_f64.
 // Prints: points, points handed on, rows that differ, error flags.
 #include "gdt_tile.h"
 #include "gdt_exact_wave.h"
@@ -10,16 +15,36 @@
 #include <cstdlib>
 #include <vector>
 
+// The FP64 tile steps of a point in a general box.
+static GdtRingResult general_ring(const GdtSet& S, const GdtTileWin& w, const GdtTileLds& L, int j,
+                                  const GdtRingIO& io)
+{
+    GdtRingResult res = {0, 0, 0u, 0u};
+    uint32_t tbl[6];
+    GdtTileLane<double> st;
+    gdt_tile_lane_init_gen(w, L, j, io, S, st);
+    st.tbl = tbl;
+    int rc = STEP_RUN;
+    while (rc == STEP_RUN) rc = gdt_tile_step_f64<1, false, true>(S, L, io, st, res.npred);
+    res.count = st.count;
+    if (rc == STEP_DEFER) res.err = ERR_DEFER;
+    if (rc == STEP_NOCLOSE) res.err = ERR_NOCLOSE;
+    return res;
+}
+
 int main(int argc, char** argv)
 {
-    if (argc != 6) return 2;
+    if (argc != 6 && argc != 8) return 2;
+    const bool general = argc == 8;
     const int n = std::atoi(argv[2]), stride = 32;
     const double lx = std::atof(argv[3]), ly = std::atof(argv[4]), cell = std::atof(argv[5]);
     std::vector<gdt_d2> xy((size_t)n);
     FILE* f = std::fopen(argv[1], "rb");
     if (!f || std::fread(xy.data(), sizeof(gdt_d2), (size_t)n, f) != (size_t)n) return 3;
     std::fclose(f);
-    const GdtSet S = gdt_make_set(0, n, 0, lx, ly, cell, 1);
+    const double box[4] = {lx, general ? std::atof(argv[6]) : 0., general ? std::atof(argv[7]) : 0.,
+                           ly};
+    const GdtSet S = gdt_make_set_box(0, n, 0, box, cell, 1);
     std::vector<uint32_t> cstart((size_t)S.nkeys + 1, 0u), scell((size_t)n);
     std::vector<int> key((size_t)n), perm((size_t)n);
     std::vector<gdt_d2> off((size_t)n);
@@ -61,20 +86,24 @@ int main(int argc, char** argv)
         cs[GDT_WIN_CELLS] = run;
         const bool fits = run <= GDT_WIN_MAXPTS && S.rmax >= GDT_SCAN;
         for (int c = 0; c < GDT_WIN_CELLS && fits; ++c)
-            gdt_tile_copy<false>(S, c, gs[c], cs[c], cnt[c], io, L);
+            for (uint32_t k = 0; k < cnt[c]; ++k) {
+                const int fx = c % GDT_WIN - GDT_FRAME, fy = c / GDT_WIN - GDT_FRAME;
+                L.X64[cs[c] + k] = gdt_frame64_gen(S, fx, fy, io.off64[gs[c] + (int)k]);
+                L.orig[cs[c] + k] = io.perm[gs[c] + (int)k];
+            }
         const int k0 = t * GDT_TILE_CELLS;
         for (int j = (int)cstart[k0]; j < (int)cstart[k0 + GDT_TILE_CELLS]; ++j) {
             io.nbrs = rows[1].data();
-            const GdtRingResult want = gdt_one_ring_exact(S, j, io);
+            const GdtRingResult want =
+                general ? gdt_one_ring_f64(S, j, io) : gdt_one_ring_exact(S, j, io);
             io.nbrs = rows[0].data();
             GdtRingResult got = {0, ERR_DEFER, 0u, 0u};
-            if (fits) got = gdt_tile_ring<GDT_EXACT>(S, w, L, j, io);
-            if (got.err & ERR_DEFER) {
-                ++handed;
-                got = gdt_wave_ring_exact(S, j, io, wave, true);
-            } else if (j % 7 == 0) {    // (the tile's row again, by a wavefront)
-                got = gdt_wave_ring_exact(S, j, io, wave, true);
-            }
+            if (fits && general) got = general_ring(S, w, L, j, io);
+            else if (fits) got = gdt_tile_ring<GDT_EXACT>(S, w, L, j, io);
+            const bool on = (got.err & ERR_DEFER) != 0;
+            handed += on;
+            if (on && general) got = gdt_wave_ring(S, j, io, wave, true);
+            else if (on || (!general && j % 7 == 0)) got = gdt_wave_ring_exact(S, j, io, wave, true);
             err |= got.err;
             bool same = got.count == want.count && got.err == want.err;
             for (int m = 0; same && m < want.count && m < stride; ++m)

@@ -1,5 +1,5 @@
 """The exact mode's tile and wavefront routines against its per-point routine, row by row, in
-a host build under AddressSanitizer and UBSan (tests/cpu_emul/exact_tile.cpp):
+a host build under AddressSanitizer and UBSan (tests/cpu_emul/tile_rows.cpp):
 random points, lattices off by rounding errors (the double-double decisions),
 exact lattices (ties, handed on), coarse and fine cells, a cluster that no
 window holds, coincident points, a grid too small for windows and coordinates
@@ -24,14 +24,15 @@ def exe(request, tmp_path_factory):
     subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-fsanitize=address,undefined",
                     "-fno-sanitize-recover=all", "-ffp-contract=off", f"-DGDT_TILE_SHIFT={ts}",
                     f"-DGDT_WIN_MAXPTS={pts}", f"-I{CSRC}",
-                    os.path.join(ROOT, "tests", "cpu_emul", "exact_tile.cpp"), "-o", out], check=True)
+                    os.path.join(ROOT, "tests", "cpu_emul", "tile_rows.cpp"), "-o", out], check=True)
     return out
 
 
-def run(exe, tmp_path, xy, lx, ly, cell):
+def run(exe, tmp_path, xy, lx, ly, cell, *off_diagonal):
     f = str(tmp_path / "p.bin")
     np.ascontiguousarray(xy, dtype=np.float64).tofile(f)
-    out = subprocess.run([exe, f, str(len(xy)), repr(lx), repr(ly), repr(cell)],
+    out = subprocess.run([exe, f, str(len(xy)), repr(lx), repr(ly), repr(cell),
+                          *map(repr, off_diagonal)],
                          capture_output=True, text=True, check=True).stdout.split()
     return [int(v) for v in out]
 
