@@ -27,6 +27,9 @@ SOURCES = ["celllist.hip", "onering.hip", "testrepair.hip", "voronoi.hip", "mdst
 # The LDS-window kernels, once per tile edge: (source, object, defines).
 TILE_SOURCES = [(src, f"{src[:-4]}_ts{ts}", [f"-DGDT_TILE_SHIFT={ts}", f"-DGDT_WIN_MAXPTS={pts}"])
                 for src in ("tile.hip", "ringtest.hip") for ts, pts in ((4, 1024), (5, 2048))]
+# ... and the ring kernels again for windows of twice the points
+TILE_SOURCES.append(("tile.hip", "tile_ts5d",
+                     ["-DGDT_TILE_SHIFT=5", "-DGDT_WIN_MAXPTS=4096", "-DGDT_WIN_DENSE"]))
 # CPU mode: the same per-point routines compiled for the host (g++, OpenMP)
 HOST_SOURCES = ["hostpath.cpp"]
 

@@ -203,6 +203,18 @@ static int ring_chunks(gdt_context* c)
     return GDT_OK;
 }
 
+// Points to a tile window of edge 2^ts + 8 cells, on average.
+static double window_points(const std::vector<GdtSet>& sets, int ts)
+{
+    double n = 0., cells = 0.;
+    for (const auto& s : sets) {
+        n += s.n;
+        cells += (double)s.xsize * s.ysize;
+    }
+    const double edge = (1 << ts) + 8;
+    return cells > 0. ? n / cells * edge * edge : 0.;
+}
+
 // The tile edge of the configuration, or the automatic one: 16x16-cell tiles
 // when the 32x32 tiling of the sets would not give every compute unit a
 // second tile (small inputs: four times the blocks, each a quarter of the
@@ -213,6 +225,20 @@ static int tile_shift_for(const gdt_context* c, const std::vector<GdtSet>& sets)
     long long tiles = 0;
     for (const auto& s : sets) tiles += (long long)(s.nkeys >> (2 * s.tshift));
     return tiles <= c->num_cu ? 4 : 5;
+}
+
+// Whether the sets' tiles take the larger windows (32x32-cell tiles).
+static bool dense_windows(const gdt_context* c)
+{
+    return c->sets[0].tshift == 5 && window_points(c->sets, 5) > GDT_DENSE_WINDOW;
+}
+
+// Whether even these will mostly overflow, so that nearly every point is handed
+// on (gdt_launch_deferred): their number, else 0.
+static int many_deferred(const gdt_context* c)
+{
+    const int ts = c->sets[0].tshift;
+    return window_points(c->sets, ts) > (ts == 4 ? 1000. : 4000.) ? c->total_n : 0;
 }
 
 // Lanes per point of the global triangulation: the configuration's; else a
@@ -289,8 +315,8 @@ static_assert((int)GDT_PREC_EXACT == (int)GDT_EXACT, "one code for the exact mod
 // 581 us per call, 2,841 with the row-major per-point kernel).
 // Sets of which one is a general box keep the row-major order where the tile
 // kernels could not take them: a grid smaller than the windows' scan block
-// (every point of such a tile is handed on), or tiles whose padding outgrows
-// the cell keys.
+// (every point of such a tile is handed on), tiles whose padding outgrows
+// the cell keys, or cells so full that every window overflows.
 static std::vector<GdtSet> sets_of(const gdt_context* c, int nsets, const int* offsets,
                                    const double* boxes, double cell_size, int words)
 {
@@ -313,7 +339,7 @@ static std::vector<GdtSet> sets_of(const gdt_context* c, int nsets, const int* o
             keys += s.nkeys;
             ok = ok && s.rmax >= GDT_MIN_TILE_RMAX;
         }
-        if (!ok || keys > GDT_MAX_KEYS) {
+        if (!ok || keys > GDT_MAX_KEYS || window_points(sets, 5) > 4000.) {
             make(0, GDT_TSHIFT_MAX);
             return sets;
         }
@@ -642,17 +668,19 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
             GDT_CHECK(gdt_tiles::one_ring_star(ts, precision, c->d_sets.p, (int)c->sets.size(), c->tch.p,
                                                c->ntch, nsplit, block, general,
                                                ring_io(c, d_nbrs, stride), d_counts, c->status.p,
-                                               c->counters.p, c->defer.p,
+                                               c->counters.p, c->defer.p, many_deferred(c),
                                                c->cfg.profile ? c->ev[2] : nullptr, s));
         } else {
-            c->stats.lanes = lanes == 4 && (general || precision != GDT_PREC_FP64) ? 2 : lanes;
+            const bool dense = dense_windows(c);
+            c->stats.lanes = dense ? 1 : lanes == 4 && (general || precision != GDT_PREC_FP64) ? 2 : lanes;
             const int one_each = std::min(1024, (1 << (2 * ts)) * lanes);
             const int block =
                 c->ntch <= c->num_cu ? std::max(tile_block(c), one_each) : tile_block(c);
             GDT_CHECK(gdt_tiles::one_ring(ts, precision, c->d_sets.p, (int)c->sets.size(),
                                           c->tch.p, c->ntch, block, lanes, general, nullptr,
-                                          nullptr, nullptr, nullptr, ring_io(c, d_nbrs, stride),
+                                          nullptr, ring_io(c, d_nbrs, stride),
                                           d_counts, c->status.p, c->counters.p, c->defer.p,
+                                          dense, many_deferred(c),
                                           c->cfg.profile ? c->ev[2] : nullptr, s));
         }
     } else {
@@ -662,12 +690,12 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
         // (the exact mode hands no point on: one beyond the search radius is an error)
         const bool exact = precision == GDT_PREC_EXACT;
         GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), c->rch.p, c->nrch,
-                                      c->cfg.block, nullptr, nullptr, 0, io, d_counts,
+                                      c->cfg.block, nullptr, nullptr, 0, 0, io, d_counts,
                                       c->status.p, c->counters.p, exact ? nullptr : c->defer.p, s));
         if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[2], s));
         if (!exact)
             GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
-                                          c->status.p, c->counters.p, c->defer.p, s));
+                                          c->status.p, c->counters.p, c->defer.p, 0, s));
     }
     if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
     rc = finish_rings(c, stride, required, s);
@@ -840,9 +868,10 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
         GDT_CHECK(gdt_tiles::one_ring(c->sets[0].tshift, precision, c->d_sets.p,
                                       (int)c->sets.size(), c->tch.p, c->ntch, tile_block(c),
                                       c->cfg.repair_lanes ? c->cfg.repair_lanes : 2,
-                                      any_general(c), nullptr, nullptr, d_repair, c->halt,
+                                      any_general(c), d_repair, c->halt,
                                       ring_io(c, d_nbrs, stride), d_counts, c->status.p,
-                                      c->counters.p, c->defer.p, nullptr, s));
+                                      c->counters.p, c->defer.p, dense_windows(c), many_deferred(c),
+                                      nullptr, s));
         return GDT_OK;
     }
     const size_t n = (size_t)c->total_n;
@@ -854,12 +883,12 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
                                  c->worklist.p, worklen, c->scan_tmp.p, c->halt, s));
     const GdtRingIO io = ring_io(c, d_nbrs, stride);
     GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), nullptr, 0,
-                                  c->cfg.block, c->worklist.p, worklen, c->total_n, io,
+                                  c->cfg.block, c->worklist.p, worklen, 0, c->total_n, io,
                                   d_counts, c->status.p, c->counters.p,
                                   exact ? nullptr : c->defer.p, s));
     if (!exact)
         GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
-                                      c->status.p, c->counters.p, c->defer.p, s));
+                                      c->status.p, c->counters.p, c->defer.p, 0, s));
     return GDT_OK;
 }
 

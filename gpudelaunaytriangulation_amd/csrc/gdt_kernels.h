@@ -74,7 +74,7 @@ hipError_t gdt_max_occupancy(const uint32_t* ccount, int total_keys, int* d_out,
 // in status[ST_NDEFER], zero on entry) for gdt_launch_deferred.
 hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                const GdtChunk* chunks, int nch, int block, const int* worklist,
-                               const uint32_t* worklen, int max_work,
+                               const uint32_t* worklen, int first, int max_work,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s);
 
@@ -85,18 +85,32 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
 // Threads per block (at most) of the exact mode's tile and star kernels: two
 // waves per SIMD, so that the double-double decisions keep 256 registers.
 #define GDT_XTILE_BLOCK 512
+// Points to a 40x40-cell window, on average, from which the ring kernels take
+// the windows of 4,096 points.  Those of 2,048 hand on the tiles that overflow
+// them: 1 tile in 180 at an average of 1,936, where the smaller windows take
+// 411 us for 600,000 points and the larger 425, and nearly all at 2,304
+// (1,926 us against 463).
+#define GDT_DENSE_WINDOW 1945.
 // Deferred points a tile block finishes itself (the rest go to the list).
 #define GDT_TILE_DEFER 64
 
 // Deferred points of the tile kernel (defer[0..status[ST_NDEFER]), count read
 // on the device): a wavefront each, then one lane each beyond GDT_WAVE_CAP.
+// many: 0, or, where more than that is expected, the most that can be.
 hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
-                               unsigned long long* counters, int* defer, hipStream_t s);
+                               unsigned long long* counters, int* defer, int many,
+                               hipStream_t s);
 
 // The LDS-window kernels, compiled once per tile edge into namespaces ts4
 // (16x16-cell tiles) and ts5 (32x32); gdt_tiles::* picks by the sets' shift.
+// ts5d: the ring kernels of 32x32-cell tiles with windows of 4,096 points, one
+// block to a compute unit, for cells too full for the usual 2,048.
+#ifdef GDT_WIN_DENSE
+#define GDT_TS_NS ts5d
+#else
 #define GDT_TS_NS GDT_TS_NS_(GDT_TILE_SHIFT)
+#endif
 #define GDT_TS_NS_(x) GDT_TS_NS__(x)
 #define GDT_TS_NS__(x) ts##x
 #define GDT_DECLARE_TILE_LAUNCHERS(ns)                                                            \
@@ -104,16 +118,15 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
     hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles, int ntiles, int block, int lanes, \
                                         bool general,                                            \
-                                        const int* list, const uint32_t* lscan,                  \
                                         const int* flags, const int* halt,                       \
                                         const GdtRingIO& io, int* counts, int* status,           \
-                                        unsigned long long* counters, int* defer,                \
+                                        unsigned long long* counters, int* defer, int many,      \
                                         hipEvent_t after_tile, hipStream_t s);                   \
     hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles,                                   \
                                         int ntiles, int nsplit, int block, bool general,         \
                                         const GdtRingIO& io, int* counts, int* status,           \
-                                        unsigned long long* counters, int* defer,                \
+                                        unsigned long long* counters, int* defer, int many,      \
                                         hipEvent_t after_tile, hipStream_t s);                   \
     hipError_t gdt_launch_ring_test_tile(const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,\
                                          const int* nbrs, const int* counts, int stride,         \
@@ -140,8 +153,7 @@ hipError_t gdt_launch_test(const GdtSet* d_sets, int nsets, const int* tris, con
                            hipStream_t s);
 
 
-// One-ring of every point (list and flags null), of the slots of a
-// slot-ordered list (lscan its exclusive scan over slots), or of the points
+// One-ring of every point (flags null), or of the points
 // flagged in a caller-order array (flags[i] >= 0; each tile finds its own
 // flagged slots, status[ST_NFLAGGED] += their count, which must start at zero;
 // nothing with *halt set), one block per tile of the tiled cell order,
@@ -162,29 +174,33 @@ hipError_t gdt_launch_test(const GdtSet* d_sets, int nsets, const int* tris, con
 // number of owned triangles; partials holds 2 * ntiles words.
 GDT_DECLARE_TILE_LAUNCHERS(ts4)
 GDT_DECLARE_TILE_LAUNCHERS(ts5)
+GDT_DECLARE_TILE_LAUNCHERS(ts5d)     // (gdt_launch_one_ring_tile alone is defined)
 static_assert(GDT_TSHIFT_MIN == 4 && GDT_TSHIFT_MAX == 5, "a launcher per supported tile edge");
 
 namespace gdt_tiles {
 inline hipError_t one_ring(int tshift, int precision, const GdtSet* d_sets, int nsets,
                            const GdtChunk* tiles, int ntiles, int block, int lanes, bool general,
-                           const int* list, const uint32_t* lscan, const int* flags,
-                           const int* halt, const GdtRingIO& io, int* counts, int* status,
-                           unsigned long long* counters, int* defer, hipEvent_t after_tile,
-                           hipStream_t s)
+                           const int* flags, const int* halt, const GdtRingIO& io, int* counts, int* status,
+                           unsigned long long* counters, int* defer, bool dense, int many,
+                           hipEvent_t after_tile, hipStream_t s)
 {
-    return (tshift == 4 ? ts4::gdt_launch_one_ring_tile : ts5::gdt_launch_one_ring_tile)(
-        precision, d_sets, nsets, tiles, ntiles, block, lanes, general, list, lscan, flags, halt,
-        io, counts, status, counters, defer, after_tile, s);
+    // (rows do not depend on the windows; 32x32-cell tiles have fuller ones)
+    return (tshift == 4 ? ts4::gdt_launch_one_ring_tile
+            : dense     ? ts5d::gdt_launch_one_ring_tile
+                        : ts5::gdt_launch_one_ring_tile)(
+        precision, d_sets, nsets, tiles, ntiles, block, lanes, general, flags, halt,
+        io, counts, status, counters, defer, many, after_tile, s);
 }
 inline hipError_t one_ring_star(int tshift, int precision, const GdtSet* d_sets, int nsets,
                                 const GdtChunk* tiles, int ntiles, int nsplit, int block,
                                 bool general, const GdtRingIO& io, int* counts, int* status,
-                                unsigned long long* counters, int* defer, hipEvent_t after_tile,
+                                unsigned long long* counters, int* defer, int many,
+                                hipEvent_t after_tile,
                                 hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_star : ts5::gdt_launch_one_ring_star)(
         precision, d_sets, nsets, tiles, ntiles, nsplit, block, general, io, counts, status, counters, defer,
-        after_tile, s);
+        many, after_tile, s);
 }
 inline hipError_t ring_test(int tshift, const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,
                             const int* nbrs, const int* counts, int stride, int total_n,

@@ -202,8 +202,9 @@ GDT_HD inline GdtRingResult gdt_wave_ring(const GdtSet& S, int j, const GdtRingI
         // bounding box of the current circle in one pass -- every later best's
         // circle lies inside it (circles through v and a with centres left of
         // v->a are nested along the bisector), so the search is then certified
-        // -- or, while there is no candidate or the box reaches past rmax, the
-        // next Chebyshev ring.
+        // -- or, while there is no candidate or the box reaches far beyond the
+        // square or past rmax, the next Chebyshev rings (one without a
+        // candidate, else two).
         int hs = S.rmax < 2 ? S.rmax : 2;
         pass(-hs, hs, -hs, hs, -1);
         for (;;) {
@@ -242,15 +243,20 @@ GDT_HD inline GdtRingResult gdt_wave_ring(const GdtSet& S, int j, const GdtRingI
                 }
                 if (boxed) {
                     if (dx0 >= -hs && dx1 <= hs && dy0 >= -hs && dy1 <= hs) return true;
-                    if (dx0 >= -S.rmax && dx1 <= S.rmax && dy0 >= -S.rmax && dy1 <= S.rmax) {
+                    // (a box far beyond the scanned square belongs to a best
+                    // that a nearer candidate will replace: the square grows
+                    // first)
+                    const int lim = gdt_imin(S.rmax, hs + 4);
+                    if (dx0 >= -lim && dx1 <= lim && dy0 >= -lim && dy1 <= lim) {
                         pass(dx0, dx1, dy0, dy1, hs);
                         return true;
                     }
                 }
             }
             if (hs >= S.rmax) return false;
-            ++hs;
-            pass(-hs, hs, -hs, hs, hs - 1);
+            const int to = gdt_imin(S.rmax, g.k >= 0 ? hs + 2 : hs + 1);
+            pass(-to, to, -to, to, hs);
+            hs = to;
         }
     };
 

@@ -160,9 +160,13 @@ extern "C" int gdt_triangulate_noalloc(const double* d_xy, int n, double lx, dou
     io.xy = nullptr;
     // the block size of gdt_triangulate's default configuration
     const int block = ntiles <= cus ? 1024 : 512;
+    // (fuller windows; those that overflow all the same hand nearly every point on)
+    const double window = 1600. * n / ((double)S.xsize * S.ysize);
+    const bool dense = window > GDT_DENSE_WINDOW;
+    const int many = window > 4000. ? n : 0;
     if (gdt_tiles::one_ring(GDT_TILE_SHIFT, precision, d_sets, 1, d_tiles, ntiles, block, 1, false,
-                            nullptr, nullptr, nullptr, nullptr, io, d_counts, status, counters,
-                            reinterpret_cast<int*>(base + L.defer), nullptr, s) != hipSuccess)
+                            nullptr, nullptr, io, d_counts, status, counters,
+                            reinterpret_cast<int*>(base + L.defer), dense, many, nullptr, s) != hipSuccess)
         return GDT_ERR_DEVICE;
     int h_status[ST_WORDS];
     if (hipMemcpyAsync(h_status, status, sizeof(h_status), hipMemcpyDeviceToHost, s) != hipSuccess ||

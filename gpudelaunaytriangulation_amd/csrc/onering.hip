@@ -95,7 +95,7 @@ __device__ inline void one_ring_lanes(const GdtSet* __restrict__ sets, int nsets
     }
 }
 
-// Worklist of slots (count in device memory), one lane each.
+// Entries from `first` of a worklist of slots (count in device memory), one lane each.
 template <int PREC>
 __global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict__ sets, int nsets,
                                                         const int* __restrict__ worklist,
@@ -103,9 +103,9 @@ __global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict
                                                         GdtRingIO io, int* __restrict__ counts,
                                                         int* __restrict__ status,
                                                         unsigned long long* __restrict__ counters,
-                                                        int* __restrict__ defer)
+                                                        int* __restrict__ defer, int first)
 {
-    one_ring_lanes<PREC>(sets, nsets, worklist, 0, (int)*worklen, io, counts, status, counters,
+    one_ring_lanes<PREC>(sets, nsets, worklist, first, (int)*worklen, io, counts, status, counters,
                          defer);
 }
 
@@ -114,6 +114,9 @@ __global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict
 // decisions in the exact mode), any beyond (dense clusters, exact lattices)
 // one lane each.  One launch for both: the second part is nearly always
 // empty, and as a kernel of its own cost its launch, 4.7 us of every call.
+// Where the caller expects a long list (waves_only), the second part is
+// k_one_ring_list: with the wavefront routine's registers beside it, it took
+// 2.9 ms for 600,000 points of 1.44 to a cell, where that takes 1.9.
 template <int PREC>
 __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restrict__ sets,
                                                            int nsets,
@@ -122,7 +125,8 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
                                                            int cap, GdtRingIO io,
                                                            int* __restrict__ counts,
                                                            int* __restrict__ status,
-                                                           unsigned long long* __restrict__ counters)
+                                                           unsigned long long* __restrict__ counters,
+                                                           int waves_only)
 {
     const int lane = (int)(threadIdx.x & 63);
     const int wid = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
@@ -160,32 +164,38 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
             if (nsum) atomicAdd(&counters[CT_NBRSUM], (unsigned long long)nsum);
         }
     }
-    if (all > cap)
+    if (all > cap && !waves_only)
         one_ring_lanes<PREC>(sets, nsets, worklist, cap, all, io, counts, status, counters,
                              nullptr);
 }
 
 hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
-                               unsigned long long* counters, int* defer, hipStream_t s)
+                               unsigned long long* counters, int* defer, int many, hipStream_t s)
 {
     // (the count is read on the device)
     const uint32_t* ndefer = reinterpret_cast<const uint32_t*>(status + ST_NDEFER);
     if (precision == 32)
         hipLaunchKernelGGL(k_one_ring_deferred<32>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
-                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
+                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
+                           many);
     else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_deferred<GDT_EXACT>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s,
-                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
+                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
+                           many);
     else
         hipLaunchKernelGGL(k_one_ring_deferred<64>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
-                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters);
-    return hipGetLastError();
+                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
+                           many);
+    const hipError_t e = hipGetLastError();
+    if (e != hipSuccess || !many) return e;
+    return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer, ndefer,
+                               GDT_WAVE_CAP, many, io, counts, status, counters, nullptr, s);
 }
 
 hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                const GdtChunk* chunks, int nch, int block, const int* worklist,
-                               const uint32_t* worklen, int max_work,
+                               const uint32_t* worklen, int first, int max_work,
                                const GdtRingIO& io, int* counts, int* status,
                                unsigned long long* counters, int* defer, hipStream_t s)
 {
@@ -202,17 +212,18 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                counts, status, counters, defer);
         return hipGetLastError();
     }
+    max_work -= first;
     if (max_work <= 0) return hipSuccess;
     int grid = (max_work + block - 1) / block;
     if (grid > 4096) grid = 4096;
     if (precision == 32)
         hipLaunchKernelGGL(k_one_ring_list<32>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, io, counts, status, counters, defer);
+                           worklist, worklen, io, counts, status, counters, defer, first);
     else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_list<GDT_EXACT>, dim3(grid), dim3(block), 0, s, d_sets,
-                           nsets, worklist, worklen, io, counts, status, counters, defer);
+                           nsets, worklist, worklen, io, counts, status, counters, defer, first);
     else
         hipLaunchKernelGGL(k_one_ring_list<64>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, io, counts, status, counters, defer);
+                           worklist, worklen, io, counts, status, counters, defer, first);
     return hipGetLastError();
 }

@@ -7,6 +7,7 @@
 // Replaces gpu_voronoi_calc_global_kernel + gpu_get_neighbors_global_kernel
 // (DelaunayGPU.cu:649-675, 981-1006) and their masked repair variants
 // (DelaunayGPU.cu:611-640, 945-975).
+#include "gdt_hull.h"
 #include "gdt_kernels.h"
 #include "gdt_stage.h"
 #include "gdt_wavedev.h"
@@ -15,22 +16,20 @@
 
 namespace GDT_TS_NS {
 
-// One block per tile (GDT_TILE x GDT_TILE cells, this file's compiled tile edge): stage the tile window in LDS, then the lanes
-// advance the tile's points one search step at a time.  With `list` and
-// `flags` null the tile's points are all its slots [T0, T1); with `list` they
-// are the slots list[lscan[T0] .. lscan[T1]) (a slot-ordered list of the
-// points to redo, with lscan its exclusive scan over slots); with `flags` (a
-// caller-order array, flagged >= 0) they are the tile's flagged slots, which
-// the block gathers first into a bit mask in LDS (status[ST_NFLAGGED] += their
-// count).  A tile with none exits before staging.  The points of a window that does not fit the LDS budget, or of a
-// grid too small for the scan block, and points with a step whose circle
+// k_one_ring_tile: one block per tile (GDT_TILE x GDT_TILE cells, this file's
+// compiled tile edge): stage the tile window in LDS, then the lanes advance the
+// tile's points one search step at a time.  With `flags` null the tile's points
+// are all its slots [T0, T1); with `flags` (a caller-order array, flagged >= 0)
+// they are the tile's flagged slots, which the block gathers first into a bit
+// mask in LDS (status[ST_NFLAGGED] += their count).  A tile with none exits
+// before staging.  The points of a window that does not fit the LDS budget, or
+// of a grid too small for the scan block, and points with a step whose circle
 // leaves the window, are appended to `defer` and handled by k_one_ring_deferred
 // in the next launch.  With W = 2 or 4 (FP64) neighbouring lanes share each
-// point, each scanning its part of every row (a list leaves most lanes of a
+// point, each scanning its part of every row (flags leave most lanes of a
 // block without a point otherwise, and a small grid leaves most of the chip
-// idle; the launcher takes W from the caller).
-// GEN: sets in general boxes (gdt_tile_search_f64), 527 us at 2^20 points where
-// the rectangles' kernel takes 496.
+// idle; the launcher takes W from the caller).  FP64 with one lane per point is
+// k_one_ring_hull's.  GEN: sets in general boxes (gdt_tile_search_f64).
 // PREC = GDT_EXACT: the FP64 steps with every decision certified
 // (gdt_tile_search_f64, CERT), bound as they are by the lanes' chains of steps;
 // all its deferred points go to the next launch, where a wavefront per point
@@ -57,6 +56,79 @@ __device__ inline int tile_flagged_slot(const TileFlags& f, int T0, int q)
     unsigned long long m = f.mask[lo];
     for (int r = q - (int)f.pre[lo]; r > 0; --r) m &= m - 1ull;
     return T0 + 64 * lo + __ffsll((long long)m) - 1;
+}
+
+// Prefix counts pre[0..nw] of a mask's words (nw <= 64), by the first wave;
+// returns the total (every thread calls it; ends with a barrier).
+__device__ inline int tile_mask_prefix(const TileFlags& f, uint32_t* pre)
+{
+    const int tid = threadIdx.x;
+    if (tid < 64) {
+        uint32_t x = tid < f.nw ? (uint32_t)__popcll(f.mask[tid]) : 0u;
+#pragma unroll
+        for (int d = 1; d < 64; d <<= 1) {
+            const uint32_t y = __shfl_up(x, d, 64);
+            if (tid >= d) x += y;
+        }
+        if (tid < f.nw) pre[tid + 1] = x;
+        if (tid == 0) pre[0] = 0u;
+    }
+    __syncthreads();
+    return (int)pre[f.nw];
+}
+
+// Gathers the tile's flagged slots (flags[caller index] >= 0) into a bit mask and
+// its prefix counts; returns their number (block-uniform, ends with a barrier).
+__device__ inline int tile_gather_flags(const int* __restrict__ flags, const int* __restrict__ perm,
+                                        int T0, int npt, unsigned long long* mask, uint32_t* pre,
+                                        TileFlags& tf)
+{
+    const int tid = threadIdx.x, nt = blockDim.x;
+    tf.mask = mask;
+    tf.pre = pre;
+    tf.nw = (npt + 63) >> 6;
+    for (int t0 = 0; t0 < 64 * tf.nw; t0 += nt) {
+        const int t = t0 + tid;
+        const bool f = t < npt && flags[perm[T0 + t]] >= 0;
+        const unsigned long long b = __ballot(f);
+        if ((tid & 63) == 0 && (t >> 6) < tf.nw) mask[t >> 6] = b;
+    }
+    __syncthreads();
+    return tile_mask_prefix(tf, pre);
+}
+
+// The points a tile block deferred (their circle left the window): one
+// wavefront each, read from global memory (gdt_wave_ring), by this block's waves while
+// other blocks still run their tiles.  Built without the tie rule and the
+// other box shape, which would cost the kernels' main loops registers: a point
+// with an exact tie goes to k_one_ring_deferred.
+template <bool GEN>
+__device__ inline void tile_finish_deferred(const GdtSet& S, const GdtRingIO& io, const int* dlist,
+                                            int ndl, int* __restrict__ counts,
+                                            int* __restrict__ status, int* __restrict__ defer,
+                                            unsigned& npred, unsigned& nsum, int& mx, int& er)
+{
+    if (ndl <= 0) return;
+    const int tid = threadIdx.x, nt = blockDim.x;
+    if (tid == 0) atomicAdd(&status[ST_NDEFER_TILE], ndl);
+    GdtWaveDev wv;
+    wv.lane = tid & 63;
+    for (int t = tid >> 6; t < ndl; t += nt >> 6) {
+        const int jd = dlist[t];
+        const GdtRingResult r = gdt_wave_ring<false, GEN>(S, jd, io, wv, wv.lane == 0);
+        npred += r.npred;
+        if (r.err & ERR_TIE) {
+            if (wv.lane == 0) {
+                const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
+                defer[pos] = jd;
+            }
+        } else if (wv.lane == 0) {
+            counts[io.perm[jd]] = r.count;
+            mx = max(mx, r.count);
+            er |= r.err;
+            nsum += (unsigned)r.count;
+        }
+    }
 }
 
 // Block totals of a ring kernel (every thread calls it): one set of atomics
@@ -100,7 +172,6 @@ __device__ inline void ring_block_totals(int mx, int er, unsigned npred, unsigne
 
 template <int PREC, int W, bool GEN = false>
 __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_tile(const GdtSet* __restrict__ sets, const GdtChunk* __restrict__ tiles,
-                     const int* __restrict__ list, const uint32_t* __restrict__ lscan,
                      const int* __restrict__ flags, const int* __restrict__ halt,
                      GdtRingIO io, int* __restrict__ counts, int* __restrict__ status,
                      unsigned long long* __restrict__ counters, int* __restrict__ defer)
@@ -126,11 +197,8 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     const int k0 = S.c0 + ch.start * GDT_TILE_CELLS;
     const int T0 = (int)io.cstart[k0], T1 = (int)io.cstart[k0 + GDT_TILE_CELLS];
     // the tile's items q in [Q0, Q1): point j = item(q)
-    int Q0 = list ? (int)lscan[T0] : T0, Q1 = list ? (int)lscan[T1] : T1;
-    TileFlags tf;
-    tf.mask = s_fmask;
-    tf.pre = s_fpre;
-    tf.nw = 0;
+    int Q0 = T0, Q1 = T1;
+    TileFlags tf = {s_fmask, s_fpre, 0};
     if (flags) {
         if (halt && *halt) return;
         const int npt = T1 - T0;
@@ -146,31 +214,11 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
             if (nf) atomicAdd(&status[ST_NFLAGGED], (int)nf);
             return;
         }
-        tf.nw = (npt + 63) >> 6;
-        for (int t0 = 0; t0 < 64 * tf.nw; t0 += nt) {
-            const int t = t0 + tid;
-            const bool f = t < npt && flags[io.perm[T0 + t]] >= 0;
-            const unsigned long long b = __ballot(f);
-            if ((tid & 63) == 0 && (t >> 6) < tf.nw) s_fmask[t >> 6] = b;
-        }
-        __syncthreads();
-        if (tid < 64) {
-            const uint32_t c = tid < tf.nw ? (uint32_t)__popcll(s_fmask[tid]) : 0u;
-            uint32_t x = c;
-#pragma unroll
-            for (int d = 1; d < 64; d <<= 1) {
-                const uint32_t y = __shfl_up(x, d, 64);
-                if (tid >= d) x += y;
-            }
-            if (tid < tf.nw) s_fpre[tid + 1] = x;
-            if (tid == 0) s_fpre[0] = 0u;
-        }
-        __syncthreads();
         Q0 = 0;
-        Q1 = (int)s_fpre[tf.nw];
+        Q1 = tile_gather_flags(flags, io.perm, T0, npt, s_fmask, s_fpre, tf);
         if (tid == 0 && Q1 > 0) atomicAdd(&status[ST_NFLAGGED], Q1);
     }
-    auto item = [&](int q) { return flags ? tile_flagged_slot(tf, T0, q) : (list ? list[q] : q); };
+    auto item = [&](int q) { return flags ? tile_flagged_slot(tf, T0, q) : q; };
     if (Q0 >= Q1) return;    // block-uniform: nothing to do in this tile
 
     const bool fits = gdt_stage_window<PREC == 32, GEN>(S, w, io, L, s_wsum);
@@ -250,37 +298,240 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
         }
     }
     if constexpr (PREC != GDT_EXACT) {
-    // Points whose circle left the window: one wavefront each, read from
-    // global memory (gdt_wave_ring), by this block's waves while other blocks
-    // still run their tiles.
+        __syncthreads();
+        tile_finish_deferred<GEN>(S, io, s_dlist, min((int)s_dn, GDT_TILE_DEFER), counts, status,
+                                  defer, npred, nsum, mx, er);
+    }
+    ring_block_totals(mx, er, npred, nfb, nsum, status, counters);
+}
+
+// Points left by the hull routine that go straight to wavefronts (at most).
+#define GDT_HULL_WAVES 16
+// Records of points with open triangles a block keeps (more are left to the
+// steps; a tile of random points has about 150).
+#define GDT_HULL_RECS 256
+// Records a wave closes together.
+#define GDT_HULL_TAKE 32
+
+// One block per tile, one point per lane: the hull routine (gdt_hull.h) over
+// all of the tile's points -- or, with `flags`, the flagged ones, as
+// k_one_ring_tile.  Waves take 64 points at a time; those with open triangles
+// (15 % of random points) are recorded in LDS, so that full waves close them,
+// where every wave would wait for its few.  The points left to the steps (under
+// 0.1 % of random points) take them, or when they are few a wavefront each, a
+// shorter chain.
+// Bound by the vector ALU and by the imbalance of its parts (1M points: 219 us
+// for staging and the lists, 100-115 us for the open triangles, 20 us for the
+// points left; FP64 adds and multiplies are half of the instructions), not by
+// memory (0.1 GB, 15 us).  Ring kernel of 1M / 4M uniform points 350 / 1,043 us
+// (the steps: 496 / 1,890), of a 1M near-lattice 282 (339).  Blocks of 512, two
+// to a compute unit: 1,024 threads took 477 us at 1M, 256 threads on 16x16
+// tiles 445, 320 threads 622; a cap of 96 registers for five waves spilled
+// (421).  Closing by each wave for its own lanes took 375 us, by single lanes
+// after a barrier 493, in block-wide rounds 460; without the drain before the
+// barrier 384.
+template <bool GEN>
+__global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict__ sets,
+                                                        const GdtChunk* __restrict__ tiles,
+                                                        const int* __restrict__ flags,
+                                                        const int* __restrict__ halt, GdtRingIO io,
+                                                        int* __restrict__ counts,
+                                                        int* __restrict__ status,
+                                                        unsigned long long* __restrict__ counters,
+                                                        int* __restrict__ defer)
+{
+    __shared__ uint32_t s_cs[GDT_WIN_CELLS + 1];
+    __shared__ gdt_d2 s_X64[GDT_WIN_MAXPTS + 1];
+    __shared__ int s_orig[GDT_WIN_MAXPTS];
+    __shared__ uint32_t s_wsum[16];
+    __shared__ int s_next, s_next2, s_rn, s_rt;
+    __shared__ int s_dlist[GDT_TILE_DEFER];
+    __shared__ uint32_t s_dn;
+    __shared__ unsigned long long s_fmask[GDT_WIN_MAXPTS / 64], s_smask[GDT_WIN_MAXPTS / 64];
+    __shared__ uint32_t s_fpre[GDT_WIN_MAXPTS / 64 + 1], s_spre[GDT_WIN_MAXPTS / 64 + 1];
+    __shared__ uint32_t s_rec[GDT_HULL_REC * GDT_HULL_RECS];
+    // [2 GDT_HULL_GROUPS * waves] the waves' queues, [GDT_HULL_WORDS * blockDim + 1] lists
+    extern __shared__ uint32_t s_dyn[];
+
+    const GdtChunk ch = tiles[blockIdx.x];
+    const GdtSet S = sets[ch.set];
+    const GdtTileWin w = gdt_tile_window(S, ch.start);
+    GdtTileLds L;
+    L.cs = s_cs; L.gstart = nullptr; L.X64 = s_X64; L.X32 = nullptr; L.orig = s_orig;
+    const int tid = threadIdx.x, nt = blockDim.x, lane = tid & 63;
+    const int k0 = S.c0 + ch.start * GDT_TILE_CELLS;
+    const int T0 = (int)io.cstart[k0], T1 = (int)io.cstart[k0 + GDT_TILE_CELLS];
+    const int npt = T1 - T0;
+    if (flags && halt && *halt) return;
+    TileFlags tf = {s_fmask, s_fpre, 0};
+    int Q0 = T0, Q1 = T1;
+    if (flags && npt <= GDT_WIN_MAXPTS) {
+        Q0 = 0;
+        Q1 = tile_gather_flags(flags, io.perm, T0, npt, s_fmask, s_fpre, tf);
+        if (tid == 0 && Q1 > 0) atomicAdd(&status[ST_NFLAGGED], Q1);
+    }
+    auto item = [&](int q) { return tf.nw ? tile_flagged_slot(tf, T0, q) : q; };
+    if (Q0 >= Q1) return;    // block-uniform: nothing to do in this tile
+
+    const bool fits = npt <= GDT_WIN_MAXPTS && gdt_stage_window<false, GEN>(S, w, io, L, s_wsum);
+    if (!fits) {
+        unsigned nf = 0;
+        for (int q = Q0 + tid; q < Q1; q += nt) {
+            const int j = item(q);
+            if (flags && !tf.nw) {      // (more points than a window holds: no mask)
+                if (flags[io.perm[j]] < 0) continue;
+                ++nf;
+            }
+            const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
+            defer[pos] = j;
+        }
+        if (nf) atomicAdd(&status[ST_NFLAGGED], (int)nf);
+        return;
+    }
+    if (tid == 0) {
+        s_next = s_next2 = s_rn = s_rt = 0;
+        s_dn = 0u;
+    }
+    const int nsw = (npt + 63) >> 6;
+    for (int t = tid; t < nsw; t += nt) s_smask[t] = 0ull;
+    for (int t = tid; t < GDT_HULL_RECS; t += nt) s_rec[GDT_HULL_REC * t + 1] = 0u;
     __syncthreads();
-    const int ndl = min((int)s_dn, GDT_TILE_DEFER);
-    if (ndl > 0) {
-        if (tid == 0) atomicAdd(&status[ST_NDEFER_TILE], ndl);
-        GdtWaveDev wv;
-        wv.lane = tid & 63;
-        for (int t = tid >> 6; t < ndl; t += nt >> 6) {
-            const int jd = s_dlist[t];
-            // (built without the tie rule and the other box shape, which would
-            // cost this kernel's main loop registers: a point with an exact tie
-            // goes to k_one_ring_deferred)
-            const GdtRingResult r = gdt_wave_ring<false, GEN>(S, jd, io, wv, wv.lane == 0);
-            npred += r.npred;
-            if (r.err & ERR_TIE) {
-                if (wv.lane == 0) {
-                    const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
-                    defer[pos] = jd;
+    uint32_t* const wq = s_dyn + 2 * GDT_HULL_GROUPS * (tid >> 6);
+    uint32_t* const wave_words =
+        s_dyn + 2 * GDT_HULL_GROUPS * (nt >> 6) + GDT_HULL_WORDS * (tid - lane);
+    uint32_t* const words = wave_words + GDT_HULL_WORDS * lane;
+    unsigned npred = 0, nsum = 0;
+    int mx = 0, er = 0;
+    // entry iv's row from the list in the lane's words
+    auto emit = [&](int iv, int n) {
+        const int i = L.orig[iv];
+        int* row = io.nbrs + (size_t)i * (size_t)io.stride;
+        for (int m = 0; m < n && m < io.stride; ++m) row[m] = L.orig[gdt_hull_entry(words, m)];
+        counts[i] = n;
+        mx = max(mx, n);
+        nsum += (unsigned)n;
+    };
+    auto lane_init = [&](GdtTileLane<double>& st, int j) {
+        if constexpr (GEN) gdt_tile_lane_init_gen(w, L, j, io, S, st);
+        else gdt_tile_lane_init<double>(w, L, j, io, S, st);
+    };
+    // slot j's point is left to the steps
+    auto leave = [&](int j) { atomicOr(&s_smask[(j - T0) >> 6], 1ull << ((j - T0) & 63)); };
+    for (;;) {
+        int c = 0;
+        if (lane == 0) c = atomicAdd(&s_next, 64);
+        const int q = Q0 + __builtin_amdgcn_readfirstlane(c) + lane;
+        if (q - lane >= Q1) break;      // (wave-uniform)
+        if (q < Q1) {
+            const int j = item(q);
+            GdtTileLane<double> st;
+            lane_init(st, j);
+            GdtHull h;
+            gdt_hull_build<GEN>(S, L, st, words, h, npred);
+            if (!h.bad && h.open != 0) {
+                const int r = atomicAdd(&s_rn, 1);
+                if (r < GDT_HULL_RECS) gdt_hull_save(h, st.iv, st.c0, words, s_rec + GDT_HULL_REC * r);
+                else h.bad = true;
+            } else if (!h.bad) {
+                emit(st.iv, h.n);
+            }
+            if (h.bad) leave(j);
+        }
+    }
+    // Records are closed by the waves that have no chunk left, while others
+    // still run theirs, and after a barrier the last ones.
+    auto drain = [&]() {
+        for (;;) {
+            int t = 0, take = 0;
+            if (lane == 0) {
+                t = __hip_atomic_load(&s_rt, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                for (;;) {
+                    const int n = min(__hip_atomic_load(&s_rn, __ATOMIC_RELAXED,
+                                                        __HIP_MEMORY_SCOPE_WORKGROUP),
+                                      GDT_HULL_RECS);
+                    take = min(GDT_HULL_TAKE, n - t);
+                    if (take <= 0) break;
+                    const int seen = atomicCAS(&s_rt, t, t + take);
+                    if (seen == t) break;
+                    t = seen;
                 }
-            } else if (wv.lane == 0) {
-                counts[io.perm[jd]] = r.count;
-                mx = max(mx, r.count);
-                er |= r.err;
-                nsum += (unsigned)r.count;
+            }
+            t = __builtin_amdgcn_readfirstlane(t);
+            take = __builtin_amdgcn_readfirstlane(take);
+            if (take <= 0) break;
+            GdtHull h = {0, 0, 0u, true, 0.};
+            int iv = 0, c0 = 0;
+            if (lane < take) {
+                const uint32_t* rec = s_rec + GDT_HULL_REC * (t + lane);
+                // (its wave reserved it just before it writes it)
+                while (__hip_atomic_load(rec + 1, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP) == 0u)
+                    __builtin_amdgcn_s_sleep(1);
+                gdt_hull_load(L, rec, h, iv, c0, words);
+            }
+            gdt_hull_close_wave<GEN>(S, L, iv, c0, wave_words, wq, h, npred);
+            if (lane < take) {
+                if (!h.bad) {
+                    emit(iv, h.n);
+                } else {
+                    // its slot: the cell's first slot plus the rank in the cell
+                    leave((int)io.cstart[gdt_tile_key(S, w, c0)] + iv - (int)L.cs[c0]);
+                }
+            }
+        }
+    };
+    drain();
+    __syncthreads();
+    drain();
+    __syncthreads();
+    // the points left to the steps, as in k_one_ring_tile; a few go straight to
+    // a wavefront each, a shorter chain than the steps'
+    TileFlags sf = {s_smask, s_spre, nsw};
+    const int nslow = tile_mask_prefix(sf, s_spre);
+    if (nslow > 0 && nslow <= GDT_HULL_WAVES) {
+        if (tid < nslow) s_dlist[tid] = tile_flagged_slot(sf, T0, tid);
+        if (tid == 0) s_dn = (uint32_t)nslow;
+    } else if (nslow > 0) {
+        int q = tid;
+        bool have = q < nslow;
+        int j = 0;
+        GdtTileLane<double> st;
+        st.tbl = words;
+        if (have) {
+            j = tile_flagged_slot(sf, T0, q);
+            lane_init(st, j);
+        }
+        while (__ballot(have) != 0) {
+            if (have) {
+                const int rc = gdt_tile_step_f64<1, false, GEN>(S, L, io, st, npred);
+                if (rc != STEP_RUN) {
+                    if (rc == STEP_DEFER) {
+                        const uint32_t dpos = atomicAdd(&s_dn, 1u);
+                        if (dpos < GDT_TILE_DEFER) {
+                            s_dlist[dpos] = j;
+                        } else {
+                            const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
+                            defer[pos] = j;
+                        }
+                    } else {
+                        counts[L.orig[st.iv]] = st.count;
+                        mx = max(mx, st.count);
+                        nsum += (unsigned)st.count;
+                        if (rc == STEP_NOCLOSE) er |= ERR_NOCLOSE;
+                    }
+                    q = nt + atomicAdd(&s_next2, 1);
+                    have = q < nslow;
+                    if (have) {
+                        j = tile_flagged_slot(sf, T0, q);
+                        lane_init(st, j);
+                    }
+                }
             }
         }
     }
-    }
-    ring_block_totals(mx, er, npred, nfb, nsum, status, counters);
+    __syncthreads();
+    tile_finish_deferred<GEN>(S, io, s_dlist, min((int)s_dn, GDT_TILE_DEFER), counts, status, defer,
+                              npred, nsum, mx, er);
+    ring_block_totals(mx, er, npred, 0u, nsum, status, counters);
 }
 
 // Words of a star lane's row table: one per cell row of the 7x7 block (the
@@ -461,62 +712,59 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
 hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nsets,
                                     const GdtChunk* tiles, int ntiles, int block, int lanes,
                                     bool general,
-                                    const int* list, const uint32_t* lscan,
                                     const int* flags, const int* halt,
                                     const GdtRingIO& io, int* counts, int* status,
-                                    unsigned long long* counters, int* defer,
+                                    unsigned long long* counters, int* defer, int many,
                                     hipEvent_t after_tile, hipStream_t s)
 {
     if (ntiles <= 0) return hipSuccess;
     if (block > 1024) block = 1024;
-    const size_t tbl = (5 * (size_t)block + 1) * sizeof(uint32_t);
-    // (the FP32-filtered step shares a point between at most two lanes)
-    const bool two = lanes == 2 || (lanes == 4 && precision == 32);
     if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) block = GDT_XTILE_BLOCK;
     if (general && precision != 64) return hipErrorInvalidValue;
-    if (general && lanes > 1)
-        hipLaunchKernelGGL((k_one_ring_tile<64, 2, true>), dim3(ntiles), dim3(block), tbl, s,
-                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
-                           defer);
-    else if (general)
-        hipLaunchKernelGGL((k_one_ring_tile<64, 1, true>), dim3(ntiles), dim3(block), tbl, s,
-                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
-                           defer);
-    else if (precision == GDT_EXACT && (lanes == 2 || lanes == 4))
-        hipLaunchKernelGGL((k_one_ring_tile<GDT_EXACT, 2>), dim3(ntiles), dim3(block), tbl, s,
-                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
-                           defer);
-    else if (precision == GDT_EXACT)
-        hipLaunchKernelGGL((k_one_ring_tile<GDT_EXACT, 1>), dim3(ntiles), dim3(block), tbl, s,
-                           d_sets, tiles, list, lscan, flags, halt, io, counts, status, counters,
-                           defer);
-    else if (precision == 64 && lanes == 4)
-        hipLaunchKernelGGL((k_one_ring_tile<64, 4>), dim3(ntiles), dim3(block), tbl, s, d_sets,
-                           tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
-    else if (precision == 32 && two)
-        hipLaunchKernelGGL((k_one_ring_tile<32, 2>), dim3(ntiles), dim3(block), tbl, s, d_sets,
-                           tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
-    else if (precision == 32)
-        hipLaunchKernelGGL((k_one_ring_tile<32, 1>), dim3(ntiles), dim3(block), tbl, s, d_sets,
-                           tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
-    else if (two)
-        hipLaunchKernelGGL((k_one_ring_tile<64, 2>), dim3(ntiles), dim3(block), tbl, s, d_sets,
-                           tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
-    else
-        hipLaunchKernelGGL((k_one_ring_tile<64, 1>), dim3(ntiles), dim3(block), tbl, s, d_sets,
-                           tiles, list, lscan, flags, halt, io, counts, status, counters, defer);
+#ifdef GDT_WIN_DENSE
+    // (windows of 4,096 points take a compute unit's LDS: one block of them)
+    block = precision == GDT_EXACT ? GDT_XTILE_BLOCK : 1024;
+    const bool hull = precision != GDT_EXACT;
+#else
+    const bool hull = precision == 64 && lanes == 1;
+#endif
+    const size_t tbl = (5 * (size_t)block + 1) * sizeof(uint32_t);
+    if (hull) {
+        // One lane per point in FP64: the hull kernel.  (Ring kernel of 1M / 4M
+        // uniform points: 350 / 1,043 us; the search steps took 496 / 1,890.)
+        const size_t words = (2 * GDT_HULL_GROUPS * (size_t)(block >> 6) +
+                              GDT_HULL_WORDS * (size_t)block + 1) * sizeof(uint32_t);
+        auto* k = general ? k_one_ring_hull<true> : k_one_ring_hull<false>;
+        hipLaunchKernelGGL(k, dim3(ntiles), dim3(block), words, s, d_sets, tiles, flags, halt, io,
+                           counts, status, counters, defer);
+    } else {
+        auto* k = k_one_ring_tile<GDT_EXACT, 1>;
+#ifndef GDT_WIN_DENSE
+        if (precision == GDT_EXACT && lanes > 1)
+            k = k_one_ring_tile<GDT_EXACT, 2>;
+        else if (precision == 32)
+            k = lanes > 1 ? k_one_ring_tile<32, 2> : k_one_ring_tile<32, 1>;
+        else if (precision == 64)
+            // (four lanes per point: in a rectangle only; elsewhere two)
+            k = general ? k_one_ring_tile<64, 2, true>
+                        : (lanes == 4 ? k_one_ring_tile<64, 4> : k_one_ring_tile<64, 2>);
+#endif
+        hipLaunchKernelGGL(k, dim3(ntiles), dim3(block), tbl, s, d_sets, tiles, flags, halt, io,
+                           counts, status, counters, defer);
+    }
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
     return gdt_launch_deferred(precision, d_sets, nsets, io, counts, status, counters,
-                               defer, s);
+                               defer, many, s);
 }
 
+#ifndef GDT_WIN_DENSE
 hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,
                                     const GdtChunk* tiles,
                                     int ntiles, int nsplit, int block, bool general,
                                     const GdtRingIO& io, int* counts, int* status,
-                                    unsigned long long* counters, int* defer,
+                                    unsigned long long* counters, int* defer, int many,
                                     hipEvent_t after_tile, hipStream_t s)
 {
     if (ntiles <= 0) return hipSuccess;
@@ -538,7 +786,8 @@ hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nse
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
     return gdt_launch_deferred(precision == GDT_EXACT ? GDT_EXACT : 64, d_sets, nsets, io, counts,
-                               status, counters, defer, s);
+                               status, counters, defer, many, s);
 }
+#endif
 
 }  // namespace GDT_TS_NS
