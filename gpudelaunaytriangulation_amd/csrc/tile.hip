@@ -28,8 +28,8 @@ namespace GDT_TS_NS {
 // in the next launch.  With W = 2 or 4 (FP64) neighbouring lanes share each
 // point, each scanning its part of every row (flags leave most lanes of a
 // block without a point otherwise, and a small grid leaves most of the chip
-// idle; the launcher takes W from the caller).  FP64 with one lane per point is
-// k_one_ring_hull's.  GEN: sets in general boxes (gdt_tile_search_f64).
+// idle; the launcher takes W from the caller).  One lane per point, in FP64 or
+// FP32-filtered, is k_one_ring_hull's.  GEN: sets in general boxes (gdt_tile_search_f64).
 // PREC = GDT_EXACT: the FP64 steps with every decision certified
 // (gdt_tile_search_f64, CERT), bound as they are by the lanes' chains of steps;
 // all its deferred points go to the next launch, where a wavefront per point
@@ -721,17 +721,19 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     if (block > 1024) block = 1024;
     if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) block = GDT_XTILE_BLOCK;
     if (general && precision != 64) return hipErrorInvalidValue;
+    // One lane per point, FP64 and FP32-filtered alike: the hull kernel, whose
+    // FP64 rows are the filtered path's too.  (Ring kernel of 1M / 4M uniform
+    // points 350 / 1,043 us; the search steps took 496 / 1,890 in FP64 and 544
+    // at 1M filtered.)
 #ifdef GDT_WIN_DENSE
     // (windows of 4,096 points take a compute unit's LDS: one block of them)
     block = precision == GDT_EXACT ? GDT_XTILE_BLOCK : 1024;
     const bool hull = precision != GDT_EXACT;
 #else
-    const bool hull = precision == 64 && lanes == 1;
+    const bool hull = precision != GDT_EXACT && lanes == 1;
 #endif
     const size_t tbl = (5 * (size_t)block + 1) * sizeof(uint32_t);
     if (hull) {
-        // One lane per point in FP64: the hull kernel.  (Ring kernel of 1M / 4M
-        // uniform points: 350 / 1,043 us; the search steps took 496 / 1,890.)
         const size_t words = (2 * GDT_HULL_GROUPS * (size_t)(block >> 6) +
                               GDT_HULL_WORDS * (size_t)block + 1) * sizeof(uint32_t);
         auto* k = general ? k_one_ring_hull<true> : k_one_ring_hull<false>;
@@ -743,7 +745,7 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
         if (precision == GDT_EXACT && lanes > 1)
             k = k_one_ring_tile<GDT_EXACT, 2>;
         else if (precision == 32)
-            k = lanes > 1 ? k_one_ring_tile<32, 2> : k_one_ring_tile<32, 1>;
+            k = k_one_ring_tile<32, 2>;
         else if (precision == 64)
             // (four lanes per point: in a rectangle only; elsewhere two)
             k = general ? k_one_ring_tile<64, 2, true>

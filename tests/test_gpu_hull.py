@@ -11,9 +11,25 @@ pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-from gpudelaunaytriangulation_amd import inputs  # noqa: E402
+from gpudelaunaytriangulation_amd import PREC_FP32F, PREC_FP64, inputs  # noqa: E402
+from gpudelaunaytriangulation_amd.delaunay import DelaunayGPU, PeriodicBoundaries  # noqa: E402
 from test_exact_mode import lattice  # noqa: E402
-from test_gpu_general_tile import rows, same  # noqa: E402
+from test_gpu_general_tile import cuda, same  # noqa: E402
+
+
+def rows(xy, moved, box, cell, precision=PREC_FP64, **config):
+    """Rows of xy, then of `moved` repaired from them, the number repaired and the statistics."""
+    n = len(xy)
+    dg = DelaunayGPU(n, 20, cell, PeriodicBoundaries(*box))
+    dg.setPrecision(precision)
+    dg.ctx.set_config(**config)
+    tri = torch.full((n * dg.MaxSize,), -7, dtype=torch.int32, device="cuda")
+    num = torch.zeros(n, dtype=torch.int32, device="cuda")
+    dg.globalDelaunayTriangulation(cuda(xy), tri, num)
+    st = dg.stats()
+    first = tri.cpu().numpy().reshape(n, -1).copy(), num.cpu().numpy().copy()
+    dg.testAndRepairDelaunayTriangulation(cuda(moved), tri, num)
+    return first, (tri.cpu().numpy().reshape(n, -1), num.cpu().numpy()), dg.last_repaired, st
 
 
 def square(n, seed):
@@ -71,3 +87,13 @@ def test_hull_kernel_ties_take_the_steps():
         print(f"[hull] ties, tile shift {ts}", flush=True)
         got, got2, _, _ = rows(xy, xy, box, 1.0, lanes=1, tile_shift=ts, repair_lanes=1)
         assert same(want, got) and same(want2, got2)
+
+
+@pytest.mark.parametrize("cell", [1.0, 1.2])
+def test_filtered_precision_takes_the_hull(cell):
+    xy, box = square(30011, 1)
+    print(f"[hull] FP32-filtered, cell {cell}", flush=True)
+    want, want2, count, _ = rows(xy, xy + 0.01, box, cell, lanes=1, tile_shift=5, repair_lanes=1)
+    got, got2, c, _ = rows(xy, xy + 0.01, box, cell, precision=PREC_FP32F, lanes=1, tile_shift=5,
+                           repair_lanes=1)
+    assert same(want, got) and same(want2, got2) and c == count
