@@ -278,12 +278,13 @@ GDT_UNROLL
             }
         }
     }
-    // angles counted from the nearest entry's, which comes first
+    // angles counted from the nearest entry's, which comes first as 0 (an entry
+    // a key's resolution before it wraps round to the end)
     const uint32_t turn = nkey & ~255u;
 GDT_UNROLL
     for (int i = 0; i < GDT_HULL_SLOTS; ++i) {
         const bool used = key[i] != 0xffffffffu;
-        const uint32_t k = key[i] == nkey ? nkey & 255u : key[i] - turn + 256u;
+        const uint32_t k = key[i] == nkey ? 0u : key[i] - turn;
         key[i] = used ? k : 0xffffffffu;
     }
     gdt_net_sort(key, std::make_index_sequence<(size_t)GDT_HULL_NET.n>{});
@@ -294,7 +295,7 @@ GDT_UNROLL
     const int n0 = ok ? ntot - 1 : 0;
     bool bad = !ok;
     auto entry = [&](uint32_t k) { return (int)(base + (k & 255u)); };
-    const int ks = ok ? entry(key[0]) : 0;
+    const int ks = ok ? entry(nkey) : 0;
     GdtHullPt s0 = pt(ks);
     int n = 1;
     lst[0] = (gdt_u16a)ks;
@@ -303,6 +304,20 @@ GDT_UNROLL
         int kb = ok ? entry(key[1]) : 0;
         GdtHullPt b = pt(kb);
         double ab = gdt_hull_cross(a, b);
+        const bool behind = (n0 > 2) & (ab < 0.) & (a.x * b.x + a.y * b.y > 0.);
+        if (gdt_hull_any(behind)) {
+            // nearly collinear with v and the first entry, but sorted after it
+            // by the keys: it comes last
+            const uint32_t k1 = key[1];
+GDT_UNROLL
+            for (int i = 1; i + 1 < GDT_HULL_SLOTS; ++i) {
+                const uint32_t next = i + 1 < n0 ? key[i + 1] : (i + 1 == n0 ? k1 : key[i]);
+                key[i] = behind ? next : key[i];
+            }
+            kb = ok ? entry(key[1]) : 0;
+            b = pt(kb);
+            ab = gdt_hull_cross(a, b);
+        }
 GDT_UNROLL
         for (int i = 2; i < GDT_HULL_SLOTS; ++i) {
             // (entry i - 1 between a and entry i, or the start after the last)

@@ -483,13 +483,27 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
     __syncthreads();
     drain();
     __syncthreads();
-    // the points left to the steps, as in k_one_ring_tile; a few go straight to
-    // a wavefront each, a shorter chain than the steps'
+    // The points left to the steps, as in k_one_ring_tile.  A few go to a
+    // wavefront each, a shorter chain than the steps': in the next launch, as
+    // one such point keeps its whole block (30 us of a tile's 120, and a third
+    // of the tiles has one: 256 sets of 3.9M points 1,378 -> 1,315 us per call,
+    // 1M points 443 -> 435); in this block for a repair's flagged points, few
+    // and far between (1M points 453 us, 473 in the next launch), and in
+    // general boxes, whose wavefronts take longer (1M points 495, 528).
     TileFlags sf = {s_smask, s_spre, nsw};
     const int nslow = tile_mask_prefix(sf, s_spre);
     if (nslow > 0 && nslow <= GDT_HULL_WAVES) {
-        if (tid < nslow) s_dlist[tid] = tile_flagged_slot(sf, T0, tid);
-        if (tid == 0) s_dn = (uint32_t)nslow;
+        const bool here = GEN || flags;
+        if (tid < nslow) {
+            const int j = tile_flagged_slot(sf, T0, tid);
+            if (here) {
+                s_dlist[tid] = j;
+            } else {
+                const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
+                defer[pos] = j;
+            }
+        }
+        if (here && tid == 0) s_dn = (uint32_t)nslow;
     } else if (nslow > 0) {
         int q = tid;
         bool have = q < nslow;
