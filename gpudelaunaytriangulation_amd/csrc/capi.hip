@@ -256,6 +256,18 @@ static int lanes_for(const gdt_context* c)
     return 2;
 }
 
+// Lanes per flagged point of a repair: the configuration's; else one, the hull
+// routine, with 32x32 tiles (1M points moved by 0.01 / 0.03: 476 / 514 us per
+// test and repair, 492 / 588 with two lanes; 64 sets of 980,000 points 476 us a
+// step, 491), and four with the 16x16 ones of smaller inputs, whose blocks end
+// with their longest chain of steps (131,072 points 187 us, 204 with two lanes
+// and 215 with one; 250,000: 212, 214, 270).
+static int repair_lanes_for(const gdt_context* c)
+{
+    if (c->cfg.repair_lanes) return c->cfg.repair_lanes;
+    return c->sets[0].tshift == 4 ? 4 : 1;
+}
+
 // Threads per block of the tile kernels: the configured count, at most 256
 // for 16x16 tiles (about 256 points each).
 static int tile_block(const gdt_context* c)
@@ -867,7 +879,7 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
     if (tiled_sets(c) && !exact) {
         GDT_CHECK(gdt_tiles::one_ring(c->sets[0].tshift, precision, c->d_sets.p,
                                       (int)c->sets.size(), c->tch.p, c->ntch, tile_block(c),
-                                      c->cfg.repair_lanes ? c->cfg.repair_lanes : 2,
+                                      repair_lanes_for(c),
                                       any_general(c), d_repair, c->halt,
                                       ring_io(c, d_nbrs, stride), d_counts, c->status.p,
                                       c->counters.p, c->defer.p, dense_windows(c), many_deferred(c),

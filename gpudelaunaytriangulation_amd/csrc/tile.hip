@@ -440,7 +440,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
     }
     // Records are closed by the waves that have no chunk left, while others
     // still run theirs, and after a barrier the last ones.
-    auto drain = [&]() {
+    auto drain = [&](int most) {
         for (;;) {
             int t = 0, take = 0;
             if (lane == 0) {
@@ -449,7 +449,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
                     const int n = min(__hip_atomic_load(&s_rn, __ATOMIC_RELAXED,
                                                         __HIP_MEMORY_SCOPE_WORKGROUP),
                                       GDT_HULL_RECS);
-                    take = min(GDT_HULL_TAKE, n - t);
+                    take = min(most, n - t);
                     if (take <= 0) break;
                     const int seen = atomicCAS(&s_rt, t, t + take);
                     if (seen == t) break;
@@ -479,9 +479,12 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
             }
         }
     };
-    drain();
+    // (a repair's few are shared out by all of the waves, most of which had no
+    // chunk)
+    if (!flags) drain(GDT_HULL_TAKE);
     __syncthreads();
-    drain();
+    const int nw = nt >> 6;
+    drain(flags ? min(GDT_HULL_TAKE, max(1, (min(s_rn, GDT_HULL_RECS) + nw - 1) / nw)) : GDT_HULL_TAKE);
     __syncthreads();
     // The points left to the steps, as in k_one_ring_tile.  A few go to a
     // wavefront each, a shorter chain than the steps': in the next launch, as
