@@ -459,11 +459,13 @@ static GdtRingIO ring_io(gdt_context* c, int* nbrs, int stride)
 }
 
 // The cell list of d_xy (no caller index -> slot map: nothing reads one).
-// (reset: zero the status words and counters on the way)
-static int build_cells(gdt_context* c, const double* d_xy, hipStream_t s, bool reset = false)
+// (reset: zero the status words and counters on the way; flags: set these [N] to -1)
+static int build_cells(gdt_context* c, const double* d_xy, hipStream_t s, bool reset = false,
+                       int* flags = nullptr)
 {
     if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[0], s));
     GdtCells cl = c->cells();
+    cl.flags = flags;
     GDT_CHECK(gdt_build_cells(c->d_sets.p, (int)c->sets.size(), c->pch.p, c->npch, c->kch.p,
                               c->nkch, c->total_n, c->total_keys, d_xy, cl, s,
                               reset ? c->status.p : nullptr, reset ? c->counters.p : nullptr));
@@ -784,34 +786,36 @@ static int enumerate(gdt_context* c, const int* d_nbrs, const int* d_counts, int
     return GDT_OK;
 }
 
-// Empty-circle test of the triangles enumerate() wrote.
-static int test_triangles(gdt_context* c, const double* d_xy, int cap, hipStream_t s)
+// Where the test leaves the triangle count: among the status words, or behind
+// the offsets of enumerate().
+static bool test_in_tiles(const gdt_context* c) { return tiled_sets(c) && !any_general(c); }
+static uint32_t* tested_triangles(gdt_context* c)
 {
-    const int n = c->total_n;
-    GDT_CHECK(gdt_fill_i32(c->repair.p, -1, (size_t)n, s));
-    GDT_CHECK(gdt_launch_test(c->d_sets.p, (int)c->sets.size(), c->tris.p, c->toff.p + n, cap,
-                              n, d_xy, c->cells(), c->repair.p, s));
-    return GDT_OK;
+    return test_in_tiles(c) ? reinterpret_cast<uint32_t*>(c->status.p + ST_NTRI)
+                            : c->toff.p + c->total_n;
 }
 
 // Triangles of the current rings and their empty-circle test: with the tiled
 // cell order of rectangles in one pass over the rings (no triangle array),
-// else enumerate() then test_triangles().  Leaves the triangle count in
-// toff[n] and the sum of counts in counters[CT_INSUM] either way.
+// else enumerate() and a test of its triangles.  Leaves the triangle count in
+// tested_triangles() and the sum of counts in counters[CT_INSUM] either way.
+// The status words are zero and the repair flags -1 on entry (the cell list's
+// first kernel does both: as launches of their own, and with the count copied
+// after the repair, they took 12 us of every call).
 static int triangles_and_test(gdt_context* c, const double* d_xy, const int* d_nbrs,
                               const int* d_counts, int stride, int cap, hipStream_t s)
 {
     const int n = c->total_n;
-    if (!tiled_sets(c) || any_general(c)) {
+    if (!test_in_tiles(c)) {
         int rc;
         if ((rc = enumerate(c, d_nbrs, d_counts, stride, c->tris.p, cap, false, s)) != GDT_OK) return rc;
-        return test_triangles(c, d_xy, cap, s);
+        GDT_CHECK(gdt_launch_test(c->d_sets.p, (int)c->sets.size(), c->tris.p, tested_triangles(c),
+                                  cap, n, d_xy, c->cells(), c->repair.p, s));
+        return GDT_OK;
     }
-    GDT_CHECK(c->toff.reserve((size_t)n + 1));
-    GDT_CHECK(gdt_fill_i32(c->repair.p, -1, (size_t)n, s));
     GDT_CHECK(gdt_tiles::ring_test(c->sets[0].tshift, c->d_sets.p, c->tch.p, c->ntch, d_nbrs,
                                    d_counts, stride, n, d_xy, c->cells(), c->repair.p, c->tpart.p,
-                                   c->toff.p + n, c->counters.p, c->status.p, s));
+                                   tested_triangles(c), c->counters.p, c->status.p, s));
     return GDT_OK;
 }
 
@@ -932,15 +936,15 @@ static int test_and_repair_sets(gdt_context* c, const double* d_xy, int stride, 
     GDT_CHECK(c->tris.reserve(3 * (size_t)cap));
     GDT_CHECK(c->repair.reserve((size_t)n));
     int rc;
-    if ((rc = reset_status(c, s)) != GDT_OK) return rc;
     // 1. cell list of the moved points (DelaunayGPU.cpp:580-586)
-    if ((rc = build_cells(c, d_xy, s)) != GDT_OK) return rc;
+    if ((rc = build_cells(c, d_xy, s, true, c->repair.p)) != GDT_OK) return rc;
     // 2. triangles of the current rings (getCircumcirclesGPU, DelaunayGPU.cpp:650-666) and
     // 3. their empty-circle test (testTriangulation, DelaunayGPU.cpp:607-648)
     if ((rc = triangles_and_test(c, d_xy, d_nbrs, d_counts, stride, cap, s)) != GDT_OK) return rc;
     // 4. repair the flagged points (locallyRepairDelaunayTriangulation, DelaunayGPU.cpp:87-115)
     if ((rc = repair_flagged(c, c->repair.p, stride, d_nbrs, d_counts, precision, s)) != GDT_OK) return rc;
-    GDT_CHECK(gdt_copy_u32(c->toff.p + n, reinterpret_cast<uint32_t*>(c->status.p + ST_NTRI), s));
+    if (!test_in_tiles(c))
+        GDT_CHECK(gdt_copy_u32(tested_triangles(c), reinterpret_cast<uint32_t*>(c->status.p + ST_NTRI), s));
     if ((rc = read_status(c, s)) != GDT_OK) return rc;
     const unsigned int h_nt = (unsigned int)c->h_status[ST_NTRI];
     const int nf = c->h_status[ST_NFLAGGED];
@@ -1013,11 +1017,10 @@ static int md_enqueue_step_halting(gdt_context* c, double* d_xy, int stride, int
     const int n = c->total_n, cap = 2 * n + 64;
     int rc;
     GDT_CHECK(gdt_launch_md_displace(c->d_sets.p, c->pch.p, c->npch, d_xy, sigma, seed, c->md.p, s));
-    if ((rc = reset_status(c, s)) != GDT_OK) return rc;
-    if ((rc = build_cells(c, d_xy, s)) != GDT_OK) return rc;
+    if ((rc = build_cells(c, d_xy, s, true, c->repair.p)) != GDT_OK) return rc;
     if ((rc = triangles_and_test(c, d_xy, d_nbrs, d_counts, stride, cap, s)) != GDT_OK) return rc;
     if ((rc = repair_flagged(c, c->repair.p, stride, d_nbrs, d_counts, precision, s)) != GDT_OK) return rc;
-    GDT_CHECK(gdt_launch_md_step_end(c->status.p, c->counters.p, c->toff.p + n, n, stride, c->md.p, s));
+    GDT_CHECK(gdt_launch_md_step_end(c->status.p, c->counters.p, tested_triangles(c), n, stride, c->md.p, s));
     return GDT_OK;
 }
 

@@ -384,7 +384,8 @@ __global__ __launch_bounds__(KB_THREADS) void k_kb_count(const GdtSet* __restric
                                                          KbPlan pl, uint32_t* __restrict__ bmat,
                                                          const int* __restrict__ halt,
                                                          int* __restrict__ st_zero,
-                                                         unsigned long long* __restrict__ ct_zero)
+                                                         unsigned long long* __restrict__ ct_zero,
+                                                         int* __restrict__ flags)
 {
     if (st_zero && blockIdx.x == 0) {
         if (threadIdx.x < ST_WORDS) st_zero[threadIdx.x] = 0;
@@ -407,6 +408,7 @@ __global__ __launch_bounds__(KB_THREADS) void k_kb_count(const GdtSet* __restric
             for (int u = 0; u < KB_BATCH; ++u) {
                 const int i = ib + u * KB_THREADS;
                 if (i < i1) {
+                    if (flags) flags[i] = -1;
                     cur.advance(i);
                     uint32_t key, packed;
                     double ox, oy;
@@ -680,6 +682,8 @@ __global__ __launch_bounds__(KB_THREADS) void k_kb_small(const GdtSet* __restric
     const uint32_t k0 = (uint32_t)bin << KB_SMALL_B;
     const int nk = min(1 << KB_SMALL_B, total_keys - (int)k0);
     if (bin == (int)gridDim.x - 1 && tid == 0) c.cstart[total_keys] = (uint32_t)n;
+    if (c.flags)
+        for (int i = bin * KB_THREADS + tid; i < n; i += (int)gridDim.x * KB_THREADS) c.flags[i] = -1;
     for (int q = tid; q <= nk; q += KB_THREADS) cst[q] = 0u;
     __syncthreads();
     // pk[u]: (cell in the bucket << 16) | arrival rank in the cell, or ~0
@@ -774,6 +778,10 @@ hipError_t gdt_build_cells(const GdtSet* d_sets, int nsets, const GdtChunk* pchu
             const hipError_t e = gdt_status_reset(status, ST_WORDS, counters, CT_WORDS, s);
             if (e != hipSuccess) return e;
         }
+        if (c.flags) {
+            const hipError_t e = gdt_fill_i32(c.flags, -1, (size_t)total_n, s);
+            if (e != hipSuccess) return e;
+        }
         return build_cells_single_level(d_sets, pchunks, npch, kchunks, nkch, total_keys, xy, c, s);
     }
     if (pl.B == KB_SMALL_B && pl.nkb <= KB_SMALL_NKB && total_n >= 1 && total_n <= KB_SMALL_N) {
@@ -782,7 +790,7 @@ hipError_t gdt_build_cells(const GdtSet* d_sets, int nsets, const GdtChunk* pchu
         return hipGetLastError();
     }
     hipLaunchKernelGGL(k_kb_count, dim3(pl.nb), dim3(KB_THREADS), pl.nkb * sizeof(uint32_t), s,
-                       d_sets, nsets, xy, total_n, pl, c.bmat, c.halt, status, counters);
+                       d_sets, nsets, xy, total_n, pl, c.bmat, c.halt, status, counters, c.flags);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     hipLaunchKernelGGL(k_kb_rowscan, dim3(pl.nkb), dim3(KB_NB), 0, s, pl, c.bmat, c.bscan);

@@ -30,6 +30,7 @@ struct GdtCells {
     uint32_t* bscan;    // [gdt_bucket_words(N, K)] their exclusive scan
     const int* halt;    // device word: when non-null and set, the kernels of the
                         // build (and of the tests that take these arrays) exit at once
+    int* flags = nullptr;   // [N] set to -1 on the way when non-null (the repair flags)
 };
 
 // Words of the (bucket, block) count table of the cell-list build.
