@@ -305,8 +305,10 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     ring_block_totals(mx, er, npred, nfb, nsum, status, counters);
 }
 
-// Points left by the hull routine that go straight to wavefronts (at most).
+// Points of a tile left by the hull routine that go straight to wavefronts (at most).
 #define GDT_HULL_WAVES 16
+// Tiles of a launch whose few points left go to the next one (at least).
+#define GDT_HULL_LATER 768u
 // Records of points with open triangles a block keeps (more are left to the
 // steps; a tile of random points has about 150).
 #define GDT_HULL_RECS 256
@@ -487,16 +489,19 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
     drain(flags ? min(GDT_HULL_TAKE, max(1, (min(s_rn, GDT_HULL_RECS) + nw - 1) / nw)) : GDT_HULL_TAKE);
     __syncthreads();
     // The points left to the steps, as in k_one_ring_tile.  A few go to a
-    // wavefront each, a shorter chain than the steps': in the next launch, as
-    // one such point keeps its whole block (30 us of a tile's 120, and a third
-    // of the tiles has one: 256 sets of 3.9M points 1,378 -> 1,315 us per call,
-    // 1M points 443 -> 435); in this block for a repair's flagged points, few
-    // and far between (1M points 453 us, 473 in the next launch), and in
-    // general boxes, whose wavefronts take longer (1M points 495, 528).
+    // wavefront each, a shorter chain than the steps': by this block's waves, or
+    // in the next launch, as one such point keeps its whole block 30 us longer and
+    // a third of the 32x32 tiles has one.  That launch takes 50 us for itself, so
+    // it pays where the tiles come round more than one and a half times
+    // (GDT_HULL_LATER of them, two to a compute unit: 256 sets of 3.9M points
+    // 1,378 -> 1,315 us per call, 1M points 443 -> 435; 200,000 points in 10 sets
+    // 241 in the next launch, 202 here), but not for a repair's flagged points, few and
+    // far between (1M points 453 us here, 473), nor in general boxes, whose
+    // wavefronts take longer (1M points 495, 528).
     TileFlags sf = {s_smask, s_spre, nsw};
     const int nslow = tile_mask_prefix(sf, s_spre);
     if (nslow > 0 && nslow <= GDT_HULL_WAVES) {
-        const bool here = GEN || flags;
+        const bool here = GEN || flags || GDT_TILE_SHIFT == 4 || gridDim.x < GDT_HULL_LATER;
         if (tid < nslow) {
             const int j = tile_flagged_slot(sf, T0, tid);
             if (here) {
