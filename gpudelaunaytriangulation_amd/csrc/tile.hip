@@ -305,10 +305,121 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     ring_block_totals(mx, er, npred, nfb, nsum, status, counters);
 }
 
+// Words of a star lane's row table: one per cell row of the 7x7 block (the
+// uniform scan reads no word beyond its rows; a step's own tables, at most
+// five rows and the word read after them, fit in the first six).
+#define STAR_TBL (2 * GDT_SCAN + 1)
+
+// One point by a wavefront (st: the point's state, the same in every lane, with
+// the lane's own table of STAR_TBL words; k_one_ring_star describes it).  Returns
+// STEP_DONE, STEP_NOCLOSE or STEP_DEFER, the row's length in count.
+template <bool CERT, bool GEN>
+__device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtRingIO& io,
+                                GdtTileLane<double>& st, unsigned& npred, int& count)
+{
+    const int lane = (int)(threadIdx.x & 63);
+    // the lanes' block, as one row table (every lane the same): the
+    // (2 GDT_SCAN + 1)^2 cells when they hold at most 64 entries, else
+    // the (2 GDT_SCAN0 + 1)^2 cells; and this lane's entry of it
+    const GdtClip whole = {0.f, 0.f, 0};
+    int ph = GDT_SCAN;
+    int tot = (int)gdt_block_rows(L, st.c0, ph, whole, st.tbl);
+    if (tot > 64) {
+        ph = GDT_SCAN0;
+        tot = (int)gdt_block_rows(L, st.c0, ph, whole, st.tbl);
+    }
+    int kg = -1;
+    for (int acc = 0, r = 0; acc < tot; ++r) {      // (the table's non-empty rows)
+        const uint32_t t = st.tbl[r];
+        const int b = (int)(t & 0xffffu), n = (int)(t >> 16) - b;
+        if (lane >= acc && lane < acc + n) kg = b + lane - acc;
+        acc += n;
+    }
+    int bk = -1, rc = STEP_DEFER;
+    if (tot <= 64 && kg >= 0) {
+        GdtTileLane<double> sl = st;
+        if (kg != st.iv) {
+            const gdt_d2 X = L.X64[kg];
+            sl.ak = kg;
+            sl.ax = X.x - st.vx;
+            sl.ay = X.y - st.vy;
+        }
+        double bx, by;
+        rc = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
+                                          (unsigned)tot, ph, &io);
+    }
+    int res = STEP_RUN;
+    if (CERT && !gdt_tile_x_range(S, io, L.orig[st.iv])) {
+        res = STEP_DEFER;
+    } else if (tot > 64) {
+        if (lane == 0) {
+            int r = STEP_RUN;
+            while (r == STEP_RUN) r = gdt_tile_step_f64<1, CERT, GEN>(S, L, io, st, npred);
+            res = r;
+            count = st.count;
+        }
+    } else {
+        const unsigned long long mv = __ballot(kg == st.iv);
+        const int hv = __ffsll((long long)mv) - 1;
+        int nn = __shfl(bk, hv, 64), nrc = __shfl(rc, hv, 64);
+        if (nrc != STEP_RUN) {
+            // not certified over the block: lane 0 runs the full search
+            if (lane == 0) {
+                double bx, by;
+                nrc = gdt_tile_search_f64<1, CERT, GEN>(S, L, st, npred, 0, true, nn, bx, by,
+                                                   nullptr, 0, GDT_SCAN0, &io);
+            }
+            nrc = __shfl(nrc, 0, 64);
+            nn = __shfl(nn, 0, 64);
+        }
+        if (nrc != STEP_RUN) {
+            res = STEP_DEFER;
+        } else {
+            if (lane == 0) st.row[0] = L.orig[nn];
+            count = 1;
+            for (int cur = nn;;) {
+                const unsigned long long m = __ballot(kg == cur && rc == STEP_RUN);
+                int nx;
+                if (m) {
+                    nx = __shfl(bk, __ffsll((long long)m) - 1, 64);
+                } else {
+                    // no lane certified cur's successor: lane 0 runs the
+                    // full search from cur (extension included)
+                    int r = STEP_DEFER, b = -1;
+                    if (lane == 0) {
+                        GdtTileLane<double> sl = st;
+                        const gdt_d2 X = L.X64[cur];
+                        sl.ak = cur;
+                        sl.ax = X.x - st.vx;
+                        sl.ay = X.y - st.vy;
+                        double bx, by;
+                        r = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, true, b, bx, by,
+                                                         nullptr, 0, GDT_SCAN0, &io);
+                    }
+                    if (__shfl(r, 0, 64) != STEP_RUN) {
+                        res = STEP_DEFER;
+                        break;
+                    }
+                    nx = __shfl(b, 0, 64);
+                }
+                if (nx == nn) {
+                    res = STEP_DONE;
+                    break;
+                }
+                if (lane == 0 && count < io.stride) st.row[count] = L.orig[nx];
+                if (++count > GDT_HARD_CAP) {
+                    res = STEP_NOCLOSE;
+                    break;
+                }
+                cur = nx;
+            }
+        }
+    }
+    return res;
+}
+
 // Points of a tile left by the hull routine that go straight to wavefronts (at most).
 #define GDT_HULL_WAVES 16
-// Tiles of a launch whose few points left go to the next one (at least).
-#define GDT_HULL_LATER 768u
 // Records of points with open triangles a block keeps (more are left to the
 // steps; a tile of random points has about 150).
 #define GDT_HULL_RECS 256
@@ -488,30 +599,31 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
     const int nw = nt >> 6;
     drain(flags ? min(GDT_HULL_TAKE, max(1, (min(s_rn, GDT_HULL_RECS) + nw - 1) / nw)) : GDT_HULL_TAKE);
     __syncthreads();
-    // The points left to the steps, as in k_one_ring_tile.  A few go to a
-    // wavefront each, a shorter chain than the steps': by this block's waves, or
-    // in the next launch, as one such point keeps its whole block 30 us longer and
-    // a third of the 32x32 tiles has one.  That launch takes 50 us for itself, so
-    // it pays where the tiles come round more than one and a half times
-    // (GDT_HULL_LATER of them, two to a compute unit: 256 sets of 3.9M points
-    // 1,378 -> 1,315 us per call, 1M points 443 -> 435; 200,000 points in 10 sets
-    // 241 in the next launch, 202 here), but not for a repair's flagged points, few and
-    // far between (1M points 453 us here, 473), nor in general boxes, whose
-    // wavefronts take longer (1M points 495, 528).
+    // The points left to the steps, as in k_one_ring_tile.  Few of them take a
+    // wavefront each, as the star kernel's points: one search's chain for the
+    // ring, and one more where a circle leaves the lanes' block, not a chain of
+    // searches (a tile in three has such a point, and ends with it).
     TileFlags sf = {s_smask, s_spre, nsw};
     const int nslow = tile_mask_prefix(sf, s_spre);
     if (nslow > 0 && nslow <= GDT_HULL_WAVES) {
-        const bool here = GEN || flags || GDT_TILE_SHIFT == 4 || gridDim.x < GDT_HULL_LATER;
-        if (tid < nslow) {
-            const int j = tile_flagged_slot(sf, T0, tid);
-            if (here) {
-                s_dlist[tid] = j;
-            } else {
-                const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
-                defer[pos] = j;
+        for (int t = tid >> 6; t < nslow; t += nt >> 6) {       // (wave-uniform)
+            const int j = tile_flagged_slot(sf, T0, t);
+            GdtTileLane<double> st;
+            st.tbl = words;
+            lane_init(st, j);
+            int count = 0;
+            const int res = star_ring<false, GEN>(S, L, io, st, npred, count);
+            if (lane == 0) {
+                if (res == STEP_DEFER) {
+                    s_dlist[atomicAdd(&s_dn, 1u)] = j;
+                } else {
+                    counts[L.orig[st.iv]] = count;
+                    mx = max(mx, count);
+                    nsum += (unsigned)count;
+                    if (res == STEP_NOCLOSE) er |= ERR_NOCLOSE;
+                }
             }
         }
-        if (here && tid == 0) s_dn = (uint32_t)nslow;
     } else if (nslow > 0) {
         int q = tid;
         bool have = q < nslow;
@@ -555,11 +667,6 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
                               npred, nsum, mx, er);
     ring_block_totals(mx, er, npred, 0u, nsum, status, counters);
 }
-
-// Words of a star lane's row table: one per cell row of the 7x7 block (the
-// uniform scan reads no word beyond its rows; a step's own tables, at most
-// five rows and the word read after them, fit in the first six).
-#define STAR_TBL (2 * GDT_SCAN + 1)
 
 // One wavefront per point (small grids; FP64 predicates): lane g takes entry g
 // of the cell block around the point's cell (7x7 cells, or 5x5 when the 7x7
@@ -619,103 +726,8 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
         st.tbl = s_tbl + STAR_TBL * tid;
         if constexpr (GEN) gdt_tile_lane_init_gen(w, L, q, io, S, st);
         else gdt_tile_lane_init<double>(w, L, q, io, S, st);
-        // the lanes' block, as one row table (every lane the same): the
-        // (2 GDT_SCAN + 1)^2 cells when they hold at most 64 entries, else
-        // the (2 GDT_SCAN0 + 1)^2 cells; and this lane's entry of it
-        const GdtClip whole = {0.f, 0.f, 0};
-        int ph = GDT_SCAN;
-        int tot = (int)gdt_block_rows(L, st.c0, ph, whole, st.tbl);
-        if (tot > 64) {
-            ph = GDT_SCAN0;
-            tot = (int)gdt_block_rows(L, st.c0, ph, whole, st.tbl);
-        }
-        int kg = -1;
-        for (int acc = 0, r = 0; acc < tot; ++r) {      // (the table's non-empty rows)
-            const uint32_t t = st.tbl[r];
-            const int b = (int)(t & 0xffffu), n = (int)(t >> 16) - b;
-            if (lane >= acc && lane < acc + n) kg = b + lane - acc;
-            acc += n;
-        }
-        int bk = -1, rc = STEP_DEFER;
-        if (tot <= 64 && kg >= 0) {
-            GdtTileLane<double> sl = st;
-            if (kg != st.iv) {
-                const gdt_d2 X = L.X64[kg];
-                sl.ak = kg;
-                sl.ax = X.x - st.vx;
-                sl.ay = X.y - st.vy;
-            }
-            double bx, by;
-            rc = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, false, bk, bx, by, st.tbl,
-                                              (unsigned)tot, ph, &io);
-        }
-        int res = STEP_RUN, count = 0;
-        if (CERT && !gdt_tile_x_range(S, io, L.orig[st.iv])) {
-            res = STEP_DEFER;
-        } else if (tot > 64) {
-            if (lane == 0) {
-                int r = STEP_RUN;
-                while (r == STEP_RUN) r = gdt_tile_step_f64<1, CERT, GEN>(S, L, io, st, npred);
-                res = r;
-                count = st.count;
-            }
-        } else {
-            const unsigned long long mv = __ballot(kg == st.iv);
-            const int hv = __ffsll((long long)mv) - 1;
-            int nn = __shfl(bk, hv, 64), nrc = __shfl(rc, hv, 64);
-            if (nrc != STEP_RUN) {
-                // not certified over the block: lane 0 runs the full search
-                if (lane == 0) {
-                    double bx, by;
-                    nrc = gdt_tile_search_f64<1, CERT, GEN>(S, L, st, npred, 0, true, nn, bx, by,
-                                                       nullptr, 0, GDT_SCAN0, &io);
-                }
-                nrc = __shfl(nrc, 0, 64);
-                nn = __shfl(nn, 0, 64);
-            }
-            if (nrc != STEP_RUN) {
-                res = STEP_DEFER;
-            } else {
-                if (lane == 0) st.row[0] = L.orig[nn];
-                count = 1;
-                for (int cur = nn;;) {
-                    const unsigned long long m = __ballot(kg == cur && rc == STEP_RUN);
-                    int nx;
-                    if (m) {
-                        nx = __shfl(bk, __ffsll((long long)m) - 1, 64);
-                    } else {
-                        // no lane certified cur's successor: lane 0 runs the
-                        // full search from cur (extension included)
-                        int r = STEP_DEFER, b = -1;
-                        if (lane == 0) {
-                            GdtTileLane<double> sl = st;
-                            const gdt_d2 X = L.X64[cur];
-                            sl.ak = cur;
-                            sl.ax = X.x - st.vx;
-                            sl.ay = X.y - st.vy;
-                            double bx, by;
-                            r = gdt_tile_search_f64<1, CERT, GEN>(S, L, sl, npred, 0, true, b, bx, by,
-                                                             nullptr, 0, GDT_SCAN0, &io);
-                        }
-                        if (__shfl(r, 0, 64) != STEP_RUN) {
-                            res = STEP_DEFER;
-                            break;
-                        }
-                        nx = __shfl(b, 0, 64);
-                    }
-                    if (nx == nn) {
-                        res = STEP_DONE;
-                        break;
-                    }
-                    if (lane == 0 && count < io.stride) st.row[count] = L.orig[nx];
-                    if (++count > GDT_HARD_CAP) {
-                        res = STEP_NOCLOSE;
-                        break;
-                    }
-                    cur = nx;
-                }
-            }
-        }
+        int count = 0;
+        const int res = star_ring<CERT, GEN>(S, L, io, st, npred, count);
         if (lane == 0) {
             if (res == STEP_DEFER) {
                 const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
