@@ -82,6 +82,11 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
 // Deferred points: the first GDT_WAVE_CAP one wavefront each (GDT_WAVE_BLOCKS
 // blocks of 256 threads), the rest one lane each, in one launch.
 #define GDT_WAVE_CAP 8192
+// The exact mode's lists up to this length take a wavefront per point, longer
+// ones a lane per point: wavefronts take about 0.45 us a point together, the lanes
+// 1.7 ms for their longest chain however many there are (lattices of exact ties,
+// 65,536 points: 4.6 ms per call with wavefronts first, 1.7 with lanes).
+#define GDT_WAVE_CAP_EXACT 3072
 #define GDT_WAVE_BLOCKS 512
 // Threads per block (at most) of the exact mode's tile and star kernels: two
 // waves per SIMD, so that the double-double decisions keep 256 registers.

@@ -131,7 +131,9 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
     const int lane = (int)(threadIdx.x & 63);
     const int wid = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const int nw = (int)((gridDim.x * blockDim.x) >> 6);
-    const int all = (int)*worklen, len = min(all, cap);
+    const int all = (int)*worklen;
+    // (the exact mode takes a longer list one lane each from its start)
+    const int len = PREC == GDT_EXACT && all > cap ? 0 : min(all, cap);
     GdtWaveDev w;
     w.lane = lane;
     unsigned npred = 0, nsum = 0;
@@ -165,7 +167,7 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
         }
     }
     if (all > cap && !waves_only)
-        one_ring_lanes<PREC>(sets, nsets, worklist, cap, all, io, counts, status, counters,
+        one_ring_lanes<PREC>(sets, nsets, worklist, len, all, io, counts, status, counters,
                              nullptr);
 }
 
@@ -181,14 +183,14 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                            many);
     else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_deferred<GDT_EXACT>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s,
-                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
-                           many);
+                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP_EXACT, io, counts, status,
+                           counters, 0);
     else
         hipLaunchKernelGGL(k_one_ring_deferred<64>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
                            nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
                            many);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !many) return e;
+    if (e != hipSuccess || !many || precision == GDT_EXACT) return e;
     return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer, ndefer,
                                GDT_WAVE_CAP, many, io, counts, status, counters, nullptr, s);
 }
