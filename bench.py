@@ -80,7 +80,7 @@ def parse():
     return ap.parse_args()
 
 
-TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_one_ring_tile_uniform1M_hbm_traffic.md")
+TRAFFIC_FILE = os.path.join(ROOT, "profiles", "k_one_ring_hull_uniform1M.md")
 
 
 def measured_traffic(kernel: str):
@@ -496,7 +496,7 @@ def main():
     # FP32-filtered path, decision-identical, is reported beside it.
     head = f64 if "fp64" in out else f32
     head_name = "fp64" if "fp64" in out else "fp32f"
-    head_kernel = "k_one_ring_tile<64, 1>" if head_name == "fp64" else "k_one_ring_tile<32, 1>"
+    head_kernel = "k_one_ring_hull<false>"      # (in either precision)
     value = n / (head["ms"] * 1e-3)
     ring_bytes = RING_BYTES_PER_POINT * n
     achieved = ring_bytes / (head["ring_ms"] * 1e-3) / 1e9
@@ -554,10 +554,8 @@ def main():
                       "cell_list": f32["cell_ms"]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": (measured_traffic("k_one_ring_tile<64>" if head_name == "fp64"
-                                                  else "k_one_ring_tile<32>")
-                                 if n == N_POINTS else None),
-                     "traffic_source": "profiles/k_one_ring_tile_uniform1M_hbm_traffic.md",
+                     "traffic": measured_traffic("k_one_ring_hull<false>") if n == N_POINTS else None,
+                     "traffic_source": "profiles/k_one_ring_hull_uniform1M.md",
                      "kernel": head_kernel, "algorithmic_bytes_per_launch": ring_bytes},
         "triangulation_roofline_frac": TRI_BYTES(n, n) / (head["ms"] * 1e-3) / 1e9 / HBM_PEAK_GBS,
         "cpu_baseline": cpu,

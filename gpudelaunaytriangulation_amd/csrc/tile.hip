@@ -431,13 +431,14 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
 // k_one_ring_tile.  Waves take 64 points at a time; those with open triangles
 // (15 % of random points) are recorded in LDS, so that full waves close them,
 // where every wave would wait for its few.  The points left to the steps (under
-// 0.1 % of random points) take them, or when they are few a wavefront each, a
-// shorter chain.
-// Bound by the vector ALU and by the imbalance of its parts (1M points: 219 us
-// for staging and the lists, 100-115 us for the open triangles, 20 us for the
-// points left; FP64 adds and multiplies are half of the instructions), not by
-// memory (0.1 GB, 15 us).  Ring kernel of 1M / 4M uniform points 350 / 1,043 us
-// (the steps: 496 / 1,890), of a 1M near-lattice 282 (339).  Blocks of 512, two
+// 0.1 % of random points) take them, or when they are few a wavefront's star
+// search each.
+// Bound by the vector ALU and by the imbalance of its parts (a 1M-point tile:
+// 9 us for staging, 65 for the lists, 39 for the open triangles, and 40 more in
+// the third of the tiles with a point left; FP64 adds and multiplies are half of
+// the instructions), not by memory (0.14 GB, 20 us).  Ring kernel of 1M / 3.9M
+// uniform points 342 / 1,149 us (the steps: 496 / 1,890 at 4M), of a 1M
+// near-lattice 228 (339).  Blocks of 512, two
 // to a compute unit: 1,024 threads took 477 us at 1M, 256 threads on 16x16
 // tiles 445, 320 threads 622; a cap of 96 registers for five waves spilled
 // (421).  Closing by each wave for its own lanes took 375 us, by single lanes
@@ -756,9 +757,8 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     if (precision == GDT_EXACT && block > GDT_XTILE_BLOCK) block = GDT_XTILE_BLOCK;
     if (general && precision != 64) return hipErrorInvalidValue;
     // One lane per point, FP64 and FP32-filtered alike: the hull kernel, whose
-    // FP64 rows are the filtered path's too.  (Ring kernel of 1M / 4M uniform
-    // points 350 / 1,043 us; the search steps took 496 / 1,890 in FP64 and 544
-    // at 1M filtered.)
+    // FP64 rows are the filtered path's too.  (Ring kernel of 1M uniform points
+    // 342 us; the search steps took 496 in FP64 and 544 filtered.)
 #ifdef GDT_WIN_DENSE
     // (windows of 4,096 points take a compute unit's LDS: one block of them)
     block = precision == GDT_EXACT ? GDT_XTILE_BLOCK : 1024;
