@@ -838,7 +838,8 @@ GDT_HD inline int gdt_tile_search_f64(const GdtSet& S, const GdtTileLds& L,
         pair_reduce();
         ok = true;
     }
-    if (!ok) return STEP_DEFER;     // (a best of GDT_TIE is never certified)
+    // (a best of GDT_TIE is never certified, and the box's rest may have met one)
+    if (!ok || bk < 0) return STEP_DEFER;
     best();
     return STEP_RUN;
 }
