@@ -461,6 +461,7 @@ GDT_HD inline double gdt_incircle64(const Circ64& k, double cx, double cy)
 // tilts the plane through the three about the line through the other two),
 // and as outside when it is c.  p* are caller indices.
 GDT_HD inline int gdt_imin(int x, int y) { return x < y ? x : y; }
+GDT_HD inline int gdt_imax(int x, int y) { return x > y ? x : y; }
 GDT_HD inline bool gdt_nn_tie(int pc, int pb) { return pc < pb; }
 GDT_HD inline bool gdt_incircle_tie(int pv, int pa, int pb, int pc, double ax, double ay,
                                     double bx, double by, double cx, double cy)

@@ -198,13 +198,17 @@ GDT_HD inline GdtRingResult gdt_wave_ring(const GdtSet& S, int j, const GdtRingI
             };
             g = w.template ring<TIES>(g, wrap, ax, ay, t, lane_fn);
         };
-        // The square [-hs,hs]^2 first (hs = 2), then either the rest of the
-        // bounding box of the current circle in one pass -- every later best's
-        // circle lies inside it (circles through v and a with centres left of
-        // v->a are nested along the bisector), so the search is then certified
-        // -- or, while there is no candidate or the box reaches far beyond the
-        // square or past rmax, the next Chebyshev rings (one without a
-        // candidate, else two).
+        // The square [-hs,hs]^2 first (hs = 2), then the rest of the current
+        // circle's bounding box -- every later best's circle lies inside it
+        // (circles through v and a with centres left of v->a are nested along
+        // the bisector), so the search is then certified.  A box far beyond the
+        // square mostly belongs to a best that a nearer candidate will replace:
+        // it is scanned from the square outwards, doubling, each time cut to
+        // the box of what was found.  (262,144 points filling 0.8 of a box, searches
+        // across the void: 8.0 ms per call, 36 with two rings of cells a pass, 13.3
+        // with the whole box at once; 2^20 random points of 0.36 to a cell 2.7 ms,
+        // with the whole box at once 28.9.)
+        // While there is no candidate or no circle, the next Chebyshev ring.
         int hs = S.rmax < 2 ? S.rmax : 2;
         pass(-hs, hs, -hs, hs, -1);
         for (;;) {
@@ -243,20 +247,19 @@ GDT_HD inline GdtRingResult gdt_wave_ring(const GdtSet& S, int j, const GdtRingI
                 }
                 if (boxed) {
                     if (dx0 >= -hs && dx1 <= hs && dy0 >= -hs && dy1 <= hs) return true;
-                    // (a box far beyond the scanned square belongs to a best
-                    // that a nearer candidate will replace: the square grows
-                    // first)
-                    const int lim = gdt_imin(S.rmax, hs + 4);
-                    if (dx0 >= -lim && dx1 <= lim && dy0 >= -lim && dy1 <= lim) {
-                        pass(dx0, dx1, dy0, dy1, hs);
-                        return true;
+                    const int to = gdt_imin(S.rmax, hs + (hs > 4 ? hs : 4));
+                    if (hs < to) {
+                        pass(gdt_imax(dx0, -to), gdt_imin(dx1, to), gdt_imax(dy0, -to),
+                             gdt_imin(dy1, to), hs);
+                        if (dx0 >= -to && dx1 <= to && dy0 >= -to && dy1 <= to) return true;
+                        hs = to;
+                        continue;
                     }
                 }
             }
             if (hs >= S.rmax) return false;
-            const int to = gdt_imin(S.rmax, g.k >= 0 ? hs + 2 : hs + 1);
-            pass(-to, to, -to, to, hs);
-            hs = to;
+            ++hs;
+            pass(-hs, hs, -hs, hs, hs - 1);
         }
     };
 
