@@ -233,12 +233,26 @@ static bool dense_windows(const gdt_context* c)
     return c->sets[0].tshift == 5 && window_points(c->sets, 5) > GDT_DENSE_WINDOW;
 }
 
-// Whether even these will mostly overflow, so that nearly every point is handed
-// on (gdt_launch_deferred): their number, else 0.
-static int many_deferred(const gdt_context* c)
+// General boxes run FP64 predicates (the FP32 filter's bounds are for
+// rectangular cells).
+static bool any_general(const gdt_context* c)
 {
+    for (const auto& s : c->sets)
+        if (s.general) return true;
+    return false;
+}
+
+// What becomes of a long list of deferred points (gdt_launch_deferred): a
+// launch behind where even the larger windows will mostly overflow, so that
+// nearly every point is handed on; else it waits for the count (read_rings) where
+// the host reads one, which the steps of a Brownian loop do not.
+static int rest_of_deferred(const gdt_context* c, int precision)
+{
+    const bool tiled = c->sets[0].tiled;
+    if (precision == GDT_PREC_EXACT) return GDT_LIST_LATER;
     const int ts = c->sets[0].tshift;
-    return window_points(c->sets, ts) > (ts == 4 ? 1000. : 4000.) ? c->total_n : 0;
+    if (tiled && window_points(c->sets, ts) > (ts == 4 ? 1000. : 4000.)) return c->total_n;
+    return c->halt ? GDT_REST_HERE : GDT_REST_LATER;
 }
 
 // Lanes per point of the global triangulation: the configuration's; else a
@@ -299,14 +313,6 @@ static bool box_ok(const double b[4], int words)
     return std::isfinite(det) && std::fabs(det) > 0.;
 }
 
-// General boxes run FP64 predicates (the FP32 filter's bounds are for
-// rectangular cells).
-static bool any_general(const gdt_context* c)
-{
-    for (const auto& s : c->sets)
-        if (s.general) return true;
-    return false;
-}
 // (general boxes run FP64; the exact mode reports them as ERR_RANGE)
 static int eff_precision(const gdt_context* c, int precision)
 {
@@ -634,16 +640,44 @@ int gdt_celllist_export(gdt_context* c, unsigned int* d_cell_sizes, int* d_idxs,
     return GDT_OK;
 }
 
-static int finish_rings(gdt_context* c, int stride, int* required, hipStream_t s)
+// The status of a call whose deferred points were launched with `rest`: those
+// that wait for the count are done, and the status read again.  Lists that wait
+// whole (the exact mode's) go one lane each, whole lattices by the per-point
+// kernel in cell order, sets uniform to a block, beyond the length that the list
+// kernel runs at full registers.
+static int read_rings(gdt_context* c, int precision, int rest, const GdtRingIO& io, int* d_counts,
+                      hipStream_t s)
 {
-    int rc = read_status(c, s);
+    const int nsets = (int)c->sets.size(), cap = gdt_wave_cap(precision);
+    const int rc = read_status(c, s);
+    const int len = c->h_status[ST_NDEFER];
+    if (rc != GDT_OK || len <= cap || rest == GDT_REST_HERE || rest > 0) return rc;
+    if (precision == GDT_PREC_EXACT && len == c->total_n && len > GDT_XLIST_SHORT) {
+        GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, nsets, c->rch.p, c->nrch, c->cfg.block,
+                                      nullptr, nullptr, 0, 0, io, d_counts, c->status.p,
+                                      c->counters.p, nullptr, s));
+    } else if (precision == GDT_PREC_EXACT) {
+        GDT_CHECK(gdt_launch_deferred_rest(precision, c->d_sets.p, nsets, 0, len, io, d_counts,
+                                           c->status.p, c->counters.p, c->defer.p, s));
+    } else {
+        GDT_CHECK(gdt_launch_deferred_rest(precision, c->d_sets.p, nsets, cap, len, io, d_counts,
+                                           c->status.p, c->counters.p, c->defer.p, s));
+    }
+    if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
+    return read_status(c, s);
+}
+
+static int finish_rings(gdt_context* c, int precision, int rest, const GdtRingIO& io, int* d_counts,
+                        int* required, hipStream_t s)
+{
+    int rc = read_rings(c, precision, rest, io, d_counts, s);
     if (rc != GDT_OK) return rc;
     record_ring_stats(c);
     const int req = c->h_status[ST_REQUIRED];
     if (required) *required = req;
     rc = status_from_flags(c->h_status[ST_ERRFLAGS]);
     if (rc != GDT_OK) return rc;
-    return req > stride ? GDT_OVERFLOW : GDT_OK;
+    return req > io.stride ? GDT_OVERFLOW : GDT_OK;
 }
 
 static bool tiled_sets(const gdt_context* c)
@@ -660,6 +694,8 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
     if ((rc = ring_chunks(c)) != GDT_OK) return rc;
     if ((rc = build_cells(c, d_xy, s, true)) != GDT_OK) return rc;
     const bool general = any_general(c);
+    const GdtRingIO io = ring_io(c, d_nbrs, stride);
+    const int rest = rest_of_deferred(c, precision);
     // (the exact mode refuses general boxes point by point, in the per-point kernel)
     if (tiled_sets(c) && !(general && precision == GDT_PREC_EXACT)) {
         // A grid of at most one tile per CU runs one wave of blocks: each lane
@@ -681,8 +717,8 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
             nsplit = std::min(nsplit, std::max(1, 4 * c->num_cu / c->ntch));
             GDT_CHECK(gdt_tiles::one_ring_star(ts, precision, c->d_sets.p, (int)c->sets.size(), c->tch.p,
                                                c->ntch, nsplit, block, general,
-                                               ring_io(c, d_nbrs, stride), d_counts, c->status.p,
-                                               c->counters.p, c->defer.p, many_deferred(c),
+                                               io, d_counts, c->status.p,
+                                               c->counters.p, c->defer.p, rest,
                                                c->cfg.profile ? c->ev[2] : nullptr, s));
         } else {
             const bool dense = dense_windows(c);
@@ -692,15 +728,14 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
                 c->ntch <= c->num_cu ? std::max(tile_block(c), one_each) : tile_block(c);
             GDT_CHECK(gdt_tiles::one_ring(ts, precision, c->d_sets.p, (int)c->sets.size(),
                                           c->tch.p, c->ntch, block, lanes, general, nullptr,
-                                          nullptr, ring_io(c, d_nbrs, stride),
+                                          nullptr, io,
                                           d_counts, c->status.p, c->counters.p, c->defer.p,
-                                          dense, many_deferred(c),
+                                          dense, rest,
                                           c->cfg.profile ? c->ev[2] : nullptr, s));
         }
     } else {
         c->stats.tile_shift = 0;
         c->stats.lanes = 1;
-        const GdtRingIO io = ring_io(c, d_nbrs, stride);
         // (the exact mode hands no point on: one beyond the search radius is an error)
         const bool exact = precision == GDT_PREC_EXACT;
         GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), c->rch.p, c->nrch,
@@ -709,10 +744,10 @@ static int triangulate_sets(gdt_context* c, const double* d_xy, int stride, int*
         if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[2], s));
         if (!exact)
             GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
-                                          c->status.p, c->counters.p, c->defer.p, 0, s));
+                                          c->status.p, c->counters.p, c->defer.p, rest, s));
     }
     if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
-    rc = finish_rings(c, stride, required, s);
+    rc = finish_rings(c, precision, rest, io, d_counts, required, s);
     if (c->cfg.profile) {
         // The status words reach the host before the runtime need have seen
         // the events complete (an elapsed time read then is "not ready"): wait
@@ -876,8 +911,9 @@ int gdt_test_circumcircles(gdt_context* c, const double* d_xy, int n, const int*
 // any exit before staging), else the flags compacted (slot order) and one
 // lane each.  status[ST_NDEFER] and status[ST_NFLAGGED] must be zero on entry
 // (reset_status).
-static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* d_nbrs,
-                          int* d_counts, int precision, hipStream_t s)
+// (rest: rest_of_deferred's)
+static int repair_flagged(gdt_context* c, const int* d_repair, const GdtRingIO& io, int* d_counts,
+                          int precision, int rest, hipStream_t s)
 {
     const bool exact = precision == GDT_PREC_EXACT;
     if (tiled_sets(c) && !exact) {
@@ -885,8 +921,8 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
                                       (int)c->sets.size(), c->tch.p, c->ntch, tile_block(c),
                                       repair_lanes_for(c),
                                       any_general(c), d_repair, c->halt,
-                                      ring_io(c, d_nbrs, stride), d_counts, c->status.p,
-                                      c->counters.p, c->defer.p, dense_windows(c), many_deferred(c),
+                                      io, d_counts, c->status.p,
+                                      c->counters.p, c->defer.p, dense_windows(c), rest,
                                       nullptr, s));
         return GDT_OK;
     }
@@ -897,14 +933,13 @@ static int repair_flagged(gdt_context* c, const int* d_repair, int stride, int* 
     uint32_t* worklen = reinterpret_cast<uint32_t*>(c->status.p + ST_NFLAGGED);
     GDT_CHECK(gdt_launch_compact(d_repair, c->perm.p, c->total_n, c->mark.p, c->markscan.p,
                                  c->worklist.p, worklen, c->scan_tmp.p, c->halt, s));
-    const GdtRingIO io = ring_io(c, d_nbrs, stride);
     GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, (int)c->sets.size(), nullptr, 0,
                                   c->cfg.block, c->worklist.p, worklen, 0, c->total_n, io,
                                   d_counts, c->status.p, c->counters.p,
                                   exact ? nullptr : c->defer.p, s));
     if (!exact)
         GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, (int)c->sets.size(), io, d_counts,
-                                      c->status.p, c->counters.p, c->defer.p, 0, s));
+                                      c->status.p, c->counters.p, c->defer.p, rest, s));
     return GDT_OK;
 }
 
@@ -919,8 +954,10 @@ int gdt_repair(gdt_context* c, const double* d_xy, int n, const int* d_repair, i
     precision = eff_precision(c, precision);
     int rc = reset_status(c, s);
     if (rc != GDT_OK) return rc;
-    if ((rc = repair_flagged(c, d_repair, stride, d_nbrs, d_counts, precision, s)) != GDT_OK) return rc;
-    rc = finish_rings(c, stride, required, s);
+    const GdtRingIO io = ring_io(c, d_nbrs, stride);
+    const int rest = rest_of_deferred(c, precision);
+    if ((rc = repair_flagged(c, d_repair, io, d_counts, precision, rest, s)) != GDT_OK) return rc;
+    rc = finish_rings(c, precision, rest, io, d_counts, required, s);
     c->stats.flagged = c->h_status[ST_NFLAGGED];
     return rc;
 }
@@ -942,10 +979,12 @@ static int test_and_repair_sets(gdt_context* c, const double* d_xy, int stride, 
     // 3. their empty-circle test (testTriangulation, DelaunayGPU.cpp:607-648)
     if ((rc = triangles_and_test(c, d_xy, d_nbrs, d_counts, stride, cap, s)) != GDT_OK) return rc;
     // 4. repair the flagged points (locallyRepairDelaunayTriangulation, DelaunayGPU.cpp:87-115)
-    if ((rc = repair_flagged(c, c->repair.p, stride, d_nbrs, d_counts, precision, s)) != GDT_OK) return rc;
+    const GdtRingIO io = ring_io(c, d_nbrs, stride);
+    const int rest = rest_of_deferred(c, precision);
+    if ((rc = repair_flagged(c, c->repair.p, io, d_counts, precision, rest, s)) != GDT_OK) return rc;
     if (!test_in_tiles(c))
         GDT_CHECK(gdt_copy_u32(tested_triangles(c), reinterpret_cast<uint32_t*>(c->status.p + ST_NTRI), s));
-    if ((rc = read_status(c, s)) != GDT_OK) return rc;
+    if ((rc = read_rings(c, precision, rest, io, d_counts, s)) != GDT_OK) return rc;
     const unsigned int h_nt = (unsigned int)c->h_status[ST_NTRI];
     const int nf = c->h_status[ST_NFLAGGED];
     if (nflagged) *nflagged = nf;
@@ -1019,7 +1058,9 @@ static int md_enqueue_step_halting(gdt_context* c, double* d_xy, int stride, int
     GDT_CHECK(gdt_launch_md_displace(c->d_sets.p, c->pch.p, c->npch, d_xy, sigma, seed, c->md.p, s));
     if ((rc = build_cells(c, d_xy, s, true, c->repair.p)) != GDT_OK) return rc;
     if ((rc = triangles_and_test(c, d_xy, d_nbrs, d_counts, stride, cap, s)) != GDT_OK) return rc;
-    if ((rc = repair_flagged(c, c->repair.p, stride, d_nbrs, d_counts, precision, s)) != GDT_OK) return rc;
+    if ((rc = repair_flagged(c, c->repair.p, ring_io(c, d_nbrs, stride), d_counts, precision,
+                             rest_of_deferred(c, precision), s)) != GDT_OK)
+        return rc;
     GDT_CHECK(gdt_launch_md_step_end(c->status.p, c->counters.p, tested_triangles(c), n, stride, c->md.p, s));
     return GDT_OK;
 }

@@ -80,13 +80,16 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
                                unsigned long long* counters, int* defer, hipStream_t s);
 
 // Deferred points: the first GDT_WAVE_CAP one wavefront each (GDT_WAVE_BLOCKS
-// blocks of 256 threads), the rest one lane each, in one launch.
+// blocks of 256 threads), the rest one lane each.
 #define GDT_WAVE_CAP 8192
 // The exact mode's lists up to this length take a wavefront per point, longer
 // ones a lane per point: wavefronts take about 0.45 us a point together, the lanes
 // 1.7 ms for their longest chain however many there are (lattices of exact ties,
 // 65,536 points: 4.6 ms per call with wavefronts first, 1.7 with lanes).
 #define GDT_WAVE_CAP_EXACT 3072
+// Exact lists up to this length (two waves to each SIMD) run with all of the
+// routine's registers, longer ones with the waves that fewer registers allow.
+#define GDT_XLIST_SHORT 131072
 #define GDT_WAVE_BLOCKS 512
 // Threads per block (at most) of the exact mode's tile and star kernels: two
 // waves per SIMD, so that the double-double decisions keep 256 registers.
@@ -101,12 +104,36 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
 #define GDT_TILE_DEFER 64
 
 // Deferred points of the tile kernel (defer[0..status[ST_NDEFER]), count read
-// on the device): a wavefront each, then one lane each beyond GDT_WAVE_CAP.
-// many: 0, or, where more than that is expected, the most that can be.
+// on the device): a wavefront each up to the cap above, the rest one lane each:
+//   rest > 0            by a launch behind, of at most `rest` points (a long
+//                       list is expected);
+//   GDT_REST_LATER      by gdt_launch_deferred_rest, once the caller has read a
+//                       count beyond the cap;
+//   GDT_REST_HERE       in the same launch (a caller that reads no count on
+//                       the host);
+// or GDT_LIST_LATER (the exact mode, always): a list beyond the cap waits whole
+// for the caller.
+// As a kernel of its own behind every call the rest costs 4.7 us where there
+// is nearly always none; in the wavefronts' launch, beside their registers and in
+// their 512 blocks, it takes longer than its own kernel where there is one (2^20
+// points, half of them in 20 clumps: 46 ms per call, GDT_REST_LATER 28; 2^20
+// points of an exact lattice in the exact mode 14.4 and 10.7).
+#define GDT_REST_HERE 0
+#define GDT_REST_LATER (-1)
+#define GDT_LIST_LATER (-2)
+inline int gdt_wave_cap(int precision)
+{
+    return precision == GDT_EXACT ? GDT_WAVE_CAP_EXACT : GDT_WAVE_CAP;
+}
 hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
-                               unsigned long long* counters, int* defer, int many,
+                               unsigned long long* counters, int* defer, int rest,
                                hipStream_t s);
+// One lane each: entries [first, len) of such a list (gdt_launch_deferred took
+// the others).
+hipError_t gdt_launch_deferred_rest(int precision, const GdtSet* d_sets, int nsets, int first,
+                                    int len, const GdtRingIO& io, int* counts, int* status,
+                                    unsigned long long* counters, const int* defer, hipStream_t s);
 
 // The LDS-window kernels, compiled once per tile edge into namespaces ts4
 // (16x16-cell tiles) and ts5 (32x32); gdt_tiles::* picks by the sets' shift.
@@ -126,13 +153,13 @@ hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                         bool general,                                            \
                                         const int* flags, const int* halt,                       \
                                         const GdtRingIO& io, int* counts, int* status,           \
-                                        unsigned long long* counters, int* defer, int many,      \
+                                        unsigned long long* counters, int* defer, int rest,      \
                                         hipEvent_t after_tile, hipStream_t s);                   \
     hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nsets,          \
                                         const GdtChunk* tiles,                                   \
                                         int ntiles, int nsplit, int block, bool general,         \
                                         const GdtRingIO& io, int* counts, int* status,           \
-                                        unsigned long long* counters, int* defer, int many,      \
+                                        unsigned long long* counters, int* defer, int rest,      \
                                         hipEvent_t after_tile, hipStream_t s);                   \
     hipError_t gdt_launch_ring_test_tile(const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,\
                                          const int* nbrs, const int* counts, int stride,         \
@@ -187,7 +214,7 @@ namespace gdt_tiles {
 inline hipError_t one_ring(int tshift, int precision, const GdtSet* d_sets, int nsets,
                            const GdtChunk* tiles, int ntiles, int block, int lanes, bool general,
                            const int* flags, const int* halt, const GdtRingIO& io, int* counts, int* status,
-                           unsigned long long* counters, int* defer, bool dense, int many,
+                           unsigned long long* counters, int* defer, bool dense, int rest,
                            hipEvent_t after_tile, hipStream_t s)
 {
     // (rows do not depend on the windows; 32x32-cell tiles have fuller ones)
@@ -195,18 +222,18 @@ inline hipError_t one_ring(int tshift, int precision, const GdtSet* d_sets, int 
             : dense     ? ts5d::gdt_launch_one_ring_tile
                         : ts5::gdt_launch_one_ring_tile)(
         precision, d_sets, nsets, tiles, ntiles, block, lanes, general, flags, halt,
-        io, counts, status, counters, defer, many, after_tile, s);
+        io, counts, status, counters, defer, rest, after_tile, s);
 }
 inline hipError_t one_ring_star(int tshift, int precision, const GdtSet* d_sets, int nsets,
                                 const GdtChunk* tiles, int ntiles, int nsplit, int block,
                                 bool general, const GdtRingIO& io, int* counts, int* status,
-                                unsigned long long* counters, int* defer, int many,
+                                unsigned long long* counters, int* defer, int rest,
                                 hipEvent_t after_tile,
                                 hipStream_t s)
 {
     return (tshift == 4 ? ts4::gdt_launch_one_ring_star : ts5::gdt_launch_one_ring_star)(
         precision, d_sets, nsets, tiles, ntiles, nsplit, block, general, io, counts, status, counters, defer,
-        many, after_tile, s);
+        rest, after_tile, s);
 }
 inline hipError_t ring_test(int tshift, const GdtSet* d_sets, const GdtChunk* tiles, int ntiles,
                             const int* nbrs, const int* counts, int stride, int total_n,

@@ -163,14 +163,23 @@ extern "C" int gdt_triangulate_noalloc(const double* d_xy, int n, double lx, dou
     // (fuller windows; those that overflow all the same hand nearly every point on)
     const double window = 1600. * n / ((double)S.xsize * S.ysize);
     const bool dense = window > GDT_DENSE_WINDOW;
-    const int many = window > 4000. ? n : 0;
+    const int rest = window > 4000. ? n : GDT_REST_LATER;
     if (gdt_tiles::one_ring(GDT_TILE_SHIFT, precision, d_sets, 1, d_tiles, ntiles, block, 1, false,
                             nullptr, nullptr, io, d_counts, status, counters,
-                            reinterpret_cast<int*>(base + L.defer), dense, many, nullptr, s) != hipSuccess)
+                            reinterpret_cast<int*>(base + L.defer), dense, rest, nullptr, s) != hipSuccess)
         return GDT_ERR_DEVICE;
     int h_status[ST_WORDS];
-    if (hipMemcpyAsync(h_status, status, sizeof(h_status), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
+    auto read = [&]() {
+        return hipMemcpyAsync(h_status, status, sizeof(h_status), hipMemcpyDeviceToHost, s) ==
+                   hipSuccess &&
+               hipStreamSynchronize(s) == hipSuccess;
+    };
+    if (!read()) return GDT_ERR_DEVICE;
+    if (rest == GDT_REST_LATER && h_status[ST_NDEFER] > gdt_wave_cap(precision) &&
+        (gdt_launch_deferred_rest(precision, d_sets, 1, gdt_wave_cap(precision), h_status[ST_NDEFER], io,
+                                  d_counts, status, counters, reinterpret_cast<const int*>(base + L.defer),
+                                  s) != hipSuccess ||
+         !read()))
         return GDT_ERR_DEVICE;
     const int req = h_status[ST_REQUIRED];
     if (required) *required = req;

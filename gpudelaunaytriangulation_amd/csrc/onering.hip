@@ -70,8 +70,8 @@ __global__ __launch_bounds__(1024) void k_one_ring(const GdtSet* __restrict__ se
 }
 
 // Entries [first, len) of a slot list, one lane each over the grid, set found
-// per lane.
-template <int PREC>
+// per lane (ONE: a single set, which then stays in scalar registers).
+template <int PREC, bool ONE = false>
 __device__ inline void one_ring_lanes(const GdtSet* __restrict__ sets, int nsets,
                                       const int* __restrict__ worklist, int first, int len,
                                       const GdtRingIO& io, int* __restrict__ counts,
@@ -85,19 +85,19 @@ __device__ inline void one_ring_lanes(const GdtSet* __restrict__ sets, int nsets
     for (int base = wave_first; base < len; base += stride) {
         const int t = base + (int)(threadIdx.x & 63);
         const bool active = t < len;
-        int j = 0, s = 0;
-        if (active) {
-            j = worklist[t];
-            s = gdt_set_of(sets, nsets, j);
-        }
-        const GdtSet S = sets[s];
+        const int j = active ? worklist[t] : 0;
+        const GdtSet S = sets[ONE || !active ? 0 : gdt_set_of(sets, nsets, j)];
         one_ring_lane<PREC>(active, S, j, io, counts, status, counters, defer);
     }
 }
 
 // Entries from `first` of a worklist of slots (count in device memory), one lane each.
-template <int PREC>
-__global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict__ sets, int nsets,
+// ONE: a single set (FP64: 68 registers and seven waves to a SIMD, 94 and five
+// with a set per lane).  THREADS: the largest block; at 256 the exact routine
+// keeps its registers, at 1,024 it spills some for twice the waves
+// (GDT_XLIST_SHORT).
+template <int PREC, bool ONE, int THREADS = 1024>
+__global__ __launch_bounds__(THREADS) void k_one_ring_list(const GdtSet* __restrict__ sets, int nsets,
                                                         const int* __restrict__ worklist,
                                                         const uint32_t* __restrict__ worklen,
                                                         GdtRingIO io, int* __restrict__ counts,
@@ -105,18 +105,14 @@ __global__ __launch_bounds__(1024) void k_one_ring_list(const GdtSet* __restrict
                                                         unsigned long long* __restrict__ counters,
                                                         int* __restrict__ defer, int first)
 {
-    one_ring_lanes<PREC>(sets, nsets, worklist, first, (int)*worklen, io, counts, status, counters,
+    one_ring_lanes<PREC, ONE>(sets, nsets, worklist, first, (int)*worklen, io, counts, status, counters,
                          defer);
 }
 
 // Deferred points (count in device memory): the first `cap` one wavefront
 // each, grid-stride over the waves (FP64 in both precision paths; exact
-// decisions in the exact mode), any beyond (dense clusters, exact lattices)
-// one lane each.  One launch for both: the second part is nearly always
-// empty, and as a kernel of its own cost its launch, 4.7 us of every call.
-// Where the caller expects a long list (waves_only), the second part is
-// k_one_ring_list: with the wavefront routine's registers beside it, it took
-// 2.9 ms for 600,000 points of 1.44 to a cell, where that takes 1.9.
+// decisions in the exact mode), and, where `rest` says so, any beyond (dense
+// clusters) one lane each; GDT_LIST_LATER: none of a longer list.
 template <int PREC>
 __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restrict__ sets,
                                                            int nsets,
@@ -126,14 +122,13 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
                                                            int* __restrict__ counts,
                                                            int* __restrict__ status,
                                                            unsigned long long* __restrict__ counters,
-                                                           int waves_only)
+                                                           int rest)
 {
     const int lane = (int)(threadIdx.x & 63);
     const int wid = (int)((blockIdx.x * blockDim.x + threadIdx.x) >> 6);
     const int nw = (int)((gridDim.x * blockDim.x) >> 6);
     const int all = (int)*worklen;
-    // (the exact mode takes a longer list one lane each from its start)
-    const int len = PREC == GDT_EXACT && all > cap ? 0 : min(all, cap);
+    const int len = rest == GDT_LIST_LATER && all > cap ? 0 : min(all, cap);
     GdtWaveDev w;
     w.lane = lane;
     unsigned npred = 0, nsum = 0;
@@ -166,33 +161,44 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
             if (nsum) atomicAdd(&counters[CT_NBRSUM], (unsigned long long)nsum);
         }
     }
-    if (all > cap && !waves_only)
-        one_ring_lanes<PREC>(sets, nsets, worklist, len, all, io, counts, status, counters,
-                             nullptr);
+    if constexpr (PREC != GDT_EXACT) {
+        if (rest == GDT_REST_HERE)
+            one_ring_lanes<PREC>(sets, nsets, worklist, len, all, io, counts, status, counters,
+                                 nullptr);
+    }
 }
 
 hipError_t gdt_launch_deferred(int precision, const GdtSet* d_sets, int nsets,
                                const GdtRingIO& io, int* counts, int* status,
-                               unsigned long long* counters, int* defer, int many, hipStream_t s)
+                               unsigned long long* counters, int* defer, int rest, hipStream_t s)
 {
+    if (precision == GDT_EXACT && rest != GDT_LIST_LATER) return hipErrorInvalidValue;
+    const int cap = gdt_wave_cap(precision);
     // (the count is read on the device)
     const uint32_t* ndefer = reinterpret_cast<const uint32_t*>(status + ST_NDEFER);
     if (precision == 32)
         hipLaunchKernelGGL(k_one_ring_deferred<32>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
-                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
-                           many);
+                           nsets, defer, ndefer, cap, io, counts, status, counters, rest);
     else if (precision == GDT_EXACT)
         hipLaunchKernelGGL(k_one_ring_deferred<GDT_EXACT>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s,
-                           d_sets, nsets, defer, ndefer, GDT_WAVE_CAP_EXACT, io, counts, status,
-                           counters, 0);
+                           d_sets, nsets, defer, ndefer, cap, io, counts, status, counters,
+                           rest);
     else
         hipLaunchKernelGGL(k_one_ring_deferred<64>, dim3(GDT_WAVE_BLOCKS), dim3(256), 0, s, d_sets,
-                           nsets, defer, ndefer, GDT_WAVE_CAP, io, counts, status, counters,
-                           many);
+                           nsets, defer, ndefer, cap, io, counts, status, counters, rest);
     const hipError_t e = hipGetLastError();
-    if (e != hipSuccess || !many || precision == GDT_EXACT) return e;
-    return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer, ndefer,
-                               GDT_WAVE_CAP, many, io, counts, status, counters, nullptr, s);
+    if (e != hipSuccess || rest <= 0) return e;
+    return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer, ndefer, cap, rest,
+                               io, counts, status, counters, nullptr, s);
+}
+
+hipError_t gdt_launch_deferred_rest(int precision, const GdtSet* d_sets, int nsets, int first,
+                                    int len, const GdtRingIO& io, int* counts, int* status,
+                                    unsigned long long* counters, const int* defer, hipStream_t s)
+{
+    return gdt_launch_one_ring(precision, d_sets, nsets, nullptr, 0, 256, defer,
+                               reinterpret_cast<const uint32_t*>(status + ST_NDEFER), first, len, io,
+                               counts, status, counters, nullptr, s);
 }
 
 hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
@@ -218,14 +224,15 @@ hipError_t gdt_launch_one_ring(int precision, const GdtSet* d_sets, int nsets,
     if (max_work <= 0) return hipSuccess;
     int grid = (max_work + block - 1) / block;
     if (grid > 4096) grid = 4096;
+    const bool one = nsets == 1;
+    auto* k = one ? k_one_ring_list<64, true> : k_one_ring_list<64, false>;
     if (precision == 32)
-        hipLaunchKernelGGL(k_one_ring_list<32>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, io, counts, status, counters, defer, first);
+        k = one ? k_one_ring_list<32, true> : k_one_ring_list<32, false>;
+    else if (precision == GDT_EXACT && block <= 256 && max_work <= GDT_XLIST_SHORT)
+        k = one ? k_one_ring_list<GDT_EXACT, true, 256> : k_one_ring_list<GDT_EXACT, false, 256>;
     else if (precision == GDT_EXACT)
-        hipLaunchKernelGGL(k_one_ring_list<GDT_EXACT>, dim3(grid), dim3(block), 0, s, d_sets,
-                           nsets, worklist, worklen, io, counts, status, counters, defer, first);
-    else
-        hipLaunchKernelGGL(k_one_ring_list<64>, dim3(grid), dim3(block), 0, s, d_sets, nsets,
-                           worklist, worklen, io, counts, status, counters, defer, first);
+        k = one ? k_one_ring_list<GDT_EXACT, true> : k_one_ring_list<GDT_EXACT, false>;
+    hipLaunchKernelGGL(k, dim3(grid), dim3(block), 0, s, d_sets, nsets, worklist, worklen, io, counts,
+                       status, counters, defer, first);
     return hipGetLastError();
 }

@@ -749,7 +749,7 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
                                     bool general,
                                     const int* flags, const int* halt,
                                     const GdtRingIO& io, int* counts, int* status,
-                                    unsigned long long* counters, int* defer, int many,
+                                    unsigned long long* counters, int* defer, int rest,
                                     hipEvent_t after_tile, hipStream_t s)
 {
     if (ntiles <= 0) return hipSuccess;
@@ -792,7 +792,7 @@ hipError_t gdt_launch_one_ring_tile(int precision, const GdtSet* d_sets, int nse
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
     return gdt_launch_deferred(precision, d_sets, nsets, io, counts, status, counters,
-                               defer, many, s);
+                               defer, rest, s);
 }
 
 #ifndef GDT_WIN_DENSE
@@ -800,7 +800,7 @@ hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nse
                                     const GdtChunk* tiles,
                                     int ntiles, int nsplit, int block, bool general,
                                     const GdtRingIO& io, int* counts, int* status,
-                                    unsigned long long* counters, int* defer, int many,
+                                    unsigned long long* counters, int* defer, int rest,
                                     hipEvent_t after_tile, hipStream_t s)
 {
     if (ntiles <= 0) return hipSuccess;
@@ -822,7 +822,7 @@ hipError_t gdt_launch_one_ring_star(int precision, const GdtSet* d_sets, int nse
     if (e != hipSuccess) return e;
     if (after_tile && (e = hipEventRecord(after_tile, s)) != hipSuccess) return e;
     return gdt_launch_deferred(precision == GDT_EXACT ? GDT_EXACT : 64, d_sets, nsets, io, counts,
-                               status, counters, defer, many, s);
+                               status, counters, defer, rest, s);
 }
 #endif
 
