@@ -250,6 +250,7 @@ static int rest_of_deferred(const gdt_context* c, int precision)
 {
     const bool tiled = c->sets[0].tiled;
     if (precision == GDT_PREC_EXACT) return GDT_LIST_LATER;
+    if (!c->halt && tiled && any_general(c)) return GDT_LIST_LATER;
     const int ts = c->sets[0].tshift;
     if (tiled && window_points(c->sets, ts) > (ts == 4 ? 1000. : 4000.)) return c->total_n;
     return c->halt ? GDT_REST_HERE : GDT_REST_LATER;
@@ -364,6 +365,8 @@ static std::vector<GdtSet> sets_of(const gdt_context* c, int nsets, const int* o
     }
     const int ts = tile_shift_for(c, sets);
     if (ts != GDT_TSHIFT_MAX) make(c->cfg.tiled, ts);
+    if (general && c->cfg.tiled && ts == GDT_TSHIFT_MIN && window_points(sets, ts) > 1000.)
+        make(0, GDT_TSHIFT_MAX);
     return sets;
 }
 
@@ -441,7 +444,8 @@ static void record_ring_stats(gdt_context* c)
     c->stats.fallbacks = c->h_counters[CT_FALLBACK];
     c->stats.neighbours = c->h_counters[CT_NBRSUM];
     c->stats.max_ring = c->h_status[ST_REQUIRED];
-    c->stats.deferred = c->h_status[ST_NDEFER] + c->h_status[ST_NDEFER_TILE];
+    c->stats.deferred = c->h_status[ST_NDEFER] + c->h_status[ST_NDEFER_TILE] +
+                        c->h_status[ST_NLISTED];
     if (!c->sets.empty()) {
         c->stats.xsize = c->sets[0].xsize;
         c->stats.ysize = c->sets[0].ysize;
@@ -642,15 +646,20 @@ int gdt_celllist_export(gdt_context* c, unsigned int* d_cell_sizes, int* d_idxs,
 
 // The status of a call whose deferred points were launched with `rest`: those
 // that wait for the count are done, and the status read again.  Lists that wait
-// whole (the exact mode's) go one lane each, whole lattices by the per-point
-// kernel in cell order, sets uniform to a block, beyond the length that the list
-// kernel runs at full registers.
+// whole go one lane each.  In general boxes these are the points of windows
+// that overflow, and those whose circles the search radius does not certify go
+// on to the wavefronts, as everywhere a general box runs the per-point kernel
+// (262,144 points in a sheared box, half of them in 20 clumps: 7.0 ms with the
+// list's first points to wavefronts).  The exact mode's whole lattices take the
+// per-point kernel in cell order, sets uniform to a block, beyond the length
+// that the list kernel runs at full registers.
 static int read_rings(gdt_context* c, int precision, int rest, const GdtRingIO& io, int* d_counts,
                       hipStream_t s)
 {
     const int nsets = (int)c->sets.size(), cap = gdt_wave_cap(precision);
-    const int rc = read_status(c, s);
-    const int len = c->h_status[ST_NDEFER];
+    int rc = read_status(c, s);
+    int len = c->h_status[ST_NDEFER];
+    const int* list = c->defer.p;
     if (rc != GDT_OK || len <= cap || rest == GDT_REST_HERE || rest > 0) return rc;
     if (precision == GDT_PREC_EXACT && len == c->total_n && len > GDT_XLIST_SHORT) {
         GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, nsets, c->rch.p, c->nrch, c->cfg.block,
@@ -658,10 +667,26 @@ static int read_rings(gdt_context* c, int precision, int rest, const GdtRingIO& 
                                       c->counters.p, nullptr, s));
     } else if (precision == GDT_PREC_EXACT) {
         GDT_CHECK(gdt_launch_deferred_rest(precision, c->d_sets.p, nsets, 0, len, io, d_counts,
-                                           c->status.p, c->counters.p, c->defer.p, s));
+                                           c->status.p, c->counters.p, list, s));
     } else {
+        if (rest == GDT_LIST_LATER) {
+            uint32_t* n = reinterpret_cast<uint32_t*>(c->status.p);
+            GDT_CHECK(c->worklist.reserve((size_t)c->total_n));
+            GDT_CHECK(gdt_copy_u32(n + ST_NDEFER, n + ST_NLISTED, s));
+            GDT_CHECK(gdt_fill_u32(n + ST_NDEFER, 0u, 1, s));
+            GDT_CHECK(gdt_launch_one_ring(precision, c->d_sets.p, nsets, nullptr, 0, 256, list,
+                                          n + ST_NLISTED, 0, len, io, d_counts, c->status.p,
+                                          c->counters.p, c->worklist.p, s));
+            list = c->worklist.p;
+            GDT_CHECK(gdt_launch_deferred(precision, c->d_sets.p, nsets, io, d_counts, c->status.p,
+                                          c->counters.p, c->worklist.p, GDT_REST_LATER, s));
+            if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
+            rc = read_status(c, s);
+            len = c->h_status[ST_NDEFER];
+            if (rc != GDT_OK || len <= cap) return rc;
+        }
         GDT_CHECK(gdt_launch_deferred_rest(precision, c->d_sets.p, nsets, cap, len, io, d_counts,
-                                           c->status.p, c->counters.p, c->defer.p, s));
+                                           c->status.p, c->counters.p, list, s));
     }
     if (c->cfg.profile) GDT_CHECK(hipEventRecord(c->ev[3], s));
     return read_status(c, s);

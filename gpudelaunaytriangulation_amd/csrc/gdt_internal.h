@@ -46,6 +46,7 @@ enum {
     ST_NTRI = 3,         // number of triangles enumerated
     ST_NDEFER = 4,       // points deferred to the wavefront kernel (tile or per-point kernels)
     ST_NDEFER_TILE = 5,  // deferred points a tile block finished itself with a wavefront
+    ST_NLISTED = 6,      // deferred points that went one lane each before the wavefronts
     ST_WORDS = 8
 };
 // ERR_DEFER is internal: the LDS routine hands the point to the direct routine.

@@ -14,31 +14,17 @@
 
 #include <type_traits>
 
-// A point whose search the grid's search radius cannot certify (boxes of a
-// few cells) is appended to `defer` (when given) for the wavefront kernel,
-// whose searches may stop at the cell box of their circle; its row is then
-// rewritten there.
 template <int PREC>
-__device__ inline void one_ring_lane(bool active, const GdtSet& S, int j, const GdtRingIO& io,
-                                     int* __restrict__ counts, int* __restrict__ status,
-                                     unsigned long long* __restrict__ counters,
-                                     int* __restrict__ defer)
+__device__ inline GdtRingResult ring_of(const GdtSet& S, int j, const GdtRingIO& io)
 {
-    GdtRingResult r = {0, 0, 0u, 0u};
-    if (active) {
-        if constexpr (PREC == GDT_EXACT)
-            r = gdt_one_ring_exact(S, j, io);
-        else
-            r = (PREC == 32) ? gdt_one_ring_f32(S, j, io) : gdt_one_ring_f64(S, j, io);
-        if (defer && (r.err & ERR_SEARCH)) {
-            defer[atomicAdd(reinterpret_cast<unsigned*>(status + ST_NDEFER), 1u)] = j;
-            r.count = 0;
-            r.err = 0;
-        } else {
-            counts[io.perm[j]] = r.count;
-        }
-    }
-    // every lane of the wave reaches the reductions below
+    if constexpr (PREC == GDT_EXACT) return gdt_one_ring_exact(S, j, io);
+    else return PREC == 32 ? gdt_one_ring_f32(S, j, io) : gdt_one_ring_f64(S, j, io);
+}
+
+// The totals of a wave's results (every lane of the wave calls it).
+__device__ inline void ring_wave_totals(bool active, const GdtRingResult& r, int* __restrict__ status,
+                                        unsigned long long* __restrict__ counters)
+{
     const int mx = wave_max_i32(r.count);
     const int er = wave_or_i32(r.err);
     const unsigned np = wave_sum_u32(r.npred);
@@ -51,6 +37,30 @@ __device__ inline void one_ring_lane(bool active, const GdtSet& S, int j, const 
         if (nf) atomicAdd(&counters[CT_FALLBACK], (unsigned long long)nf);
         if (ns) atomicAdd(&counters[CT_NBRSUM], (unsigned long long)ns);
     }
+}
+
+// A point whose search the grid's search radius cannot certify (boxes of a
+// few cells) is appended to `defer` (when given) for the wavefront kernel,
+// whose searches may stop at the cell box of their circle; its row is then
+// rewritten there.
+template <int PREC>
+__device__ inline void one_ring_lane(bool active, const GdtSet& S, int j, const GdtRingIO& io,
+                                     int* __restrict__ counts, int* __restrict__ status,
+                                     unsigned long long* __restrict__ counters,
+                                     int* __restrict__ defer)
+{
+    GdtRingResult r = {0, 0, 0u, 0u};
+    if (active) {
+        r = ring_of<PREC>(S, j, io);
+        if (defer && (r.err & ERR_SEARCH)) {
+            defer[atomicAdd(reinterpret_cast<unsigned*>(status + ST_NDEFER), 1u)] = j;
+            r.count = 0;
+            r.err = 0;
+        } else {
+            counts[io.perm[j]] = r.count;
+        }
+    }
+    ring_wave_totals(active, r, status, counters);
 }
 
 // All points: block b handles chunk b (one set, blockDim consecutive slots).
@@ -112,7 +122,8 @@ __global__ __launch_bounds__(THREADS) void k_one_ring_list(const GdtSet* __restr
 // Deferred points (count in device memory): the first `cap` one wavefront
 // each, grid-stride over the waves (FP64 in both precision paths; exact
 // decisions in the exact mode), and, where `rest` says so, any beyond (dense
-// clusters) one lane each; GDT_LIST_LATER: none of a longer list.
+// clusters) one lane each, and again by the wavefront where the lane's search does
+// not certify a circle; GDT_LIST_LATER: none of a longer list.
 template <int PREC>
 __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restrict__ sets,
                                                            int nsets,
@@ -162,9 +173,25 @@ __global__ __launch_bounds__(256) void k_one_ring_deferred(const GdtSet* __restr
         }
     }
     if constexpr (PREC != GDT_EXACT) {
-        if (rest == GDT_REST_HERE)
-            one_ring_lanes<PREC>(sets, nsets, worklist, len, all, io, counts, status, counters,
-                                 nullptr);
+        if (rest != GDT_REST_HERE) return;
+        for (int base = len + 64 * wid; base < all; base += 64 * nw) {      // (wave-uniform)
+            const bool active = base + lane < all;
+            const int j = active ? worklist[base + lane] : 0;
+            GdtRingResult r = {0, 0, 0u, 0u};
+            if (active) r = ring_of<PREC>(sets[gdt_set_of(sets, nsets, j)], j, io);
+            for (unsigned long long m = __ballot((r.err & ERR_SEARCH) != 0); m; m &= m - 1ull) {
+                const int from = __ffsll((long long)m) - 1, jw = __shfl(j, from, 64);
+                const GdtSet S = sets[gdt_set_of(sets, nsets, jw)];
+                const GdtRingResult g = gdt_wave_ring(S, jw, io, w, lane == 0);
+                r.npred += g.npred;
+                if (lane == from) {
+                    r.count = g.count;
+                    r.err = g.err;
+                }
+            }
+            if (active) counts[io.perm[j]] = r.count;
+            ring_wave_totals(active, r, status, counters);
+        }
     }
 }
 

@@ -335,6 +335,9 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
         if (lane >= acc && lane < acc + n) kg = b + lane - acc;
         acc += n;
     }
+    // (a block that holds too many for the lanes: in general boxes, whose clumps
+    // are handed on, lane 0's chain of steps is the slower way)
+    if (GEN && tot > 64) return STEP_DEFER;
     int bk = -1, rc = STEP_DEFER;
     if (tot <= 64 && kg >= 0) {
         GdtTileLane<double> sl = st;
@@ -635,12 +638,25 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
             j = tile_flagged_slot(sf, T0, q);
             lane_init(st, j);
         }
+        // (clumps in a general box are handed on: their steps are long chains, and
+        // its lists go one lane each: 262,144 points, half of them in 200 clumps,
+        // 6.6 ms per call with the steps, 5.0 without)
+        auto full = [&]() {
+            int n = 0;
+            for (int r = -1; r <= 1; ++r) {
+                const uint32_t* row = L.cs + st.c0 + r * GDT_WIN;
+                n += (int)(row[2] - row[-1]);
+            }
+            return n > GDT_HULL_SLOTS;
+        };
         while (__ballot(have) != 0) {
             if (have) {
-                const int rc = gdt_tile_step_f64<1, false, GEN>(S, L, io, st, npred);
+                const bool hand_on = GEN && full();
+                const int rc = hand_on ? STEP_DEFER
+                                       : gdt_tile_step_f64<1, false, GEN>(S, L, io, st, npred);
                 if (rc != STEP_RUN) {
                     if (rc == STEP_DEFER) {
-                        const uint32_t dpos = atomicAdd(&s_dn, 1u);
+                        const uint32_t dpos = hand_on ? GDT_TILE_DEFER : atomicAdd(&s_dn, 1u);
                         if (dpos < GDT_TILE_DEFER) {
                             s_dlist[dpos] = j;
                         } else {

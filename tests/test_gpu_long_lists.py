@@ -1,8 +1,9 @@
 """Long lists of deferred points on the GPU, the rest of which goes one lane
 each: rows equal to the row-major per-point kernel's.  Clumps that no window
-holds (FP64 and FP32-filtered, a repair, the call without allocations) and
-exact lattices just below and above the length that wavefronts take in the exact
-mode."""
+holds (FP64 and FP32-filtered, a repair, the call without allocations), exact
+lattices just below and above the length that wavefronts take in the exact
+mode, and in a sheared box clumps beside a void, where some of the list's points
+have circles that only a wavefront's search certifies."""
 import ctypes
 
 import numpy as np
@@ -18,6 +19,19 @@ from test_gpu_exact_tile import rows as exact_rows  # noqa: E402
 from test_gpu_general_tile import cuda, rows, same  # noqa: E402
 
 WAVE_CAP, WAVE_CAP_EXACT = 8192, 3072      # lists up to these take a wavefront a point
+
+
+def void_in_a_sheared_box():
+    """A square void of 0.49 of the box, in which four circles are certified by
+    a wavefront's search alone, and clumps close to their points."""
+    L = 140.0
+    rng = np.random.default_rng(6)
+    u = rng.random((12000, 2)) * L
+    u = u[~(np.abs(u - L / 2.0) < 0.245 * L).all(1)]
+    near = [(75.9, 32.5), (107.4, 62.4), (107.4, 64.5), (32.6, 80.5)]
+    u = np.concatenate([u] + [np.array(p) + 0.4 * rng.standard_normal((2700, 2)) for p in near])
+    u = u[~(np.abs(u - L / 2.0) < 0.245 * L).all(1)]
+    return np.stack([u[:, 0] + u[:, 1] / 6.0, u[:, 1]], 1), (L, L / 6.0, 0.0, L)
 
 
 def clumps(n, each, k, L, seed):
@@ -93,3 +107,38 @@ def test_exact_lattices_whole(n_side):
     got, gn, st = exact_rows(xy, lx, ly, 0.1)
     assert st["deferred"] == len(xy)
     assert np.array_equal(wn, gn) and np.array_equal(want, got)
+
+
+@pytest.mark.parametrize("config", [{}, {"lanes": 1, "tile_shift": 5}, {"lanes": 2, "tile_shift": 4},
+                                    {"lanes": 64, "tile_shift": 4}], ids=str)
+def test_clumps_beside_a_void_in_a_sheared_box(config):
+    xy, box = void_in_a_sheared_box()
+    print(f"[long lists] void {config}", flush=True)
+    want = rows(xy, xy, box, 1.0, tiled=0)
+    got = rows(xy, xy, box, 1.0, **config)
+    assert got[3]["deferred"] > WAVE_CAP
+    assert same(want[0], got[0]) and int(got[0][1].sum()) == 6 * len(xy)
+
+
+def test_brownian_steps_beside_a_void_in_a_sheared_box():
+    """The loop reads no count on the host: its longer lists go one lane each in
+    the wavefronts' launch, which takes their uncertified points again."""
+    from gpudelaunaytriangulation_amd.delaunay import BatchedDelaunayGPU
+    xy, box = void_in_a_sheared_box()
+    n = len(xy)
+    print("[long lists] void, md", flush=True)
+
+    def go(**config):
+        bd = BatchedDelaunayGPU([n], [box], 24, 1.0)
+        bd.ctx.set_config(**config)
+        pts = cuda(xy)
+        tri = torch.full((n * 24,), -7, dtype=torch.int32, device="cuda")
+        num = torch.zeros(n, dtype=torch.int32, device="cuda")
+        bd.globalDelaunayTriangulation(pts, tri, num)
+        out = bd.md_run(pts, tri, num, 3, 0.02, seed=3)
+        return (tri.cpu().numpy().reshape(n, -1), num.cpu().numpy()), pts.cpu().numpy(), out
+
+    want, wp, wo = go(tiled=0)
+    got, gp, go_ = go()
+    assert go_["max_flagged"] > WAVE_CAP and go_["flagged_total"] == wo["flagged_total"]
+    assert np.array_equal(wp, gp) and same(want, got)
