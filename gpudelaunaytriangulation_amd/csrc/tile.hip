@@ -309,13 +309,45 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
 // uniform scan reads no word beyond its rows; a step's own tables, at most
 // five rows and the word read after them, fit in the first six).
 #define STAR_TBL (2 * GDT_SCAN + 1)
+// Points handed on that a star block keeps for one append (more go one by one).
+#define STAR_HAND 256
+
+// Whether two entries of the lanes' block (one each, kg; half its edge ph) are at the
+// point's smallest distance as far as the exact mode's bounds tell.
+__device__ inline bool star_nn_tie(const GdtSet& S, const GdtTileLds& L, const GdtRingIO& io,
+                                   const GdtTileLane<double>& st, int kg, int ph)
+{
+    const bool here = kg >= 0 && kg != st.iv;
+    const gdt_d2 X = L.X64[here ? kg : st.iv];
+    const double x = X.x - st.vx, y = X.y - st.vy;
+    const double d2 = here ? gdt_dist2_64(x, y) : 1e300;
+    double least = d2;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) least = GDT_FMIN(least, __shfl_xor(least, o, 64));
+    const double Lbox = GDT_FMAX(S.lx, S.ly), M = (double)(ph + 1) * GDT_FMAX(S.bsx, S.bsy);
+    const bool near = here && d2 <= least + 2. * gdt_x_tol2(gdt_x_err(Lbox, M), M);
+    const unsigned long long m = __ballot(near);
+    if (m == 0ull || (m & (m - 1ull)) == 0ull) return false;
+    // (against the first of them)
+    const int first = __ffsll((long long)m) - 1;
+    const gdt_d2 pv = io.xy[L.orig[st.iv]];
+    GdtDDVec c = {{0., 0.}, {0., 0.}}, b;
+    if (near) c = gdt_dd_disp(pv, io.xy[L.orig[kg]], S.lx, S.ly, x, y);
+    b.x.h = __shfl(c.x.h, first, 64);
+    b.x.l = __shfl(c.x.l, first, 64);
+    b.y.h = __shfl(c.y.h, first, 64);
+    b.y.l = __shfl(c.y.l, first, 64);
+    const int s = gdt_dd_sign(gdt_dd_dist_cmp(c, b), 2. * gdt_dd_tol2(gdt_dd_err(Lbox, M), M));
+    return __any(near && (int)(threadIdx.x & 63) != first && s == 0);
+}
 
 // One point by a wavefront (st: the point's state, the same in every lane, with
 // the lane's own table of STAR_TBL words; k_one_ring_star describes it).  Returns
-// STEP_DONE, STEP_NOCLOSE or STEP_DEFER, the row's length in count.
+// STEP_DONE, STEP_NOCLOSE or STEP_DEFER, the row's length in count (CERT: tied,
+// where a lane met a tie).
 template <bool CERT, bool GEN>
 __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtRingIO& io,
-                                GdtTileLane<double>& st, unsigned& npred, int& count)
+                                GdtTileLane<double>& st, unsigned& npred, int& count, bool& tied)
 {
     const int lane = (int)(threadIdx.x & 63);
     // the lanes' block, as one row table (every lane the same): the
@@ -335,9 +367,18 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
         if (lane >= acc && lane < acc + n) kg = b + lane - acc;
         acc += n;
     }
-    // (a block that holds too many for the lanes: in general boxes, whose clumps
-    // are handed on, lane 0's chain of steps is the slower way)
-    if (GEN && tot > 64) return STEP_DEFER;
+    // (a block that holds too many for the lanes: lane 0's chain of steps is the
+    // slower way with certified decisions, and in general boxes, whose clumps are
+    // handed on)
+    if ((CERT || GEN) && tot > 64) return STEP_DEFER;
+    if constexpr (CERT) {
+        // a point with two nearest neighbours, which the lanes' searches would
+        // end at (every point of a square lattice), is handed on at once
+        if (star_nn_tie(S, L, io, st, kg, ph)) {
+            tied = true;
+            return STEP_DEFER;
+        }
+    }
     int bk = -1, rc = STEP_DEFER;
     if (tot <= 64 && kg >= 0) {
         GdtTileLane<double> sl = st;
@@ -418,6 +459,7 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
             }
         }
     }
+    if (CERT && res == STEP_DEFER) tied = __any(bk == GDT_TIE);
     return res;
 }
 
@@ -616,7 +658,8 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
             st.tbl = words;
             lane_init(st, j);
             int count = 0;
-            const int res = star_ring<false, GEN>(S, L, io, st, npred, count);
+            bool tied = false;
+            const int res = star_ring<false, GEN>(S, L, io, st, npred, count, tied);
             if (lane == 0) {
                 if (res == STEP_DEFER) {
                     s_dlist[atomicAdd(&s_dn, 1u)] = j;
@@ -699,7 +742,9 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
 // block of more than 64 entries runs the sequential steps in lane 0.  Blocks
 // (tile, y) share a tile's points: wave w of block y takes the points
 // T0 + y nw + w + m gridDim.y nw.  Deferred points go to `defer` (handled by
-// k_one_ring_deferred in the next launch).
+// k_one_ring_deferred in the next launch); the exact mode's, which may be all of a
+// lattice, a block's together (an atomic for each took 160 of 195 us where all of
+// 16,384 points were handed on).
 template <bool CERT, bool GEN = false>
 __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star(const GdtSet* __restrict__ sets,
                                                         const GdtChunk* __restrict__ tiles,
@@ -713,6 +758,8 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
     __shared__ gdt_f2 s_X32[1];
     __shared__ int s_orig[GDT_WIN_MAXPTS];
     __shared__ uint32_t s_wsum[16];
+    __shared__ int s_hand[CERT ? STAR_HAND : 1];
+    __shared__ uint32_t s_hn, s_hpos;
     extern __shared__ uint32_t s_tbl[];     // [STAR_TBL * blockDim + 1] the lanes' row tables
 
     const GdtChunk ch = tiles[blockIdx.x];
@@ -736,6 +783,15 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
             }
         return;
     }
+    if constexpr (CERT) {
+        if (tid == 0) s_hn = 0u;
+        __syncthreads();
+    }
+    auto hand_on = [&](int q) {
+        const uint32_t h = CERT ? atomicAdd(&s_hn, 1u) : STAR_HAND;
+        if (h < STAR_HAND) s_hand[h] = q;
+        else defer[atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u)] = q;
+    };
     unsigned npred = 0, nsum = 0;
     int mx = 0, er = 0;
     for (int q = qb + (tid >> 6); q < T1; q += qstep) {     // wave-uniform
@@ -744,17 +800,32 @@ __global__ __launch_bounds__(CERT ? GDT_XTILE_BLOCK : 1024) void k_one_ring_star
         if constexpr (GEN) gdt_tile_lane_init_gen(w, L, q, io, S, st);
         else gdt_tile_lane_init<double>(w, L, q, io, S, st);
         int count = 0;
-        const int res = star_ring<CERT, GEN>(S, L, io, st, npred, count);
+        bool tied = false;
+        const int res = star_ring<CERT, GEN>(S, L, io, st, npred, count, tied);
+        if (CERT && tied) {
+            // (ties come by the lattice: the wave's other points are handed on unseen)
+            for (int p = q + lane * qstep; p < T1; p += 64 * qstep) hand_on(p);
+            break;
+        }
         if (lane == 0) {
             if (res == STEP_DEFER) {
-                const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
-                defer[pos] = q;
+                hand_on(q);
             } else {
                 counts[L.orig[st.iv]] = count;
                 mx = max(mx, count);
                 nsum += (unsigned)count;
                 if (res == STEP_NOCLOSE) er |= ERR_NOCLOSE;
             }
+        }
+    }
+    if constexpr (CERT) {
+        __syncthreads();
+        const int nh = min((int)s_hn, STAR_HAND);
+        if (nh > 0) {       // (block-uniform)
+            if (tid == 0)
+                s_hpos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), (unsigned)nh);
+            __syncthreads();
+            for (int t = tid; t < nh; t += (int)blockDim.x) defer[s_hpos + t] = s_hand[t];
         }
     }
     ring_block_totals(mx, er, npred, 0u, nsum, status, counters);
