@@ -558,10 +558,12 @@ GDT_HD inline void gdt_hull_insert(const GdtTileLds& L, int iv, uint32_t* words,
         p.w = gdt_dist2_64(p.x, p.y);
         return p;
     };
-    const GdtHullPt c = pt(k);
+    const GdtHullPt c = pt(k), a = pt(lst[i]);
     // (the list stays short enough for the row table; the first entry stays
-    // the nearest)
-    h.bad |= h.n + 1 > GDT_HULL_RING || c.w <= h.w0;
+    // the nearest; and the triangle that this closes is no sliver, which every
+    // other routine leaves uncertified)
+    h.bad |= h.n + 1 > GDT_HULL_RING || c.w <= h.w0 ||
+             !(gdt_hull_cross(a, c) > 1e-6 * (fabs(a.x * c.y) + fabs(a.y * c.x)));
     if (h.bad) {
         h.open = 0;
         return;
