@@ -42,7 +42,7 @@
 #define GDT_HULL_LIST 22
 #define GDT_HULL_RING 12      // longest ring that leaves room for a row table behind it
 #define GDT_HULL_TBL 6        // the row table's five words (and the one read after them)
-#define GDT_HULL_ROUNDS 64    // triangles (a wave: rounds) of part 3 before a point is left
+#define GDT_HULL_ROUNDS 64    // triangles of part 3 before a point is left
 
 // List entries (the lane's words also hold a row table).
 typedef uint16_t __attribute__((may_alias)) gdt_u16a;
@@ -664,7 +664,8 @@ GDT_HD inline void gdt_hull_load(const GdtTileLds& L, const uint32_t* rec, GdtHu
 // kernel 350 us with two, 575 with one, 358 with four): up to two
 // triangles of each lane at a time go to groups of lanes, which each scan a
 // part of every row and agree on the first of their finds; the triangles' lanes
-// then put those in.  Every lane of the wave calls it (open = 0 where it has no
+// then put those in, each lane's in the order that gdt_hull_close takes them, so that
+// its row does not depend on the points that share the wave.  Every lane of the wave calls it (open = 0 where it has no
 // point).  wave_words: the words of the wave's first lane; q: the wave's
 // 2 GDT_HULL_GROUPS words.
 #define GDT_HULL_W 2
@@ -681,8 +682,8 @@ __device__ inline void gdt_hull_close_wave(const GdtSet& S, const GdtTileLds& L,
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
     };
-    for (int round = 0;; ++round) {
-        if (round >= GDT_HULL_ROUNDS && h.open != 0) {
+    for (int taken = 0;;) {
+        if (taken >= GDT_HULL_ROUNDS && h.open != 0) {
             h.bad = true;
             h.open = 0;
         }
@@ -744,6 +745,7 @@ __device__ inline void gdt_hull_close_wave(const GdtSet& S, const GdtTileLds& L,
                 r = gdt_hull_probe<GEN>(S, L, iv, c0, h.lv, gdt_hull_entry(words, idx), kn,
                                         words + GDT_HULL_TBL, 0, 1, npred);
             }
+            ++taken;
             h.open &= ~(1u << idx);
             if (r == HULL_FAIL) {
                 h.bad = true;
@@ -753,7 +755,7 @@ __device__ inline void gdt_hull_close_wave(const GdtSet& S, const GdtTileLds& L,
             }
             return r == HULL_NONE;
         };
-        if (first && take(p1, i1) && second) take(p2, i2);
+        if (first && take(p1, i1) && second && taken < GDT_HULL_ROUNDS) take(p2, i2);
         sync();
     }
 }

@@ -465,19 +465,27 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
 
 // Points of a tile left by the hull routine that go straight to wavefronts (at most).
 #define GDT_HULL_WAVES 16
-// Records of points with open triangles a block keeps (more are left to the
-// steps; a tile of random points has about 150).
+// Records of points with open triangles a block keeps (32x32-cell tiles of random
+// points have about 200 of one point to a cell, 280 of 1.2, and in the larger
+// windows 480 of 1.44 and 700 of 2).
+#ifdef GDT_WIN_DENSE
+#define GDT_HULL_RECS 640
+#else
 #define GDT_HULL_RECS 256
+#endif
 // Records a wave closes together.
 #define GDT_HULL_TAKE 32
 
 // One block per tile, one point per lane: the hull routine (gdt_hull.h) over
 // all of the tile's points -- or, with `flags`, the flagged ones, as
 // k_one_ring_tile.  Waves take 64 points at a time; those with open triangles
-// (15 % of random points) are recorded in LDS, so that full waves close them,
+// (a fifth of random points) are recorded in LDS, so that full waves close them,
 // where every wave would wait for its few.  The points left to the steps (under
 // 0.1 % of random points) take them, or when they are few a wavefront's star
 // search each.
+// (Overfull pools that left points to the steps cost more at other cell sizes: 2^20
+// points of 1.2 to a cell 648 us per call, now 540, of 1.44 680 and 508, of 0.64 990
+// and 757.)
 // Bound by the vector ALU and by the imbalance of its parts (a 1M-point tile:
 // 9 us for staging, 65 for the lists, 39 for the open triangles, and 40 more in
 // the third of the tiles with a point left; FP64 adds and multiplies are half of
@@ -576,26 +584,53 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
     };
     // slot j's point is left to the steps
     auto leave = [&](int j) { atomicOr(&s_smask[(j - T0) >> 6], 1ull << ((j - T0) & 63)); };
+    // the wave's points (`mine`: this lane has one) closed, and their rows
+    auto close = [&](bool mine, GdtHull& h, int iv, int c0) {
+        gdt_hull_close_wave<GEN>(S, L, iv, c0, wave_words, wq, h, npred);
+        if (!mine) return;
+        if (!h.bad) {
+            emit(iv, h.n);
+        } else {
+            // its slot: the cell's first slot plus the rank in the cell
+            leave((int)io.cstart[gdt_tile_key(S, w, c0)] + iv - (int)L.cs[c0]);
+        }
+    };
+    // (cells of more than two points: what a 3x3 block leaves open is a third of the
+    // points, whose steps, all at once, take less than their closing: 2^20 points of 2.25
+    // to a cell 700 us per call, 787 closed; of 1.7 to a cell 622 closed, 780 by steps)
+    const bool full = npt > 2 * GDT_TILE_CELLS;
     for (;;) {
         int c = 0;
         if (lane == 0) c = atomicAdd(&s_next, 64);
         const int q = Q0 + __builtin_amdgcn_readfirstlane(c) + lane;
         if (q - lane >= Q1) break;      // (wave-uniform)
+        GdtHull h = {0, 0, 0u, true, 0.};
+        int iv = 0, c0 = 0;
+        bool mine = false;
         if (q < Q1) {
             const int j = item(q);
             GdtTileLane<double> st;
             lane_init(st, j);
-            GdtHull h;
             gdt_hull_build<GEN>(S, L, st, words, h, npred);
-            if (!h.bad && h.open != 0) {
-                const int r = atomicAdd(&s_rn, 1);
-                if (r < GDT_HULL_RECS) gdt_hull_save(h, st.iv, st.c0, words, s_rec + GDT_HULL_REC * r);
-                else h.bad = true;
-            } else if (!h.bad) {
+            if (h.bad || (full && h.open != 0)) {
+                leave(j);
+                h.open = 0;
+            } else if (h.open == 0) {
                 emit(st.iv, h.n);
+            } else {
+                const int r = atomicAdd(&s_rn, 1);
+                mine = r >= GDT_HULL_RECS;
+                iv = st.iv;
+                c0 = st.c0;
+                if (!mine) {
+                    gdt_hull_save(h, iv, c0, words, s_rec + GDT_HULL_REC * r);
+                    h.open = 0;
+                }
             }
-            if (h.bad) leave(j);
         }
+        // (no room among the records: closed by this wave; which points these are
+        // is up to the waves' order, but not what a row is)
+        if (__any(mine)) close(mine, h, iv, c0);
     }
     // Records are closed by the waves that have no chunk left, while others
     // still run theirs, and after a barrier the last ones.
@@ -627,24 +662,17 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
                     __builtin_amdgcn_s_sleep(1);
                 gdt_hull_load(L, rec, h, iv, c0, words);
             }
-            gdt_hull_close_wave<GEN>(S, L, iv, c0, wave_words, wq, h, npred);
-            if (lane < take) {
-                if (!h.bad) {
-                    emit(iv, h.n);
-                } else {
-                    // its slot: the cell's first slot plus the rank in the cell
-                    leave((int)io.cstart[gdt_tile_key(S, w, c0)] + iv - (int)L.cs[c0]);
-                }
-            }
+            close(lane < take, h, iv, c0);
         }
     };
     // (a repair's few are shared out by all of the waves, most of which had no
     // chunk)
-    if (!flags) drain(GDT_HULL_TAKE);
-    __syncthreads();
-    const int nw = nt >> 6;
-    drain(flags ? min(GDT_HULL_TAKE, max(1, (min(s_rn, GDT_HULL_RECS) + nw - 1) / nw)) : GDT_HULL_TAKE);
-    __syncthreads();
+    if (flags) __syncthreads();
+    for (int last = flags ? 1 : 0; last < 2; ++last) {
+        const int nw = nt >> 6;
+        drain(flags ? min(GDT_HULL_TAKE, max(1, (min(s_rn, GDT_HULL_RECS) + nw - 1) / nw)) : GDT_HULL_TAKE);
+        __syncthreads();
+    }
     // The points left to the steps, as in k_one_ring_tile.  Few of them take a
     // wavefront each, as the star kernel's points: one search's chain for the
     // ring, and one more where a circle leaves the lanes' block, not a chain of
@@ -684,7 +712,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
         // (clumps in a general box are handed on: their steps are long chains, and
         // its lists go one lane each: 262,144 points, half of them in 200 clumps,
         // 6.6 ms per call with the steps, 5.0 without)
-        auto full = [&]() {
+        auto clumped = [&]() {
             int n = 0;
             for (int r = -1; r <= 1; ++r) {
                 const uint32_t* row = L.cs + st.c0 + r * GDT_WIN;
@@ -694,7 +722,7 @@ __global__ __launch_bounds__(1024) void k_one_ring_hull(const GdtSet* __restrict
         };
         while (__ballot(have) != 0) {
             if (have) {
-                const bool hand_on = GEN && full();
+                const bool hand_on = GEN && clumped();
                 const int rc = hand_on ? STEP_DEFER
                                        : gdt_tile_step_f64<1, false, GEN>(S, L, io, st, npred);
                 if (rc != STEP_RUN) {
