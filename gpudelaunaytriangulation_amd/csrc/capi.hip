@@ -276,7 +276,7 @@ static int lanes_for(const gdt_context* c)
 // test and repair, 492 / 588 with two lanes; 64 sets of 980,000 points 476 us a
 // step, 491), and four with the 16x16 ones of smaller inputs, whose blocks end
 // with their longest chain of steps (131,072 points 187 us, 204 with two lanes
-// and 215 with one; 250,000: 212, 214, 270).
+// and 215 with one; tiles with many flagged points then take two).
 static int repair_lanes_for(const gdt_context* c)
 {
     if (c->cfg.repair_lanes) return c->cfg.repair_lanes;

@@ -236,66 +236,80 @@ __global__ __launch_bounds__(PREC == GDT_EXACT ? GDT_XTILE_BLOCK : 1024) void k_
     static_assert(W == 1 || W == 2 || (W == 4 && PREC == 64), "1, 2 or (FP64) 4 lanes per point");
     static_assert(!GEN || (PREC == 64 && W <= 2), "general boxes: FP64, one or two lanes");
     static_assert(PREC == 32 || PREC == 64 || PREC == GDT_EXACT, "a precision code");
-    if (tid == 0) {
-        s_next = Q0 + nt / W;
-        s_dn = 0u;
-    }
-    __syncthreads();
-    using Real = typename std::conditional<PREC == 32, float, double>::type;
-    GdtTileLane<Real> st;
-    st.tbl = s_tbl + 5 * tid;
-    const int sub = tid & (W - 1);      // the lane's part of its point's rows
-    int q = Q0 + tid / W;
-    bool have = q < Q1;
-    int j = have ? item(q) : 0;
-    auto lane_init = [&]() {
-        if constexpr (GEN) gdt_tile_lane_init_gen(w, L, j, io, S, st);
-        else gdt_tile_lane_init<Real>(w, L, j, io, S, st);
-    };
-    if (have) lane_init();
     unsigned npred = 0, nfb = 0, nsum = 0;
     int mx = 0, er = 0;
-    while (__ballot(have) != 0) {
-        if (have) {
-            int rc;
-            if constexpr (PREC == 32)
-                rc = gdt_tile_step_f32<W>(S, L, io, st, npred, nfb, sub);
-            else
-                rc = gdt_tile_step_f64<W, PREC == GDT_EXACT, GEN>(S, L, io, st, npred, sub);
-            // (both lanes of a pair end each step in the same state; the first reports)
-            if (rc != STEP_RUN && sub == 0) {
-                if (rc == STEP_DEFER) {
-                    // the block's own waves finish it after the tile (below)
-                    // (the exact mode's go to the per-point routine)
-                    const uint32_t dpos = PREC == GDT_EXACT ? GDT_TILE_DEFER : atomicAdd(&s_dn, 1u);
-                    if (dpos < GDT_TILE_DEFER) {
-                        s_dlist[dpos] = j;
+    auto run = [&](auto lanes_each) {
+        constexpr int V = decltype(lanes_each)::value;      // lanes per point
+        if (tid == 0) {
+            s_next = Q0 + nt / V;
+            s_dn = 0u;
+        }
+        __syncthreads();
+        using Real = typename std::conditional<PREC == 32, float, double>::type;
+        GdtTileLane<Real> st;
+        st.tbl = s_tbl + 5 * tid;
+        const int sub = tid & (V - 1);      // the lane's part of its point's rows
+        int q = Q0 + tid / V;
+        bool have = q < Q1;
+        int j = have ? item(q) : 0;
+        auto lane_init = [&]() {
+            if constexpr (GEN) gdt_tile_lane_init_gen(w, L, j, io, S, st);
+            else gdt_tile_lane_init<Real>(w, L, j, io, S, st);
+        };
+        if (have) lane_init();
+        while (__ballot(have) != 0) {
+            if (have) {
+                int rc;
+                if constexpr (PREC == 32)
+                    rc = gdt_tile_step_f32<V>(S, L, io, st, npred, nfb, sub);
+                else
+                    rc = gdt_tile_step_f64<V, PREC == GDT_EXACT, GEN>(S, L, io, st, npred, sub);
+                // (both lanes of a pair end each step in the same state; the first reports)
+                if (rc != STEP_RUN && sub == 0) {
+                    if (rc == STEP_DEFER) {
+                        // the block's own waves finish it after the tile (below)
+                        // (the exact mode's go to the per-point routine)
+                        const uint32_t dpos = PREC == GDT_EXACT ? GDT_TILE_DEFER : atomicAdd(&s_dn, 1u);
+                        if (dpos < GDT_TILE_DEFER) {
+                            s_dlist[dpos] = j;
+                        } else {
+                            const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
+                            defer[pos] = j;
+                        }
                     } else {
-                        const uint32_t pos = atomicAdd(reinterpret_cast<unsigned int*>(&status[ST_NDEFER]), 1u);
-                        defer[pos] = j;
+                        counts[L.orig[st.iv]] = st.count;
+                        mx = max(mx, st.count);
+                        nsum += (unsigned)st.count;
+                        if (rc == STEP_NOCLOSE) er |= ERR_NOCLOSE;
                     }
-                } else {
-                    counts[L.orig[st.iv]] = st.count;
-                    mx = max(mx, st.count);
-                    nsum += (unsigned)st.count;
-                    if (rc == STEP_NOCLOSE) er |= ERR_NOCLOSE;
                 }
-            }
-            if (rc != STEP_RUN) {
-                if constexpr (W > 1) {
-                    int qq = 0;
-                    if (sub == 0) qq = atomicAdd(&s_next, 1);
-                    q = __shfl(qq, (tid & 63) & ~(W - 1), 64);
-                } else {
-                    q = atomicAdd(&s_next, 1);
-                }
-                have = q < Q1;
-                if (have) {
-                    j = item(q);
-                    lane_init();
+                if (rc != STEP_RUN) {
+                    if constexpr (V > 1) {
+                        int qq = 0;
+                        if (sub == 0) qq = atomicAdd(&s_next, 1);
+                        q = __shfl(qq, (tid & 63) & ~(V - 1), 64);
+                    } else {
+                        q = atomicAdd(&s_next, 1);
+                    }
+                    have = q < Q1;
+                    if (have) {
+                        j = item(q);
+                        lane_init();
+                    }
                 }
             }
         }
+    };
+    // A repair's four lanes per point are for the few points of a tile; where they
+    // outnumber the block's groups of four, two lanes each take them in half as many
+    // turns (test and repair of 65,536 points moved by 0.05, 143 of a tile's 256
+    // flagged: 223 us, 244 with four lanes; by 0.01, 40 flagged: 176 with four, 198 with
+    // two; the line at 64 or 85 flagged made no difference).
+    if constexpr (W == 4) {
+        if (flags && 4 * (Q1 - Q0) > nt) run(std::integral_constant<int, 2>{});
+        else run(std::integral_constant<int, 4>{});
+    } else {
+        run(std::integral_constant<int, W>{});
     }
     if constexpr (PREC != GDT_EXACT) {
         __syncthreads();

@@ -73,7 +73,9 @@ typedef struct {
                            2 with 16x16 tiles that do not outnumber the compute units,
                            else 1 */
     int repair_lanes;   /* lanes per point of the repairs' tile kernel, 1, 2 or 4 (as
-                           lanes); 0 (default) = 4 with 16x16 tiles, else 1 */
+                           lanes); 0 (default) = 4 with 16x16 tiles, else 1; 4 takes 2
+                           in tiles with more flagged points than a quarter of
+                           the block */
 } gdt_config;
 
 /* Statistics of the last triangulate / repair call. */
