@@ -364,10 +364,14 @@ GDT_HD inline double gdt_dd_incircle(const GdtDDVec& a, const GdtDDVec& b, const
     return P.h;
 }
 
-// Their error bounds: those of gdt_x_tol2 and gdt_x_tol4 with a displacement
-// error of 64 u^2 (L + |d|) (the pair holds (c - v) exactly; the rounding of
-// its sum with m L, |m L| at most five box lengths, is below 16 u^2 L) and
-// 16 u^2 for u.
+// Their error bounds: those of gdt_x_tol2 and gdt_x_tol4 with 16 u^2 for u and a
+// displacement error of 64 u^2 (L + |d|).  The displacement (gdt_dd_disp1): both
+// coordinates lie within four box lengths, so c - v = s + e exactly with |s| <= 8L
+// and |e| <= 8uL; the image seen lies within three (the window's 20 cells), so |m| <= 11
+// and m L = p + q exactly with |q| <= 11uL; s + p = h + l exactly with |h| <= 3L, |l| <=
+// 3uL.  What is rounded is e + q, by at most 19 u^2 L, and l + (e + q), by at
+// most 22 u^2 L: 41 u^2 L together.  (Where |h| is below l + e + q, the points all but
+// coincide, l is zero, and the last sum's rounding of 19 u^2 L takes its place.)
 #define GDT_XU2 (16. * GDT_XU * GDT_XU)
 GDT_HD inline double gdt_dd_err(double L, double d)
 {
