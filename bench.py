@@ -1,9 +1,10 @@
 #!/usr/bin/env python3
 """Headline benchmark: points/sec of the global periodic Delaunay
 triangulation of 1,048,576 uniform points (box 1024 x 1024, cell size 1) on
-one MI355X, FP32-filtered predicates with FP64 fallback and all-FP64 timed
-side by side (rows identical).  The headline value is the library's default
-path, FP64; the FP32-filtered rate is reported beside it.
+one MI355X.  The headline value is the library's default path, FP64.  Beside it:
+the calls in FP32-filtered precision, which at this size run the same FP64
+kernel, and the filtered kernel itself (FP32 predicates with FP64 fallback, two
+lanes per point), whose rows are compared with FP64's.
 
 A step is one DelaunayGPU.globalDelaunayTriangulation call (counting-sort
 cell list + one-ring kernel + the status readback of the C ABI) on points
@@ -122,6 +123,12 @@ def time_path(dg, pts, tri, num, steps, warmup, torch):
     return ms, wall, per["ms_ring"], per["ms_cells"], per["ms_defer"], s1
 
 
+def filtered_config(dg):
+    """A configuration that runs the FP32-filtered kernel (with one lane per
+    point, the automatic choice for large grids, both precisions run FP64)."""
+    dg.ctx.set_config(lanes=2)
+
+
 def cpu_model():
     """The host CPU's model name (first /proc/cpuinfo entry), or 'unknown'."""
     try:
@@ -169,9 +176,9 @@ def bench_c1(torch, cpu_runs, with_cpu):
 def bench_c3b(torch, steps, warmup):
     """The jittered triangular lattice: 1024 x 1024 points, spacing 1, rows
     sqrt(3)/2 apart, Gaussian jitter sigma = 1e-5 (near-cocircular quads),
-    box 1024 x 886.81, cell size 1: points/s and fallback fraction per
-    precision, rows identical across precisions and equal to the committed
-    oracle hash."""
+    box 1024 x 886.81, cell size 1: points/s per precision and of the FP32-filtered kernel (two
+    lanes per point) with its fallback fraction, rows identical and equal to the
+    committed oracle hash."""
     from gpudelaunaytriangulation_amd import PREC_FP32F, PREC_FP64, inputs, rings
     from gpudelaunaytriangulation_amd.delaunay import DelaunayGPU, PeriodicBoundaries
     lx, ly = inputs.lattice_box(1024, 1024)
@@ -181,10 +188,12 @@ def bench_c3b(torch, steps, warmup):
     res = {"workload": f"jittered triangular lattice 1024x1024 (sigma 1e-5), box {lx:g}x{ly:.6f}, "
                        f"cell 1.0"}
     hashes = {}
-    for name, prec in (("fp32f", PREC_FP32F), ("fp64", PREC_FP64)):
+    for name, prec in (("fp32f", PREC_FP32F), ("filtered", PREC_FP32F), ("fp64", PREC_FP64)):
         dg = DelaunayGPU(n, 16, 1.0, PeriodicBoundaries(lx, ly))
         dg.setPrecision(prec)
         dg.ctx.set_config(profile=1)
+        if name == "filtered":
+            filtered_config(dg)
         tri = torch.zeros(n * dg.MaxSize, dtype=torch.int32, device="cuda")
         num = torch.zeros(n, dtype=torch.int32, device="cuda")
         ms, _, ring_ms, _, _, st = time_path(dg, pts, tri, num, steps, warmup, torch)
@@ -193,14 +202,14 @@ def bench_c3b(torch, steps, warmup):
         res[f"{name}_ms_per_step"] = ms
         res[f"{name}_one_ring_ms"] = ring_ms
         res[f"{name}_deferred_points"] = st["deferred"]
-        if name == "fp32f":
+        if name == "filtered":
             res["fallback_fraction"] = st["fallbacks"] / max(1, st["predicates"])
             res["predicates_per_point"] = st["predicates"] / n
-    res["topology_identical_fp32_fp64"] = hashes["fp32f"] == hashes["fp64"]
+    res["topology_identical_fp32_fp64"] = hashes["filtered"] == hashes["fp64"]
     gpath = os.path.join(ROOT, "tests", "golden", "golden.json")
     with open(gpath) as fh:
         res["matches_golden_oracle_hash"] = (json.load(fh)["workloads"]["c3b"]["ring_sha256"]
-                                             == hashes["fp32f"])
+                                             == hashes["fp64"])
     return res
 
 
@@ -251,9 +260,8 @@ def bench_exact(torch, steps, warmup):
 
 def bench_general(torch, steps, warmup):
     """A general (triclinic) box: 2^20 uniform points in the sheared box with
-    lattice vectors (1024, 0) and (320, 1024) (density 1, cell size 1), FP64
-    (general boxes run the row-major per-point kernels): points/s of the
-    global triangulation, time of a test-and-repair after a Gaussian move of
+    lattice vectors (1024, 0) and (320, 1024) (density 1, cell size 1), FP64:
+    points/s of the global triangulation, time of a test-and-repair after a Gaussian move of
     sigma 0.01 (wrapped by whole lattice vectors), and whether the rings equal
     the CPU mode's (the same routines on the host)."""
     import ctypes
@@ -462,13 +470,15 @@ def main():
     pts = torch.from_numpy(xy).cuda()
     out = {}
     wanted = args.precisions.split(",")
-    for name, prec in (("fp32f", PREC_FP32F), ("fp64", PREC_FP64)):
-        if name not in wanted and not (name == "fp32f"):
+    for name, prec in (("fp32f", PREC_FP32F), ("filtered", PREC_FP32F), ("fp64", PREC_FP64)):
+        if name not in wanted and name == "fp64":
             continue
         dg = DelaunayGPU(n, 16, 1.0, PeriodicBoundaries(L, L))
         dg.setPrecision(prec)
         dg.ctx.set_config(profile=1, block=args.block, tiled=args.tiled, cell_scale=args.cell_scale,
                           tile_shift=args.tile_shift, lanes=args.lanes)
+        if name == "filtered":
+            filtered_config(dg)
         tri = torch.zeros(n * dg.MaxSize, dtype=torch.int32, device="cuda")
         num = torch.zeros(n, dtype=torch.int32, device="cuda")
         ms, wall, ring_ms, cell_ms, defer_ms, st = time_path(dg, pts, tri, num, args.steps,
@@ -476,7 +486,8 @@ def main():
         nb = tri.cpu().numpy().reshape(n, dg.MaxSize)
         cnt = num.cpu().numpy()
         out[name] = dict(ms=ms, wall=wall, ring_ms=ring_ms, cell_ms=cell_ms, defer_ms=defer_ms,
-                         st=st, hash=rings.ring_hash(nb, cnt), sum=int(cnt.sum()), nb=nb, cnt=cnt)
+                         st=st, hash=rings.ring_hash(nb, cnt), sum=int(cnt.sum()), nb=nb, cnt=cnt,
+                         block=dg.ctx.config().block)
         print(f"[bench] {name}: {ms:.3f} ms/step (one-ring {ring_ms:.3f} ms, deferred "
               f"{defer_ms:.3f} ms, cell list {cell_ms:.3f} ms), {n / ms * 1e3 / 1e9:.3f} Gpoints/s, "
               f"deferred {st['deferred']}, pred/pt {st['predicates'] / n:.1f}", file=sys.stderr,
@@ -484,8 +495,9 @@ def main():
 
     f32 = out["fp32f"]
     f64 = out.get("fp64", f32)
-    identical = (f32["hash"] == f64["hash"] and np.array_equal(f32["nb"], f64["nb"])
-                 and np.array_equal(f32["cnt"], f64["cnt"]))
+    filt = out["filtered"]
+    identical = (filt["hash"] == f64["hash"] and np.array_equal(filt["nb"], f64["nb"])
+                 and np.array_equal(filt["cnt"], f64["cnt"]))
     golden_ok = None
     gpath = os.path.join(ROOT, "tests", "golden", "golden.json")
     if n == N_POINTS and os.path.exists(gpath):
@@ -493,7 +505,7 @@ def main():
             golden_ok = json.load(fh)["workloads"]["c2"]["ring_sha256"] == f32["hash"]
 
     # The headline is the library's default path, FP64 (when measured); the
-    # FP32-filtered path, decision-identical, is reported beside it.
+    # FP32-filtered precision and its kernel are reported beside it.
     head = f64 if "fp64" in out else f32
     head_name = "fp64" if "fp64" in out else "fp32f"
     head_kernel = "k_one_ring_hull<false>"      # (in either precision)
@@ -533,23 +545,30 @@ def main():
         "data": "synthetic: SplitMix64 uniform points, seed 2",
         "config": {"workload": f"uniform periodic {n} points, box {L:g}x{L:g}, cell 1.0, "
                                + ("FP64 global triangulation (the library default; the "
-                                  "FP32-filtered path is reported beside it)"
+                                  "FP32-filtered precision is reported beside it)"
                                   if head_name == "fp64" else "FP32-filtered global triangulation"),
                    "headline_path": head_name,
-                   "n": n, "box": L, "cell_size": 1.0, "block": dg.ctx.config().block,
+                   "n": n, "box": L, "cell_size": 1.0, "block": head["block"],
                    "tile_cells": 1 << st["tile_shift"], "lanes_per_point": st["lanes"]},
         "fp64_points_per_s": n / (f64["ms"] * 1e-3),
         "fp64_ms_per_step": f64["ms"],
         "fp32f_points_per_s": n / (f32["ms"] * 1e-3),
         "fp32f_ms_per_step": f32["ms"],
-        "fp32_over_fp64": f64["ms"] / f32["ms"],
+        "fp32f_path": "the FP64 kernel (one lane per point takes no filtered decision)"
+                      if f32["st"]["lanes"] == 1 else "the FP32-filtered kernel",
+        "filtered_kernel": {"lanes_per_point": filt["st"]["lanes"],
+                            "points_per_s": n / (filt["ms"] * 1e-3), "ms_per_step": filt["ms"],
+                            "one_ring_ms": filt["ring_ms"],
+                            "fallback_fraction": filt["st"]["fallbacks"]
+                            / max(1, filt["st"]["predicates"]),
+                            "predicates_per_point": filt["st"]["predicates"] / n},
+        "fp32_over_fp64": f64["ms"] / filt["ms"],
         "topology_identical_fp32_fp64": bool(identical),
         "matches_golden_oracle_hash": golden_ok,
         "sum_counts_eq_6N": f32["sum"] == 6 * n,
-        "fallback_fraction": st["fallbacks"] / max(1, st["predicates"]),
         "predicates_per_point": st["predicates"] / n,
         "deferred_points": st["deferred"],
-        "kernel_ms": {"one_ring_tile_fp32f": f32["ring_ms"], "one_ring_tile_fp64": f64["ring_ms"],
+        "kernel_ms": {"one_ring_fp32f": f32["ring_ms"], "one_ring_fp64": f64["ring_ms"],
                       "deferred_fp32f": f32["defer_ms"], "deferred_fp64": f64["defer_ms"],
                       "cell_list": f32["cell_ms"]},
         "roofline": {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",

@@ -520,7 +520,8 @@ class DelaunayGPU:
 
     def setPrecision(self, precision: int) -> None:
         """64: all-FP64 predicates; 32: FP32 with certified bound + FP64
-        fallback; 128 (PREC_EXACT): every decision exact -- FP64 where its
+        fallback where the kernels filter (large and small grids and general
+        boxes run FP64 in it too: the same rows); 128 (PREC_EXACT): every decision exact -- FP64 where its
         error bound certifies it, expansion arithmetic otherwise, exact ties
         by the symbolic perturbation (rectangular boxes, coordinates within
         four box lengths of the box)."""

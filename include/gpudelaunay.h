@@ -42,7 +42,11 @@ typedef enum {
 
 typedef enum {
     GDT_PREC_FP64 = 64,        /* all predicates in FP64 */
-    GDT_PREC_FP32F = 32,       /* FP32 with certified error bound, FP64 fallback */
+    GDT_PREC_FP32F = 32,       /* FP32 with certified error bound, FP64 fallback, where the
+                                  kernel filters: two or four lanes per point, and the
+                                  row-major order; with one lane or 64 per point (see
+                                  gdt_config) and in general boxes the FP64 kernels,
+                                  which are faster there; the rows are FP64's either way */
     GDT_PREC_EXACT = 128       /* every decision exact (FP64 where its error bound
                                   certifies it, else double-double, else expansion
                                   arithmetic; exact ties by the symbolic
@@ -63,8 +67,10 @@ typedef struct {
     int tile_shift;     /* LDS tile of the tiled orders: 2^tile_shift cells a side, 4 (16x16)
                            or 5 (32x32); 0 (default) = automatic: 16x16 when the 32x32
                            tiles would not outnumber the compute units, else 32x32 */
-    int lanes;          /* lanes per point of the global triangulation's tile kernel, 1, 2
-                           or 4 (4: FP64; the FP32-filtered kernel takes 2 then), or 64:
+    int lanes;          /* lanes per point of the global triangulation's tile kernel, 1 (FP64
+                           predicates in either precision), 2 or 4 (4: FP64; the
+                           FP32-filtered kernel takes 2 then; windows of more than 1,945
+                           points on average take 1 whatever is set), or 64:
                            one wavefront per point whose lanes search from every candidate
                            of the point's cell block at once (FP64 predicates in either
                            precision, the same rings; 256-thread blocks; for small grids);
@@ -81,7 +87,8 @@ typedef struct {
 /* Statistics of the last triangulate / repair call. */
 typedef struct {
     unsigned long long predicates;   /* predicate evaluations */
-    unsigned long long fallbacks;    /* FP64 fallbacks of the filtered path */
+    unsigned long long fallbacks;    /* FP64 fallbacks of the filtered kernels (0 where FP32F
+                                        runs the FP64 ones) */
     unsigned long long neighbours;   /* sum of ring lengths written */
     int max_ring;                    /* largest ring */
     int flagged;                     /* points flagged by the last circumcircle test */

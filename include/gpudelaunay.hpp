@@ -735,6 +735,7 @@ public:
     void setGPUcompute(bool flag) { GPUcompute = flag; }
     void setOMPthreads(unsigned int num) { OMPThreadsNum = num; }
     //! 64: all-FP64 predicates; 32: FP32 with a certified bound + FP64 fallback
+    //! where the kernels filter (see gdt_precision; the rows are the same)
     void setPrecision(int p)
     {
         if (p != GDT_PREC_FP64 && p != GDT_PREC_FP32F && p != GDT_PREC_EXACT)
