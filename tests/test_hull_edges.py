@@ -73,3 +73,18 @@ def test_slivers_are_left(exe, tmp_path, seed):
     xy, L = pairs(seed)
     n, _, differ, err = run(exe, tmp_path, xy, L, L, 1.0)
     assert n == len(xy) and differ == 0 and err     # (rows and flags alike, among them the refusal)
+
+
+# (FP64 rows of every routine hold from 1e-30 to 1e36; FP32's squared distances, by
+# which the hull finds the nearest entry, from 1e-17 to 1e19: beyond, the steps)
+@pytest.mark.parametrize("general", [False, True])
+@pytest.mark.parametrize("scale", [1e-30, 1e-22, 1e-12, 1e12, 1e19, 1e20, 1e25, 1e36])
+def test_scales(exe, tmp_path, scale, general):
+    L = 40.0 * scale
+    xy = np.random.default_rng(3).random((1600, 2)) * L
+    if general:
+        xy = np.stack([xy[:, 0] + 0.3 * xy[:, 1], xy[:, 1]], 1)
+    n, left, differ, err = run(exe, tmp_path, xy, L, L, scale, *((0.3 * L, 0.0) if general else ()))
+    assert n == len(xy) and differ == 0 and err == 0
+    if 1e-20 < scale < 1e19:
+        assert 10 * left < n
