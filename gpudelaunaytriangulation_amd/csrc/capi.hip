@@ -331,7 +331,7 @@ static_assert((int)GDT_PREC_EXACT == (int)GDT_EXACT, "one code for the exact mod
 // of `boxes`, words per box 2 or 4 as box_of): in the configured cell order,
 // tiled orders with the tile edge of the configuration or the automatic one.
 // General boxes take the tile kernels too (2^20 points in a box sheared by 0.31:
-// 581 us per call, 2,841 with the row-major per-point kernel).
+// 430 us per call, 2,841 with the row-major per-point kernel).
 // Sets of which one is a general box keep the row-major order where the tile
 // kernels could not take them: a grid smaller than the windows' scan block
 // (every point of such a tile is handed on), tiles whose padding outgrows

@@ -504,7 +504,7 @@ __device__ inline int star_ring(const GdtSet& S, const GdtTileLds& L, const GdtR
 // 9 us for staging, 65 for the lists, 39 for the open triangles, and 40 more in
 // the third of the tiles with a point left; FP64 adds and multiplies are half of
 // the instructions), not by memory (0.14 GB, 20 us).  Ring kernel of 1M / 3.9M
-// uniform points 342 / 1,149 us (the steps: 496 / 1,890 at 4M), of a 1M
+// uniform points 342 / 1,155 us (the steps: 496 / 1,890 at 4M), of a 1M
 // near-lattice 228 (339).  Blocks of 512, two
 // to a compute unit: 1,024 threads took 477 us at 1M, 256 threads on 16x16
 // tiles 445, 320 threads 622; a cap of 96 registers for five waves spilled
